@@ -26,11 +26,12 @@
 // annihilates column s below its subdiagonal; its tasks k = 0, 1, ... each apply one
 // reflector (ZLARFG) two-sidedly to a diagonal block and the previous one from the right
 // to the block below it (creating the bulge whose first column the next reflector
-// annihilates).  One persistent kernel whose workgroups claim sweeps in order from a
-// counter; task k of sweep s waits until sweep s - 1 has finished its tasks 0..k+1 (its
-// later tasks touch only rows below this task's), signalled through a per-sweep progress
-// counter (device-scope accesses, no cache maintenance).  Every wait is bounded: past the limit the
-// kernel sets an error flag that every waiting workgroup sees, and all of them return.
+// annihilates).  One persistent kernel (k_chase) whose workgroups claim groups of sweeps in
+// order from a counter; task k of sweep s waits until sweep s - 1 has finished its tasks
+// 0..k+1 (its later tasks touch only rows below this task's), signalled through counters in
+// LDS inside a group and through a progress counter in memory between groups (device-scope
+// accesses, no cache maintenance).  Every wait is bounded: past the limit the kernel sets an
+// error flag that every waiting workgroup sees, and all of them return.
 #include "wtb_kernels.h"
 
 namespace wtb {
@@ -51,7 +52,6 @@ __device__ inline zc zdiv(zc a, zc b) {
   return mkz(xr / den, xi / den);
 }
 
-__device__ inline zc shfl_z(zc v, int src) { return mkz(__shfl(v.re, src), __shfl(v.im, src)); }
 __device__ inline zc shfl_xor_z(zc v, int off) { return mkz(__shfl_xor(v.re, off), __shfl_xor(v.im, off)); }
 
 // x of another lane by a DPP lane permutation (within rows of 16 lanes) or a swizzle
@@ -69,7 +69,6 @@ __device__ inline double swz16_d(double x) {   // lane ^ 16 within 32 lanes
   const int hi = __builtin_amdgcn_ds_swizzle((int)(v >> 32), 0x401F);
   return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
 }
-__device__ inline zc swz16_z(zc v) { return mkz(swz16_d(v.re), swz16_d(v.im)); }
 template <int CTRL>
 __device__ inline zc dpp_z(zc v) { return mkz(dpp_d<CTRL>(v.re), dpp_d<CTRL>(v.im)); }
 
@@ -983,215 +982,431 @@ __global__ void k_conj_vec(int n, const zc* __restrict__ x, zc* __restrict__ y) 
 // ---------------------------------------------------------------------------
 // stage 2: bulge chasing
 // ---------------------------------------------------------------------------
+template <int B>
+struct ChaseDim {
+  static constexpr int SW = (B == 16) ? 3 : 2;   // sweeps per workgroup, one wave each
+  static constexpr int R = (B == 16) ? 4 : 2;    // LDS slots per boundary between sweeps
+  static constexpr int NC = B * B / 64;          // columns per thread
+  static constexpr int P = B + 1;                // column length of a slot
+  static constexpr int G = 2 * B * P;            // offset of its tracked rows
+  static constexpr int SLOT = G + 6 * P;
+};
+
 struct ChaseArgs {
-  zc* BD;            // [N][LB]
-  int N, b, LB;
+  zc* BD;            // [N][2 B + 1]
+  int N;
   zc* gc;            // nrhs x N (conjugated tracked vectors)
   int nrhs;
-  int* prog;         // [N] tasks completed per sweep
-  int* ctl;          // [0] error flag, [32] next sweep to claim
+  int* prog;         // [group] tasks that the group's last sweep has finished
+  int* ctl;          // [0] error flag, [32] next group to claim
   long long spin_limit;
 };
 
-__device__ inline int chase_ntasks(int N, int b, int s) { return 1 + (N - 2 - s) / b; }
+__host__ __device__ inline int chase_ntasks(int N, int b, int s) { return 1 + (N - 2 - s) / b; }
 
-// element (r, c) of the band, r >= c
-__device__ inline zc& bd(const ChaseArgs& a, int r, int c) { return a.BD[(size_t)c * a.LB + (r - c)]; }
+// Lane halves and 16-lane rows by the swap instructions (VALU, no LDS round trip): after
+// swap32(a, b) lane l < 32 holds a(l) and a(l + 32), lane l >= 32 b(l - 32) and b(l); swap16
+// does the same within each pair of 16-lane rows.  a + b is then a sum over that lane bit,
+// of a in the lanes where the bit is clear and of b where it is set.
+__device__ inline void swap32(double& a, double& b) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
+  b = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline void swap16(double& a, double& b) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
+  b = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline double add32(double a, double b) {
+  swap32(a, b);
+  return a + b;
+}
+__device__ inline double add16(double a, double b) {
+  swap16(a, b);
+  return a + b;
+}
 
-
-// sum over the B (16 or 32) lanes of a row group: lane pairs ^1, ^2 (quad permutations),
-// then i <-> 7 - i, i <-> 15 - i within rows (half mirror, mirror), then ^16.  Every step
-// adds two equal partial sums in either order, so every lane of the group ends with the
-// same bits.
+// The chase keeps row r of a block in the lanes r (64 / B) + (column group), so that rows
+// lie on the lane's high bits.  Sum over the rows (every lane ends with it): both halves,
+// both rows of 16, rotations by 8 and 4 in a row of 16, and for B = 32 lane pairs ^2.
 template <int B>
-__device__ inline double group_sum(double x) {
-  x += dpp_d<0xB1>(x);    // quad_perm [1, 0, 3, 2]
-  x += dpp_d<0x4E>(x);    // quad_perm [2, 3, 0, 1]
-  x += dpp_d<0x141>(x);   // row_half_mirror
-  x += dpp_d<0x140>(x);   // row_mirror
-  if constexpr (B == 32) x += swz16_d(x);
+__device__ inline double row_group_sum(double x) {
+  x = add32(x, x);
+  x = add16(x, x);
+  x += dpp_d<0x128>(x);                        // row_ror:8
+  x += dpp_d<0x124>(x);                        // row_ror:4
+  if constexpr (B == 32) x += dpp_d<0x4E>(x);  // quad_perm [2, 3, 0, 1]
   return x;
 }
 template <int B>
-__device__ inline zc group_sum(zc x) {
-  return mkz(group_sum<B>(x.re), group_sum<B>(x.im));
+__device__ inline zc row_group_sum(zc x) {
+  return mkz(row_group_sum<B>(x.re), row_group_sum<B>(x.im));
 }
 
-// Column sums of a B x B block held as thread (r, h) = (t % B, t / B) owning row r and
-// columns h NC .. h NC + NC - 1 (NC = B^2 / 256); the B rows of a column group lie in one
-// wave.  B = 32: a halving butterfly on row bits 4 (swizzle) and 3 (DPP rotate by 8 in a
-// row of 16), each lane keeping the half its bit selects, then a DPP sum over the 8-lane
-// block: thread (r, h) ends with the sum of local column r >> 3.  B = 16 (one column per
-// thread): the group sum.
+// Column sums of NC values: halved over the two highest row bits by the swaps (the lanes
+// of row quarter u keep columns u NC / 4 ..), then summed over the row bits left
 template <int B, int NC>
-__device__ inline zc col_sums(zc (&t)[NC], int lane) {
-  if constexpr (NC == 4) {
-    static_assert(B == 32, "four columns per thread for B = 32");
-    bf_step<16, 2>(t, lane);
-    bf_step<8, 1>(t, lane);
-    zc x = t[0] + xchg<4>(t[0]);
-    x += xchg<2>(x);
-    x += xchg<1>(x);
-    return x;
-  } else {
-    static_assert(B == 16 && NC == 1, "one column per thread for B = 16");
-    return group_sum<16>(t[0]);
+__device__ inline void col_sums(zc (&v)[NC]) {
+#pragma unroll
+  for (int q = 0; q < NC / 2; ++q) v[q] = mkz(add32(v[q].re, v[q + NC / 2].re), add32(v[q].im, v[q + NC / 2].im));
+#pragma unroll
+  for (int q = 0; q < NC / 4; ++q) {
+    zc x = mkz(add16(v[q].re, v[q + NC / 4].re), add16(v[q].im, v[q + NC / 4].im));
+    x += dpp_z<0x128>(x);
+    x += dpp_z<0x124>(x);
+    if constexpr (B == 32) x += dpp_z<0x4E>(x);
+    v[q] = x;
   }
 }
 
-// Row sums: a thread's own columns, the column groups of its wave, then the four waves
-// through LDS in wave order (red: [4][B]); every thread gets the sum of its row.
+// sum over the column groups of a wave (the lane's low bits)
 template <int B>
-__device__ inline zc row_sum(zc x, zc* red, int t) {
-#pragma unroll
-  for (int off = B; off < 64; off <<= 1) x += shfl_xor_z(x, off);
-  const int wave = t >> 6, lane = t & 63;
-  if (lane < B) red[wave * B + lane] = x;
-  __syncthreads();
-  const int r = t & (B - 1);
-  return ((red[r] + red[B + r]) + red[2 * B + r]) + red[3 * B + r];
+__device__ inline zc lane_group_sum(zc x) {
+  x += dpp_z<0xB1>(x);
+  if constexpr (B == 16) x += dpp_z<0x4E>(x);
+  return x;
 }
 
-// One sweep per 256-thread workgroup, claimed in order from a counter; task k of sweep
-// s waits until sweep s - 1 has finished its tasks 0..k+1 (the later tasks of sweep
-// s - 1 touch only rows below this task's last row).  Thread (r, h) keeps row r, columns
-// h NC .. of the task's blocks in registers: column sums stay inside a wave, row sums
-// cross the waves through LDS (two barriers per task), and the reflector's scalars and
-// v are formed redundantly by every column group from column 0, which every thread
-// holds for its row.
+__device__ inline zc fnma_z(zc a, zc b, zc c) {          // c - a b
+  return mkz(fma(-a.re, b.re, fma(a.im, b.im, c.re)), fma(-a.re, b.im, fma(-a.im, b.re, c.im)));
+}
+__device__ inline zc fnma_zc(zc a, zc b, zc c) {         // c - a conj(b)
+  return mkz(fma(-a.re, b.re, fma(-a.im, b.im, c.re)), fma(a.re, b.im, fma(-a.im, b.re, c.im)));
+}
+
+// ZLARFG as above for the chase's latency chain: beta from one reciprocal square root
+// (two Newton steps, then a correction of the root), 1/(alpha - beta) from one reciprocal;
+// where squares near the range's ends would not do, as above
+__device__ inline void larfg_fast(zc alpha, double xn2, zc& beta, zc& tau, zc& scale) {
+  const bool ident = xn2 == 0.0 && alpha.im == 0.0;
+  const double n2 = ident ? 1.0 : alpha.re * alpha.re + alpha.im * alpha.im + xn2;
+  if (!(n2 > 1e-280 && n2 < 1e280)) {
+    larfg(alpha, xn2, beta, tau, scale);
+    return;
+  }
+  double y = __builtin_amdgcn_rsq(n2);
+  const double hn = 0.5 * n2;
+  y = fma(y, fma(-hn * y, y, 0.5), y);
+  y = fma(y, fma(-hn * y, y, 0.5), y);
+  double nrm = n2 * y;
+  nrm = fma(fma(-nrm, nrm, n2), 0.5 * y, nrm);
+  const double sg = alpha.re >= 0.0 ? -1.0 : 1.0;
+  const double b = sg * nrm, rb = sg * y;
+  const double dr = alpha.re - b;               // same signs: no cancellation
+  const double den = fma(dr, dr, alpha.im * alpha.im);
+  double rd = __builtin_amdgcn_rcp(den);
+  rd = fma(rd, fma(-den, rd, 1.0), rd);
+  rd = fma(rd, fma(-den, rd, 1.0), rd);
+  beta = ident ? alpha : mkz(b, 0.0);
+  tau = ident ? mkz(0, 0) : mkz(-dr * rb, -alpha.im * rb);
+  scale = ident ? mkz(0, 0) : mkz(dr * rd, -alpha.im * rd);
+}
+
+// One element by a buffer load that the caches of other XCDs see (sc1), 16 bytes at once;
+// offsets past the buffer's end give zero.  Aux bit 4 is sc1 on gfx94x and gfx950.
+__device__ inline __amdgpu_buffer_rsrc_t dev_buffer(void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(bytes > 0xFFFFFFF0ull ? 0xFFFFFFF0ull : bytes), 0x00027000);
+}
+__device__ inline zc ld_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff) {
+  return __builtin_bit_cast(zc, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 16));
+}
+// device-scope store of one element at a base that is uniform in the wave plus a byte offset
+__device__ inline void st_dev_at(zc* base, unsigned off, zc v) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  const d2 x = {v.re, v.im};
+  __asm__ volatile("global_store_dwordx4 %0, %1, %2 sc1" ::"v"(off), "v"(x), "s"(base) : "memory");
+}
+
+__device__ inline double first_lane(double x) {
+  const unsigned long long v = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)v), hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__device__ inline zc first_lane(zc v) { return mkz(first_lane(v.re), first_lane(v.im)); }
+
+// a flag in LDS: LDS operations of a wave execute in order, so a wave's stores before
+// lds_set are seen by a wave whose lds_get returned the value, and its loads are done
+__device__ inline void lds_set(int* f, int v) {
+  __asm__ volatile("" ::: "memory");
+  __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __asm__ volatile("" ::: "memory");
+}
+__device__ inline int lds_get(int* f) {
+  const int v = __builtin_amdgcn_readfirstlane(__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+  __asm__ volatile("" ::: "memory");
+  return v;
+}
+
+// Band -> tridiagonal.  A workgroup takes SW consecutive sweeps at a time (a group, claimed
+// in order from a counter), one wave each, and one wave more that loads.  Task k of sweep s
+// needs the tasks <= k + 1 of sweep s - 1 (the later ones touch only rows below).  The
+// blocks move from sweep to sweep through rings of LDS slots with a counter of tasks
+// written and one of tasks read, so that no wave waits at a barrier; only the group's ends
+// meet global memory: the loader fetches what the sweep before the group left, the last
+// sweep stores its blocks and publishes the count of a task one task later, when its stores
+// are complete (device-scope accesses, no cache maintenance).  Every wait is bounded, and
+// past the limit the error flag makes every workgroup return.
+//
+// An LDS slot holds the window [left block | diagonal block] of a task, element (r, c) at
+// (c - 1) P + r, column 0 at (2B - 1) P + r; of the diagonal block the lower triangle counts
+// (what lies above it is written and not read).  The tracked rows follow.  The next sweep
+// reads its blocks one row and column on: rows 1 .. B - 1 of the slot, and for its last row
+// row 0 of the slot of the next task (in the left block zero but for its last column: row B
+// of every slot's first columns stays zero).
+//
+// What bounds it is the chain of 2 N dependent tasks, so a task is arranged for its latency,
+// and that is its instruction count (a SIMD issues a wave's instructions four to five cycles
+// apart, dependent or not) and its LDS traffic (about 70 cycles a round trip, 40 for every
+// 16-byte access of a wave): lane (r, hg) keeps row r and NC columns of the two blocks in
+// registers, exchanges go by swaps and DPP, and a row vector gets to the columns through LDS.
+// Measured at N = 5184: 21.3 ms for band 16 (4.1 us a sweep, about 3600 cycles a task),
+// 50.8 ms for band 32, whose wave holds four times the elements; a sweep per workgroup of
+// four waves that met at barriers and moved every block through memory took 62 ms (band 32,
+// 12 us a sweep).  With eight waves a sweep and barriers, band 16 took 28 ms.
 template <int B>
-__global__ __launch_bounds__(256) void k_chase(ChaseArgs a) {
-  constexpr int LB2 = (B == 32) ? 5 : 4;
-  constexpr int NC = B * B / 256;
-  constexpr int LNC = (NC == 4) ? 2 : 0;
-  constexpr int NG = 256 / B;                  // column groups
-  __shared__ zc red1[4 * B], red2[4 * B];
-  __shared__ int flag;
-  const int t = threadIdx.x, lane = t & 63;
-  const int r = t & (B - 1), h = t >> LB2;
-  const int c0 = h * NC;
-  const int gb = lane & ~(B - 1);              // lane of row 0 of this thread's group
-  const int N = a.N, b = B;
+__global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseArgs a) {
+  typedef ChaseDim<B> C;
+  constexpr int SW = C::SW, R = C::R, NC = C::NC, P = C::P;
+  constexpr int GPW = 64 / B;                  // column groups
+  constexpr int NV = (6 + GPW - 1) / GPW;      // tracked vectors per column group: hg, hg + GPW, ..
+  constexpr int LB = 2 * B + 1;
+  constexpr unsigned CB = (LB - 1) * (unsigned)sizeof(zc);   // bytes from (r, c) to (r, c + 1) of the band
+  __shared__ zc slot[SW][R][C::SLOT];          // boundary i: what sweep i of the group reads
+  __shared__ zc xw[SW][B], zw[SW][B];          // a wave's own: v, then tau y, of every row; v^H O
+  __shared__ int wrote[SW], read[SW];          // tasks written to and read from a boundary's slots
+  __shared__ int group, bad;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int N = a.N, nrhs = a.nrhs;
   int* const err = a.ctl;
+  for (int i = threadIdx.x; i < SW * R * C::SLOT; i += (SW + 1) * 64) (&slot[0][0][0])[i] = mkz(0, 0);
+  if (threadIdx.x == 0) bad = 0;
+  // wait for *f >= need; seen keeps the last count read
+  auto wait_lds = [&](int* f, int need, int& seen) {
+    for (int n = 0; seen < need; ++n) {
+      seen = lds_get(f);
+      if (seen >= need) break;
+      if (lds_get(&bad) || n > (1 << 25)) {
+        bad = 1;
+        return false;
+      }
+    }
+    return true;
+  };
   for (;;) {
-    if (t == 0) flag = atomicAdd(a.ctl + 32, 1);
     __syncthreads();
-    const int s = flag;
+    if (threadIdx.x == 0) group = atomicAdd(a.ctl + 32, 1);
+    if ((int)threadIdx.x < SW) wrote[threadIdx.x] = read[threadIdx.x] = 0;
     __syncthreads();
-    if (s > N - 2) return;
-    const int nt = chase_ntasks(N, b, s);
-    const int ntp = s > 0 ? chase_ntasks(N, b, s - 1) : 0;
-    int lenp = 0;
+    const int gidx = __builtin_amdgcn_readfirstlane(group);
+    const int s0 = gidx * SW;
+    if (s0 > N - 2) return;
+    // each role takes its own opaque copy of the lane, so that the roles' addresses are not
+    // kept in registers side by side
+    int lane = threadIdx.x & 63;
+    __asm__ volatile("" : "+v"(lane));
+    if (wave == SW) {
+      // ---- loader: the tasks of sweep s0 - 1 (s0 = 0: blocks of the band) ----------------
+      const int r = lane / GPW, hg = lane % GPW, c0 = hg * NC;
+      const unsigned bo = (unsigned)(c0 * (LB - 1) + r) * (unsigned)sizeof(zc);
+      const int w0 = (hg == 0) ? (2 * B - 1) * P : (c0 - 1) * P;   // column c0 of the left block in a slot
+      const __amdgpu_buffer_rsrc_t bd = dev_buffer(a.BD, (size_t)N * LB * sizeof(zc));
+      const __amdgpu_buffer_rsrc_t gb = dev_buffer(a.gc, (size_t)nrhs * N * sizeof(zc));
+      const int ntp = chase_ntasks(N, B, s0 - 1);
+      int have = (gidx == 0) ? ntp : 0, seen = 0;
+      for (int k = 0; k < ntp; ++k) {
+        for (long long n = 0; have < k + 1; ++n) {
+          have = __builtin_amdgcn_readfirstlane(
+              __hip_atomic_load(a.prog + gidx - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+          if (have >= k + 1) break;
+          if (n > a.spin_limit ||
+              ((n & 63) == 63 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+            lds_set(&bad, 1);
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+          }
+        }
+        // past the last row and above the diagonal something else is read and not used
+        const int st = s0 + k * B;
+        const unsigned sb = (unsigned)st * LB * (unsigned)sizeof(zc);
+        zc o[NC], d[NC], g[NV];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) o[q] = ld_buf(bd, bo + q * CB, k > 0 ? sb - B * CB : 0u);
+#pragma unroll
+        for (int q = 0; q < NC; ++q) d[q] = ld_buf(bd, bo + q * CB, sb);
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+          if (u * GPW < nrhs)
+            g[u] = ld_buf(gb, (unsigned)((hg + u * GPW) * N + r) * (unsigned)sizeof(zc), (unsigned)st * (unsigned)sizeof(zc));
+        if (!wait_lds(&read[0], k + 1 - R, seen)) return;
+        zc* const sl = slot[0][k & (R - 1)] + r;
+#pragma unroll
+        for (int q = 0; q < NC; ++q) sl[q == 0 ? w0 : (c0 + q - 1) * P] = o[q];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) sl[(c0 + q + B - 1) * P] = d[q];
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+          if (hg + u * GPW < nrhs) sl[C::G + (hg + u * GPW) * P] = g[u];
+        lds_set(&wrote[0], k + 1);
+      }
+      continue;
+    }
+    // ---- sweep s ------------------------------------------------------------------------
+    const int s = s0 + wave;
+    if (s > N - 2) continue;
+    const int r = lane / GPW, hg = lane % GPW, c0 = hg * NC;
+    const unsigned bo = (unsigned)(c0 * (LB - 1) + r) * (unsigned)sizeof(zc);
+    const bool last = wave == SW - 1 || s == N - 2;
+    const int nt = chase_ntasks(N, B, s), ntp = chase_ntasks(N, B, s - 1);
+    const int w0 = (hg == 0) ? (2 * B - 1) * P : (c0 - 1) * P;   // column c0 of the left block in a slot
+    const bool lastrow = r == B - 1, corner = lastrow && hg == GPW - 1;
+    int seen_w = 0, seen_r = 0;
+    zc* const xv = xw[wave];
     zc taup = mkz(0, 0);
     zc vp[NC];                                 // previous reflector at this thread's columns
 #pragma unroll
     for (int q = 0; q < NC; ++q) vp[q] = mkz(0, 0);
+    auto publish = [&](int k) {                // the stores of task k - 1 are complete
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (lane == 0) __hip_atomic_store(a.prog + gidx, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
     for (int k = 0; k < nt; ++k) {
-      if (s > 0) {
-        if (t == 0) {
-          const int need = min(k + 2, ntp);
-          long long n = 0;
-          int bad = 0;
-          while (__hip_atomic_load(&a.prog[s - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
-            if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || ++n > a.spin_limit) {
-              bad = 1;
-              __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-          }
-          flag = bad;
-        }
-        __syncthreads();
-        if (flag) return;
-      }
-      // rows st..ed of this task; for k >= 1 the previous reflector's rows sp..sp+lenp-1
-      const int sp = s + 1 + (k - 1) * b;
-      const int st = (k == 0) ? s + 1 : sp + lenp;
-      const int ed = min(st + b - 1, N - 1), len = ed - st + 1;
+      if (!wait_lds(&wrote[wave], min(k + 2, ntp), seen_w)) return;
+      const int st = s + 1 + k * B;            // rows st .. st + len - 1
+      const int len = min(B, N - st);
       const bool rin = r < len;
-      // loads: diagonal block (full Hermitian), the block left of it (k >= 1) and its
-      // column 0 for every row, or column s (k = 0); the tracked vector of this group
-      zc D[NC], O[NC];
+      const zc* const s1 = slot[wave][k & (R - 1)];
+      const zc* const s2 = slot[wave][(k + 1) & (R - 1)];
+      zc O[NC], D[NC], g[NV];
 #pragma unroll
-      for (int q = 0; q < NC; ++q) {
+      for (int q = 0; q < NC; ++q)
+        O[q] = *(q == NC - 1 && corner ? s2 + (2 * B - 1) * P : s1 + (c0 + q) * P + r + 1);
+      const zc* const dr = lastrow ? s2 : s1 + B * P + r + 1;       // D(r, 0)
+      const zc* const dc = s1 + (r + B) * P + 1;                    // D(0, r)
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {           // above the diagonal: the conjugate of (c, r)
         const int c = c0 + q;
-        zc v = mkz(0, 0);
-        if (rin && c < len) v = (r >= c) ? ld_dev(&bd(a, st + r, st + c)) : conj(ld_dev(&bd(a, st + c, st + r)));
-        D[q] = v;
-        zc o = mkz(0, 0);
-        if (k > 0 && rin && c < lenp) o = ld_dev(&bd(a, st + r, sp + c));
-        O[q] = o;
+        D[q] = *(c <= r ? dr + c * P : (q == NC - 1 && hg == GPW - 1) ? s2 + r * P : dc + c);
       }
-      zc x0 = mkz(0, 0);
-      if (rin) x0 = (k == 0) ? ld_dev(&bd(a, st + r, s)) : ld_dev(&bd(a, st + r, sp));
-      const bool gq = h < a.nrhs;
-      zc g = (rin && gq) ? ld_dev(&a.gc[(size_t)h * N + st + r]) : mkz(0, 0);
+      // column 0 of the left block (k = 0: column s of the matrix; there is no left block
+      // then, and nothing formed from O is used)
+      zc x0 = *(k > 0 ? s1 + r + 1 : lastrow ? s2 + (2 * B - 1) * P : s1 + (B - 1) * P + r + 1);
+#pragma unroll
+      for (int u = 0; u < NV; ++u)
+        if (u * GPW < nrhs) g[u] = (lastrow ? s2 : s1 + r + 1)[C::G + min(hg + u * GPW, 5) * P];
+      lds_set(&read[wave], k + 1);
+#pragma unroll
+      for (int q = 0; q < NC; ++q)
+        if (c0 + q > r) D[q].im = -D[q].im;
+      if (len < B) {                           // the last task: nothing past row N - 1
+        if (!rin) x0 = mkz(0, 0);
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+          if (!rin) O[q] = mkz(0, 0);
+          if (!(rin && c0 + q < len)) D[q] = mkz(0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+          if (!rin) g[u] = mkz(0, 0);
+      }
       if (k > 0) {
-        // (i) the block times the previous reflector from the right: O -= taup (O vp) vp^H
+        // (i) O -= tau' (O v') v'^H (v'(0) = 1)
         zc w = mkz(0, 0);
 #pragma unroll
         for (int q = 0; q < NC; ++q) w = fma_z(O[q], vp[q], w);
-        w = row_sum<B>(w, red1, t);
-        const zc tw = taup * w;
+        const zc tw = taup * lane_group_sum<B>(w);
 #pragma unroll
-        for (int q = 0; q < NC; ++q) O[q] = O[q] - tw * conj(vp[q]);
-        x0 = x0 - tw;                          // column 0: vp[0] = 1
+        for (int q = 0; q < NC; ++q) O[q] = fnma_zc(tw, vp[q], O[q]);
+        x0 -= tw;
+        if (last) publish(k);
       }
-      // (ii) reflector of x = rows st..ed of the column (ZLARFG), in every column group
-      const double xn2 = group_sum<B>((r >= 1 && rin) ? norm2(x0) : 0.0);
-      const zc alpha = shfl_z(x0, gb);
+      // (ii) the reflector of x0, at the columns too
+      const double xn2 = row_group_sum<B>((r > 0) ? norm2(x0) : 0.0);
       zc beta, tau, scale;
-      larfg(alpha, xn2, beta, tau, scale);
-      const zc vr = (r == 0) ? mkz(1, 0) : (rin ? x0 * scale : mkz(0, 0));
-      zc vc[NC];                               // v at this thread's columns
+      larfg_fast(first_lane(x0), xn2, beta, tau, scale);
+      const zc vr = (r == 0) ? mkz(1, 0) : scale * x0;
+      if (hg == 0) xv[r] = vr;
 #pragma unroll
-      for (int q = 0; q < NC; ++q) vc[q] = shfl_z(vr, gb + c0 + q);
-      if (k > 0) {
-        // (iii) O(:, 1:) <- H^H O(:, 1:): z_c = v^H O(:, c), O -= conj(tau) v z
-        zc tq[NC];
+      for (int q = 0; q < NC; ++q) vp[q] = xv[c0 + q];
+      // (iii) z = v^H O, row quarter u summing columns u NC / 4 ..
+      zc tq[NC];
 #pragma unroll
-        for (int q = 0; q < NC; ++q) tq[q] = fma_conj(vr, O[q], mkz(0, 0));
-        const zc z = col_sums<B, NC>(tq, lane);
-        const zc ctv = conj(tau) * vr;
+      for (int q = 0; q < NC; ++q) tq[q] = fma_conj(vr, O[q], mkz(0, 0));
+      col_sums<B, NC>(tq);
+      if (r % (B / 4) == 0) {
 #pragma unroll
-        for (int q = 0; q < NC; ++q) {
-          const int c = c0 + q;
-          const zc zq = shfl_z(z, gb + (q << (LB2 - LNC)));   // the lane holding column c0 + q
-          if (c == 0) O[q] = (r == 0) ? beta : mkz(0, 0);
-          else O[q] = O[q] - ctv * zq;
-          if (rin && c < lenp) st_dev(&bd(a, st + r, sp + c), O[q]);
-        }
+        for (int q = 0; q < NC / 4; ++q) zw[wave][c0 + (r / (B / 4)) * (NC / 4) + q] = tq[q];
       }
-      // (iv) D <- H^H D H: y = D v, g = v^H y, w = tau y - |tau|^2 g / 2 v, D -= v w^H + w v^H
+      // (iv) D <- H^H D H: y = D v, w = tau y - |tau|^2 (v^H y) / 2 v, D -= v w^H + w v^H
       zc y = mkz(0, 0);
 #pragma unroll
-      for (int q = 0; q < NC; ++q) y = fma_z(D[q], vc[q], y);
-      y = row_sum<B>(y, red2, t);
-      // column s (task 0): beta then zeros, stored only now that every wave has loaded it
-      // (row_sum's barrier)
-      if (k == 0 && h == 0 && rin) st_dev(&bd(a, st + r, s), (r == 0) ? beta : mkz(0, 0));
-      const double gam = group_sum<B>(vr.re * y.re + vr.im * y.im);
-      const zc wr = tau * y - (0.5 * norm2(tau) * gam) * vr;
+      for (int q = 0; q < NC; ++q) y = fma_z(D[q], vp[q], y);
+      y = lane_group_sum<B>(y);
+      const zc ty = tau * y;
+      if (hg == 0) xv[r] = ty;
+      const double kap = 0.5 * norm2(tau) * row_group_sum<B>(fma(vr.re, y.re, vr.im * y.im));
+      const zc wr = mkz(fma(-kap, vr.re, ty.re), fma(-kap, vr.im, ty.im));
+      const zc ctv = conj(tau) * vr;
+      // O(:, 1:) -= conj(tau) v z
+#pragma unroll
+      for (int q = 0; q < NC; ++q) O[q] = fnma_z(ctv, zw[wave][c0 + q], O[q]);
+      if (hg == 0) O[0] = (r == 0) ? beta : mkz(0, 0);
 #pragma unroll
       for (int q = 0; q < NC; ++q) {
-        const int c = c0 + q;
-        const zc wc = shfl_z(wr, gb + c);
-        const zc d = D[q] - vr * conj(wc) - wr * conj(vc[q]);
-        if (rin && c <= r) st_dev(&bd(a, st + r, st + c), (r == c) ? mkz(d.re, 0.0) : d);
+        const zc tyc = xv[c0 + q];
+        const zc wc = mkz(fma(-kap, vp[q].re, tyc.re), fma(-kap, vp[q].im, tyc.im));
+        D[q] = fnma_zc(wr, vp[q], fnma_zc(vr, wc, D[q]));
       }
-      // (v) tracked vector h, rows st..ed: gc -= conj(tau) v (v^H gc)
-      const zc al = group_sum<B>(fma_conj(vr, g, mkz(0, 0)));
-      if (rin && gq) st_dev(&a.gc[(size_t)h * N + st + r], g - vr * (conj(tau) * al));
-      lenp = len;
-      taup = tau;
+      // (v) tracked vectors: gc -= conj(tau) v (v^H gc)
 #pragma unroll
-      for (int q = 0; q < NC; ++q) vp[q] = vc[q];
-      // publish: every wave's stores have completed before the counter moves
-      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (t == 0) __hip_atomic_store(&a.prog[s], k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int q = 0; q < NV; ++q)
+        if (q * GPW < nrhs) g[q] = fnma_z(ctv, row_group_sum<B>(fma_conj(vr, g[q], mkz(0, 0))), g[q]);
+      if (k == 0 && r == 0) {
+        // finished: the subdiagonal of column s, the diagonal and tracked rows of s + 1
+        if (hg == 0) {
+          st_dev(a.BD + (size_t)s * LB + 1, beta);
+          st_dev(a.BD + (size_t)(s + 1) * LB, D[0]);
+        }
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+          if (hg + q * GPW < nrhs) st_dev(a.gc + (size_t)(hg + q * GPW) * N + s + 1, g[q]);
+      }
+      if (last) {
+        if (rin) {
+          zc* bp = a.BD + (size_t)st * LB;
+#pragma unroll
+          for (int q = 0; q < NC; ++q)
+            if (c0 + q <= r) st_dev_at(bp + q * (LB - 1), bo, D[q]);
+          if (k > 0) {
+#pragma unroll
+            for (int q = 0; q < NC; ++q) st_dev_at(bp + (q - B) * (LB - 1), bo, O[q]);
+          }
+#pragma unroll
+          for (int q = 0; q < NV; ++q)
+            if (hg + q * GPW < nrhs)
+              st_dev_at(a.gc + st, (unsigned)((hg + q * GPW) * N + r) * (unsigned)sizeof(zc), g[q]);
+        }
+      } else {
+        const int nx = min(wave + 1, SW - 1);
+        if (!wait_lds(&read[nx], k + 1 - R, seen_r)) return;
+        zc* const so = slot[nx][k & (R - 1)] + r;
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+          so[q == 0 ? w0 : (c0 + q - 1) * P] = O[q];
+          so[(c0 + q + B - 1) * P] = D[q];
+        }
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+          if (hg + q * GPW < nrhs) so[C::G + (hg + q * GPW) * P] = g[q];
+        lds_set(&wrote[nx], k + 1);
+      }
+      taup = tau;
     }
+    if (last) publish(nt);
   }
 }
 
@@ -1396,16 +1611,18 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
   ChaseArgs ca;
   ca.BD = w.BD;
   ca.N = N;
-  ca.b = b;
-  ca.LB = w.LB;
   ca.gc = w.gc;
   ca.nrhs = nrhs;
   ca.prog = w.prog;
   ca.ctl = w.err;
-  ca.spin_limit = 1ll << 20;   // polls of about a microsecond each: about a second
-  const int P = min(N - 1, 128);   // workgroups claiming sweeps
-  if (b == 16) hipLaunchKernelGGL(k_chase<16>, dim3(P), dim3(256), 0, s, ca);
-  else hipLaunchKernelGGL(k_chase<32>, dim3(P), dim3(256), 0, s, ca);
+  ca.spin_limit = 1ll << 21;   // polls of about half a microsecond each: about a second
+  // groups of sweeps that can be at work at once: each follows the one before by more than
+  // two tasks a sweep
+  const int sw = (b == 16) ? ChaseDim<16>::SW : ChaseDim<32>::SW;
+  const int ngrp = (N - 1 + sw - 1) / sw;
+  const int P = min(ngrp, min(256, chase_ntasks(N, b, 0) / (2 * sw) + 4));
+  if (b == 16) hipLaunchKernelGGL(k_chase<16>, dim3(P), dim3((sw + 1) * 64), 0, s, ca);
+  else hipLaunchKernelGGL(k_chase<32>, dim3(P), dim3((sw + 1) * 64), 0, s, ca);
   hipLaunchKernelGGL(k_band_finish, dim3((N + 255) / 256), dim3(256), 0, s, w.BD, N, w.LB, d, e, w.gc, g, nrhs,
                      w.err, status);
   WTB_LAUNCH_CHECK();
