@@ -1107,19 +1107,17 @@ __device__ inline void larfg_fast(zc alpha, double xn2, zc& beta, zc& tau, zc& s
   scale = ident ? mkz(0, 0) : mkz(dr * rd, -alpha.im * rd);
 }
 
-// One element by a buffer load that the caches of other XCDs see (sc1), 16 bytes at once;
-// offsets past the buffer's end give zero.  Aux bit 4 is sc1 on gfx94x and gfx950.
+// One element by a buffer load or store that the caches of other XCDs see (sc1), 16 bytes at
+// once; loads past the buffer's end give zero.  Aux bit 4 is sc1 on gfx94x and gfx950.
 __device__ inline __amdgpu_buffer_rsrc_t dev_buffer(void* p, size_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(bytes > 0xFFFFFFF0ull ? 0xFFFFFFF0ull : bytes), 0x00027000);
 }
 __device__ inline zc ld_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff) {
   return __builtin_bit_cast(zc, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 16));
 }
-// device-scope store of one element at a base that is uniform in the wave plus a byte offset
-__device__ inline void st_dev_at(zc* base, unsigned off, zc v) {
-  typedef double d2 __attribute__((ext_vector_type(2)));
-  const d2 x = {v.re, v.im};
-  __asm__ volatile("global_store_dwordx4 %0, %1, %2 sc1" ::"v"(off), "v"(x), "s"(base) : "memory");
+__device__ inline void st_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff, zc v) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rs, voff, soff, 16);
 }
 
 __device__ inline double first_lane(double x) {
@@ -1183,6 +1181,8 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int N = a.N, nrhs = a.nrhs;
   int* const err = a.ctl;
+  const __amdgpu_buffer_rsrc_t bd = dev_buffer(a.BD, (size_t)N * LB * sizeof(zc));
+  const __amdgpu_buffer_rsrc_t gb = dev_buffer(a.gc, (size_t)nrhs * N * sizeof(zc));
   for (int i = threadIdx.x; i < SW * R * C::SLOT; i += (SW + 1) * 64) (&slot[0][0][0])[i] = mkz(0, 0);
   if (threadIdx.x == 0) bad = 0;
   // wait for *f >= need; seen keeps the last count read
@@ -1214,8 +1214,6 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
       const int r = lane / GPW, hg = lane % GPW, c0 = hg * NC;
       const unsigned bo = (unsigned)(c0 * (LB - 1) + r) * (unsigned)sizeof(zc);
       const int w0 = (hg == 0) ? (2 * B - 1) * P : (c0 - 1) * P;   // column c0 of the left block in a slot
-      const __amdgpu_buffer_rsrc_t bd = dev_buffer(a.BD, (size_t)N * LB * sizeof(zc));
-      const __amdgpu_buffer_rsrc_t gb = dev_buffer(a.gc, (size_t)nrhs * N * sizeof(zc));
       const int ntp = chase_ntasks(N, B, s0 - 1);
       int have = (gidx == 0) ? ntp : 0, seen = 0;
       for (int k = 0; k < ntp; ++k) {
@@ -1377,18 +1375,18 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
       }
       if (last) {
         if (rin) {
-          zc* bp = a.BD + (size_t)st * LB;
+          const unsigned sb = (unsigned)st * LB * (unsigned)sizeof(zc);
 #pragma unroll
           for (int q = 0; q < NC; ++q)
-            if (c0 + q <= r) st_dev_at(bp + q * (LB - 1), bo, D[q]);
+            if (c0 + q <= r) st_buf(bd, bo + q * CB, sb, D[q]);
           if (k > 0) {
 #pragma unroll
-            for (int q = 0; q < NC; ++q) st_dev_at(bp + (q - B) * (LB - 1), bo, O[q]);
+            for (int q = 0; q < NC; ++q) st_buf(bd, bo + q * CB, sb - B * CB, O[q]);
           }
 #pragma unroll
           for (int q = 0; q < NV; ++q)
             if (hg + q * GPW < nrhs)
-              st_dev_at(a.gc + st, (unsigned)((hg + q * GPW) * N + r) * (unsigned)sizeof(zc), g[q]);
+              st_buf(gb, (unsigned)((hg + q * GPW) * N + r) * (unsigned)sizeof(zc), (unsigned)st * (unsigned)sizeof(zc), g[q]);
         }
       } else {
         const int nx = min(wave + 1, SW - 1);
