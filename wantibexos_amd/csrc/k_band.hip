@@ -979,31 +979,6 @@ __global__ void k_conj_vec(int n, const zc* __restrict__ x, zc* __restrict__ y) 
   if (i < n) y[i] = conj(x[i]);
 }
 
-// ---------------------------------------------------------------------------
-// stage 2: bulge chasing
-// ---------------------------------------------------------------------------
-template <int B>
-struct ChaseDim {
-  static constexpr int SW = (B == 16) ? 3 : 2;   // sweeps per workgroup, one wave each
-  static constexpr int R = (B == 16) ? 4 : 2;    // LDS slots per boundary between sweeps
-  static constexpr int NC = B * B / 64;          // columns per thread
-  static constexpr int P = B + 1;                // column length of a slot
-  static constexpr int G = 2 * B * P;            // offset of its tracked rows
-  static constexpr int SLOT = G + 6 * P;
-};
-
-struct ChaseArgs {
-  zc* BD;            // [N][2 B + 1]
-  int N;
-  zc* gc;            // nrhs x N (conjugated tracked vectors)
-  int nrhs;
-  int* prog;         // [group] tasks that the group's last sweep has finished
-  int* ctl;          // [0] error flag, [32] next group to claim
-  long long spin_limit;
-};
-
-__host__ __device__ inline int chase_ntasks(int N, int b, int s) { return 1 + (N - 2 - s) / b; }
-
 // Lane halves and 16-lane rows by the swap instructions (VALU, no LDS round trip): after
 // swap32(a, b) lane l < 32 holds a(l) and a(l + 32), lane l >= 32 b(l - 32) and b(l); swap16
 // does the same within each pair of 16-lane rows.  a + b is then a sum over that lane bit,
@@ -1030,6 +1005,554 @@ __device__ inline double add16(double a, double b) {
   swap16(a, b);
   return a + b;
 }
+
+// sum over groups of SUB (8 or 16) consecutive lanes, the same bits in each: ^1, ^2, then
+// i <-> 7 - i and i <-> 15 - i
+template <int SUB>
+__device__ inline zc sub_sum(zc x) {
+  x += dpp_z<0xB1>(x);
+  x += dpp_z<0x4E>(x);
+  x += dpp_z<0x141>(x);
+  if constexpr (SUB == 16) x += dpp_z<0x140>(x);
+  return x;
+}
+
+__device__ inline zc fnma_z(zc a, zc b, zc c) {          // c - a b
+  return mkz(fma(-a.re, b.re, fma(a.im, b.im, c.re)), fma(-a.re, b.im, fma(-a.im, b.re, c.im)));
+}
+__device__ inline zc fnma_zc(zc a, zc b, zc c) {         // c - a conj(b)
+  return mkz(fma(-a.re, b.re, fma(-a.im, b.im, c.re)), fma(a.re, b.im, fma(-a.im, b.re, c.im)));
+}
+
+// ZLARFG as above for latency chains: beta from one reciprocal square root
+// (two Newton steps, then a correction of the root), 1/(alpha - beta) from one reciprocal;
+// where squares near the range's ends would not do, as above
+__device__ inline void larfg_fast(zc alpha, double xn2, zc& beta, zc& tau, zc& scale) {
+  const bool ident = xn2 == 0.0 && alpha.im == 0.0;
+  const double n2 = ident ? 1.0 : alpha.re * alpha.re + alpha.im * alpha.im + xn2;
+  if (!(n2 > 1e-280 && n2 < 1e280)) {
+    larfg(alpha, xn2, beta, tau, scale);
+    return;
+  }
+  double y = __builtin_amdgcn_rsq(n2);
+  const double hn = 0.5 * n2;
+  y = fma(y, fma(-hn * y, y, 0.5), y);
+  y = fma(y, fma(-hn * y, y, 0.5), y);
+  double nrm = n2 * y;
+  nrm = fma(fma(-nrm, nrm, n2), 0.5 * y, nrm);
+  const double sg = alpha.re >= 0.0 ? -1.0 : 1.0;
+  const double b = sg * nrm, rb = sg * y;
+  const double dr = alpha.re - b;               // same signs: no cancellation
+  const double den = fma(dr, dr, alpha.im * alpha.im);
+  double rd = __builtin_amdgcn_rcp(den);
+  rd = fma(rd, fma(-den, rd, 1.0), rd);
+  rd = fma(rd, fma(-den, rd, 1.0), rd);
+  beta = ident ? alpha : mkz(b, 0.0);
+  tau = ident ? mkz(0, 0) : mkz(-dr * rb, -alpha.im * rb);
+  scale = ident ? mkz(0, 0) : mkz(dr * rd, -alpha.im * rd);
+}
+
+// One element by a buffer load or store that the caches of other XCDs see (sc1), 16 bytes at
+// once; loads past the buffer's end give zero.  Aux bit 4 is sc1 on gfx94x and gfx950.
+__device__ inline __amdgpu_buffer_rsrc_t dev_buffer(void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(bytes > 0xFFFFFFF0ull ? 0xFFFFFFF0ull : bytes), 0x00027000);
+}
+__device__ inline zc ld_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff) {
+  return __builtin_bit_cast(zc, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 16));
+}
+__device__ inline void st_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff, zc v) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rs, voff, soff, 16);
+}
+
+// ---------------------------------------------------------------------------
+// stage 1, COMPLEX*16 matrix: the whole panel step up to Y in one launch
+// ---------------------------------------------------------------------------
+#define QP_WG 64          // most workgroups of the launch (panel rows up to 256 QP_WG)
+
+// workgroup barrier for LDS traffic alone: global loads and stores stay in flight
+__device__ inline void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// a uniform lane's value, in scalar registers
+__device__ inline double lane_value(double x, int l) {
+  const unsigned long long v = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_readlane((int)v, l), hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__device__ inline zc lane_value(zc v, int l) { return mkz(lane_value(v.re, l), lane_value(v.im, l)); }
+
+// Values handed from every workgroup to every workgroup: slot [round][workgroup][B], each
+// slot written once per panel and filled with the bits ~0 before (no arithmetic result has
+// them), so that a reader polls the value itself: no counter, no fence, one store and one
+// load apart.  Rounds 0 .. B - 1 are the panel's columns, B .. B + 5 the tracked vectors;
+// entry nwg of a column's round is row c of the panel.
+struct QrPanelArgs {
+  zc* A;                 // the matrix, ld
+  int ld, N;
+  int c0, r0, m, k;      // panel columns c0 .. c0 + B - 1, rows r0 .. N - 1 (m), k reflectors
+  zc *V, *Y;             // [B][N]
+  zc* Tm;                // T(q, c) at [c][q]
+  zc* gc;                // nrhs x N
+  int nrhs;
+  zc *ex, *ex_next;      // this panel's slots; the next panel's, filled here
+  int exs;               // workgroups per round of the slots
+  int nwg;
+  int* err;
+  int spin_limit;
+};
+
+__device__ inline bool is_empty(zc v) {
+  return __builtin_bit_cast(unsigned long long, v.re) == ~0ull || __builtin_bit_cast(unsigned long long, v.im) == ~0ull;
+}
+
+template <int B>
+__host__ __device__ constexpr size_t qr_slots(int nwg_max) { return (size_t)(B + 6) * (nwg_max + 1) * B; }
+
+// Householder QR of the panel (ZGEQRF's reflectors), V, R, T (ZLARFT), Y = V T and
+// gc <- Q^H gc.  Workgroup w keeps rows 256 w .. of the panel in registers, one a thread.
+// Per column one exchange: the sums d_j = sum over rows i > c of conj(x_i) row_j(i), for the
+// columns j > c not yet reduced, j = c (|x|^2) and the finished reflectors j < c alike, and
+// row c.  From these every workgroup forms the reflector, the update of its rows
+// (v^H P_j = P(c, j) + conj(scale) d_j) and column c of T (v_j^H v_c = conj(V(c, j)) +
+// scale conj(d_j)), the latter while the next column's sums are on their way; thread
+// (i, j sub) holds T(i, j).
+//
+// Bound by latency: about 4300 cycles a column, of which the exchange (store, first load
+// that sees it) takes about half.  The launch needs every workgroup resident, so it is used
+// for at most QP_WG of them: eight streams' launches fit at two workgroups per compute unit.
+template <int B>
+__global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
+  constexpr int SUB = 256 / B;                 // threads per exchanged value
+  constexpr int NT = B / SUB;                  // T entries per thread
+  __shared__ zc lp[4][4][B / 4][16];           // partial sums [wave][row quarter][column][lane]
+  __shared__ zc dq[B], rq[B], rowc[B];         // totals and row c; row c on its way out
+  __shared__ zc Ts[B][B + 1];
+  __shared__ zc t1s[6][B], t2s[6][B];
+  __shared__ int bad;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int i = blockIdx.x * 256 + t;          // panel row
+  const bool live = i < a.m;
+  const int q = t / SUB, sub = t % SUB;        // exchanged value; T row and its columns sub + SUB u
+  const size_t N = a.N;
+  const unsigned RS = (unsigned)(a.exs * B) * (unsigned)sizeof(zc);   // bytes per round
+  const __amdgpu_buffer_rsrc_t ex = dev_buffer(a.ex, (size_t)(B + 6) * RS);
+  const unsigned mine = (unsigned)(blockIdx.x * B) * (unsigned)sizeof(zc);
+  if (t == 0) bad = 0;
+  zc row[B];
+  {
+    const zc* ap = a.A + (size_t)(a.r0 + min(i, a.m - 1)) + (size_t)a.ld * a.c0;
+#pragma unroll
+    for (int j = 0; j < B; ++j) row[j] = ap[(size_t)a.ld * j];
+    if (!live) {
+#pragma unroll
+      for (int j = 0; j < B; ++j) row[j] = mkz(0, 0);
+    }
+  }
+  // the next panel's slots
+  const zc empty = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
+  for (int e = t; e < (B + 6) * B; e += 256) a.ex_next[(size_t)(e / B) * a.exs * B + (size_t)blockIdx.x * B + e % B] = empty;
+  if (blockIdx.x == 0)
+    for (int e = t; e < B * B; e += 256) a.ex_next[(size_t)(e / B) * a.exs * B + (size_t)a.nwg * B + e % B] = empty;
+
+  // sum over the workgroup of B values a thread: halved over the lane halves and the rows of
+  // 16, the rest through LDS; threads (q, .) end with the sum of value q
+  auto block_sums = [&](zc (&v)[B]) {
+#pragma unroll
+    for (int j = 0; j < B / 2; ++j) v[j] = mkz(add32(v[j].re, v[j + B / 2].re), add32(v[j].im, v[j + B / 2].im));
+#pragma unroll
+    for (int j = 0; j < B / 4; ++j) {
+      v[j] = mkz(add16(v[j].re, v[j + B / 4].re), add16(v[j].im, v[j + B / 4].im));
+      lp[wave][lane >> 4][j][lane & 15] = v[j];
+    }
+    lds_barrier();
+    zc s = mkz(0, 0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int u = 0; u < 16; u += SUB) s += lp[w][q / (B / 4)][q % (B / 4)][sub + u];
+    return sub_sum<SUB>(s);
+  };
+  // value q of rounds c .. c + nr - 1 summed over the workgroups, and entry nwg of round c
+  // (row c); all loads of a pass at once, repeated until every value is there (bounded)
+  auto gather = [&](auto nrc, int c, int nr, bool with_row, zc* tot, zc& rowv) {
+    constexpr int NR = decltype(nrc)::value, U = NR == 1 ? 4 : 2;
+    const int n = a.nwg + (with_row ? 1 : 0);
+    zc s[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) s[r] = mkz(0, 0);
+    for (int w0 = sub; w0 < n; w0 += U * SUB) {
+      zc v[NR][U];
+      for (int tries = 0;; ++tries) {
+        bool ok = true;
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (r < nr)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              v[r][u] = ld_buf(ex, (unsigned)(min(w0 + u * SUB, n - 1) * B + q) * (unsigned)sizeof(zc), (c + r) * RS);
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (r < nr)
+#pragma unroll
+            for (int u = 0; u < U; ++u) ok = ok && !is_empty(v[r][u]);
+        if (ok) break;
+        if (tries > a.spin_limit ||
+            ((tries & 255) == 255 && __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+          bad = 1;
+          __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int w = w0 + u * SUB;
+        if (w < a.nwg) {
+#pragma unroll
+          for (int r = 0; r < NR; ++r)
+            if (r < nr) s[r] += v[r][u];
+        } else if (with_row && w == a.nwg) {
+          rowv = v[0][u];
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (r < nr) tot[r] = sub_sum<SUB>(s[r]);
+  };
+
+  zc T[NT], gcol[NT], taup = mkz(0, 0);
+#pragma unroll
+  for (int u = 0; u < NT; ++u) T[u] = mkz(0, 0);
+  // column c of T: T(0:c, c) = -tau T(0:c, 0:c) (V^H v_c)(0:c), T(c, c) = tau
+  auto t_column = [&](int c) {
+    zc s = mkz(0, 0);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+      if (sub + SUB * u < c) s = fma_z(T[u], gcol[u], s);
+    s = sub_sum<SUB>(s);
+    const zc v = (q < c) ? mkz(0, 0) - taup * s : (q == c) ? taup : mkz(0, 0);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+      if (sub + SUB * u == c) T[u] = v;
+  };
+  // four columns at a time, then the registers turn by four: in block cb register p holds
+  // column (p + 4 cb) % B, so that the column at work is register cc, a constant
+  for (int cb = 0; cb < B / 4; ++cb) {
+    const int base = 4 * cb;
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) {
+      const int c = base + cc;
+      if (c < a.k) {
+        if (blockIdx.x == 0 && i == c) {
+#pragma unroll
+          for (int p = 0; p < B; ++p) rowc[p] = row[p];
+        }
+        const zc x = row[cc];
+        const zc xm = (i > c) ? x : mkz(0, 0);
+        zc v[B];
+#pragma unroll
+        for (int p = 0; p < B; ++p) v[p] = fma_conj(xm, row[p], mkz(0, 0));
+        const zc part = block_sums(v);
+        if (sub == 0) st_buf(ex, mine + q * (unsigned)sizeof(zc), c * RS, part);
+        if (blockIdx.x == 0 && sub == 1) st_buf(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
+        if (c > 0) t_column(c - 1);            // while the sums are on their way
+        zc rowv = mkz(0, 0);
+        zc tot;
+        gather(std::integral_constant<int, 1>{}, c, 1, true, &tot, rowv);
+        if (sub == 0) dq[q] = tot;
+        if (sub == a.nwg % SUB) rq[q] = rowv;
+        lds_barrier();
+        if (bad) return;
+        // lane l of every wave: register l % B of row c and its sum
+        const zc dl = dq[lane % B], rl = rq[lane % B];
+        zc beta, scale;
+        larfg_fast(lane_value(rl, cc), lane_value(dl.re, cc), beta, taup, scale);
+        // v^H P of the columns not yet reduced
+        zc wl = fma_conj(scale, dl, rl);
+        if (lane % B <= cc || lane % B >= B - base) wl = mkz(0, 0);
+        const zc vi = (i > c) ? x * scale : (i == c ? mkz(1, 0) : mkz(0, 0));
+        const zc cv = conj(taup) * vi;
+#pragma unroll
+        for (int p = cc + 1; p < B; ++p) row[p] = fnma_z(cv, lane_value(wl, p), row[p]);
+        row[cc] = (i == c) ? beta : (i > c ? vi : x);
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+          const int p = (sub + SUB * u - base) & (B - 1);
+          gcol[u] = fma_z(scale, conj(dq[p]), conj(rq[p]));
+        }
+      }
+    }
+    zc turn[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) turn[p] = row[p];
+#pragma unroll
+    for (int p = 0; p < B - 4; ++p) row[p] = row[p + 4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) row[B - 4 + p] = turn[p];
+  }
+  // R into the matrix, V explicit
+#pragma unroll
+  for (int j = 0; j < B; ++j) {
+    const zc p = row[j];
+    if (live && i <= j) a.A[(size_t)(a.r0 + i) + (size_t)a.ld * (a.c0 + j)] = p;
+    const zc x = (j < a.k) ? (i == j ? mkz(1, 0) : (i > j ? p : mkz(0, 0))) : mkz(0, 0);
+    row[j] = x;
+    if (live) a.V[i + N * j] = x;
+  }
+  // t1 = V^H gc
+  zc g[6];
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    if (r >= a.nrhs) break;
+    g[r] = live ? a.gc[(size_t)r * N + a.r0 + i] : mkz(0, 0);
+    zc v[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) v[j] = fma_conj(row[j], g[r], mkz(0, 0));
+    if (r > 0) lds_barrier();                  // the partial sums of r - 1 are read
+    const zc part = block_sums(v);
+    if (sub == 0) st_buf(ex, mine + q * (unsigned)sizeof(zc), (B + r) * RS, part);
+  }
+  t_column(a.k - 1);
+#pragma unroll
+  for (int u = 0; u < NT; ++u) Ts[q][sub + SUB * u] = T[u];
+  if (a.nrhs > 0) {
+    zc tot[6], none;
+    gather(std::integral_constant<int, 6>{}, B, a.nrhs, false, tot, none);
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+      if (r < a.nrhs && sub == 0) t1s[r][q] = tot[r];
+  }
+  lds_barrier();
+  if (bad) return;
+  if (blockIdx.x == 0)
+    for (int e = t; e < B * B; e += 256) a.Tm[e] = Ts[e % B][e / B];
+  // t2 = T^H t1, gc -= V t2
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    if (r >= a.nrhs) break;
+    zc s = mkz(0, 0);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) s = fma_conj(Ts[sub + SUB * u][q], t1s[r][sub + SUB * u], s);
+    s = sub_sum<SUB>(s);
+    if (sub == 0) t2s[r][q] = s;
+  }
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    if (r >= a.nrhs) break;
+    const zc tl = t2s[r][lane % B];
+    zc s = g[r];
+#pragma unroll
+    for (int j = 0; j < B; ++j) s = fnma_z(row[j], lane_value(tl, j), s);
+    if (live) a.gc[(size_t)r * N + a.r0 + i] = s;
+  }
+  // Y = V T, four columns at a time (T upper triangular)
+  for (int cb = 0; cb < B / 4; ++cb) {
+    zc tl[4], y[4];
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) {
+      tl[cc] = Ts[lane % B][4 * cb + cc];
+      y[cc] = mkz(0, 0);
+    }
+#pragma unroll
+    for (int jb = 0; jb < B / 4; ++jb)
+      if (jb <= cb) {
+#pragma unroll
+        for (int j = 4 * jb; j < 4 * jb + 4; ++j)
+#pragma unroll
+          for (int cc = 0; cc < 4; ++cc) y[cc] = fma_z(row[j], lane_value(tl[cc], j), y[cc]);
+      }
+    if (live) {
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) a.Y[i + N * (4 * cb + cc)] = y[cc];
+    }
+  }
+}
+
+// W = X - 1/2 V (T^H (V^H X)) with X the sum of the K slices of A22 Y, in one launch:
+// workgroup w takes rows 256 w .., its part of M = V^H X on FP64 MFMA (operands straight
+// from memory in the MFMA's layout), one exchange of the B x B parts as above (slots
+// [workgroup][B B]), then Z = T^H M and its rows of W.
+struct QrWArgs {
+  int m, N, ns;          // rows; slices of part (0: X holds the product)
+  const zc *part, *V, *Tm;
+  zc* X;                 // in (ns = 0), out: W
+  zc *ex, *ex_next;
+  int nwg;
+  int* err;
+  int spin_limit;
+};
+
+template <int B>
+__global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
+  constexpr int TI = B / 16, NE = B * B / 256;
+  __shared__ zc buf[4 * B * B];                // the waves' parts, then M, Z, T
+  typedef zc Mat[B][B + 1];
+  zc (*const red)[B * B] = reinterpret_cast<zc(*)[B * B]>(buf);
+  Mat &Ms = *reinterpret_cast<Mat*>(buf), &Zs = *reinterpret_cast<Mat*>(buf + B * (B + 1)),
+      &Ts = *reinterpret_cast<Mat*>(buf + 2 * B * (B + 1));
+  __shared__ int bad;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
+  const size_t N = a.N;
+  const int row0 = blockIdx.x * 256, i = row0 + t;
+  const __amdgpu_buffer_rsrc_t ex = dev_buffer(a.ex, (size_t)a.nwg * B * B * sizeof(zc));
+  if (t == 0) bad = 0;
+  const zc empty = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
+#pragma unroll
+  for (int u = 0; u < NE; ++u) a.ex_next[(size_t)blockIdx.x * B * B + t + 256 * u] = empty;
+  if (a.ns > 0 && i < a.m)
+    for (int c = 0; c < B; ++c) {
+      const zc* pp = a.part + (size_t)c * a.m + i;
+      a.X[i + N * c] = strided_sum(pp, (size_t)a.m * B, 0, a.ns, 1, mkz(0, 0));
+    }
+  __syncthreads();
+  // this wave's 64 rows of M = V^H X
+  d4 mr[TI][TI], mi[TI][TI];
+#pragma unroll
+  for (int x = 0; x < TI; ++x)
+#pragma unroll
+    for (int y = 0; y < TI; ++y) mr[x][y] = mi[x][y] = d4{0, 0, 0, 0};
+  const int w0 = row0 + 64 * wave;
+#pragma unroll 4
+  for (int k0 = 0; k0 < 64; k0 += 4) {
+    const int rr = w0 + k0 + lk;
+    const bool on = rr < a.m;
+    zc av[TI], xv[TI];
+#pragma unroll
+    for (int x = 0; x < TI; ++x) {
+      av[x] = on ? a.V[rr + N * (16 * x + lr)] : mkz(0, 0);
+      xv[x] = on ? a.X[rr + N * (16 * x + lr)] : mkz(0, 0);
+    }
+    // conj(v) x = (vr xr + vi xi) + i (vr xi - vi xr)
+#pragma unroll
+    for (int x = 0; x < TI; ++x)
+#pragma unroll
+      for (int y = 0; y < TI; ++y) {
+        mr[x][y] = mfma16x16x4(av[x].re, xv[y].re, mr[x][y]);
+        mi[x][y] = mfma16x16x4(av[x].re, xv[y].im, mi[x][y]);
+        mr[x][y] = mfma16x16x4(av[x].im, xv[y].im, mr[x][y]);
+        mi[x][y] = mfma16x16x4(-av[x].im, xv[y].re, mi[x][y]);
+      }
+  }
+#pragma unroll
+  for (int x = 0; x < TI; ++x)
+#pragma unroll
+    for (int y = 0; y < TI; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][(16 * x + lk + 4 * r) * B + 16 * y + lr] = mkz(mr[x][y][r], mi[x][y][r]);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = t + 256 * u;
+    const zc p = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+    st_buf(ex, (unsigned)((size_t)blockIdx.x * B * B + e) * (unsigned)sizeof(zc), 0,
+           p);
+  }
+  lds_barrier();                               // red is read
+  for (int e = t; e < B * B; e += 256) Ts[e % B][e / B] = a.Tm[e];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = t + 256 * u;
+    zc s = mkz(0, 0);
+    for (int wg0 = 0; wg0 < a.nwg; wg0 += 8) {
+      zc v[8];
+      for (int tries = 0;; ++tries) {
+        bool ok = true;
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          v[x] = ld_buf(ex, (unsigned)(min(wg0 + x, a.nwg - 1) * (B * B) + e) * (unsigned)sizeof(zc), 0);
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          ok = ok && !is_empty(v[x]);
+        if (ok) break;
+        if (tries > a.spin_limit ||
+            ((tries & 255) == 255 && __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+          bad = 1;
+          __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        if (wg0 + x < a.nwg) s += v[x];
+    }
+    Ms[e / B][e % B] = s;
+  }
+  __syncthreads();
+  if (bad) return;
+  // Z = T^H M
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = t + 256 * u, p = e / B, c = e % B;
+    zc s = mkz(0, 0);
+#pragma unroll 4
+    for (int r = 0; r < B; ++r)
+      if (r <= p) s = fma_conj(Ts[r][p], Ms[r][c], s);
+    Zs[p][c] = s;
+  }
+  __syncthreads();
+  // (V Z)^T by 16 x 16 tiles: MFMA rows over the columns of W, MFMA columns over its rows,
+  // so that a lane's results lie next to its neighbours' in memory
+  for (int rt = 0; rt < 4; ++rt) {
+    const int rr = w0 + 16 * rt + lr;
+    d4 cr[TI], ci[TI];
+#pragma unroll
+    for (int x = 0; x < TI; ++x) cr[x] = ci[x] = d4{0, 0, 0, 0};
+#pragma unroll
+    for (int k0 = 0; k0 < B; k0 += 4) {
+      const zc vv = rr < a.m ? a.V[rr + N * (k0 + lk)] : mkz(0, 0);
+#pragma unroll
+      for (int x = 0; x < TI; ++x) {
+        const zc zz = Zs[k0 + lk][16 * x + lr];
+        cr[x] = mfma16x16x4(zz.re, vv.re, cr[x]);
+        ci[x] = mfma16x16x4(zz.re, vv.im, ci[x]);
+        cr[x] = mfma16x16x4(-zz.im, vv.im, cr[x]);
+        ci[x] = mfma16x16x4(zz.im, vv.re, ci[x]);
+      }
+    }
+    if (rr < a.m)
+#pragma unroll
+      for (int x = 0; x < TI; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const size_t at = rr + N * (16 * x + lk + 4 * r);
+          const zc v = a.X[at];
+          a.X[at] = mkz(v.re - 0.5 * cr[x][r], v.im - 0.5 * ci[x][r]);
+        }
+  }
+}
+
+__global__ void k_fill_empty(zc* p, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
+}
+
+// ---------------------------------------------------------------------------
+// stage 2: bulge chasing
+// ---------------------------------------------------------------------------
+template <int B>
+struct ChaseDim {
+  static constexpr int SW = (B == 16) ? 3 : 2;   // sweeps per workgroup, one wave each
+  static constexpr int R = (B == 16) ? 4 : 2;    // LDS slots per boundary between sweeps
+  static constexpr int NC = B * B / 64;          // columns per thread
+  static constexpr int P = B + 1;                // column length of a slot
+  static constexpr int G = 2 * B * P;            // offset of its tracked rows
+  static constexpr int SLOT = G + 6 * P;
+};
+
+struct ChaseArgs {
+  zc* BD;            // [N][2 B + 1]
+  int N;
+  zc* gc;            // nrhs x N (conjugated tracked vectors)
+  int nrhs;
+  int* prog;         // [group] tasks that the group's last sweep has finished
+  int* ctl;          // [0] error flag, [32] next group to claim
+  long long spin_limit;
+};
+
+__host__ __device__ inline int chase_ntasks(int N, int b, int s) { return 1 + (N - 2 - s) / b; }
 
 // The chase keeps row r of a block in the lanes r (64 / B) + (column group), so that rows
 // lie on the lane's high bits.  Sum over the rows (every lane ends with it): both halves,
@@ -1070,54 +1593,6 @@ __device__ inline zc lane_group_sum(zc x) {
   x += dpp_z<0xB1>(x);
   if constexpr (B == 16) x += dpp_z<0x4E>(x);
   return x;
-}
-
-__device__ inline zc fnma_z(zc a, zc b, zc c) {          // c - a b
-  return mkz(fma(-a.re, b.re, fma(a.im, b.im, c.re)), fma(-a.re, b.im, fma(-a.im, b.re, c.im)));
-}
-__device__ inline zc fnma_zc(zc a, zc b, zc c) {         // c - a conj(b)
-  return mkz(fma(-a.re, b.re, fma(-a.im, b.im, c.re)), fma(a.re, b.im, fma(-a.im, b.re, c.im)));
-}
-
-// ZLARFG as above for the chase's latency chain: beta from one reciprocal square root
-// (two Newton steps, then a correction of the root), 1/(alpha - beta) from one reciprocal;
-// where squares near the range's ends would not do, as above
-__device__ inline void larfg_fast(zc alpha, double xn2, zc& beta, zc& tau, zc& scale) {
-  const bool ident = xn2 == 0.0 && alpha.im == 0.0;
-  const double n2 = ident ? 1.0 : alpha.re * alpha.re + alpha.im * alpha.im + xn2;
-  if (!(n2 > 1e-280 && n2 < 1e280)) {
-    larfg(alpha, xn2, beta, tau, scale);
-    return;
-  }
-  double y = __builtin_amdgcn_rsq(n2);
-  const double hn = 0.5 * n2;
-  y = fma(y, fma(-hn * y, y, 0.5), y);
-  y = fma(y, fma(-hn * y, y, 0.5), y);
-  double nrm = n2 * y;
-  nrm = fma(fma(-nrm, nrm, n2), 0.5 * y, nrm);
-  const double sg = alpha.re >= 0.0 ? -1.0 : 1.0;
-  const double b = sg * nrm, rb = sg * y;
-  const double dr = alpha.re - b;               // same signs: no cancellation
-  const double den = fma(dr, dr, alpha.im * alpha.im);
-  double rd = __builtin_amdgcn_rcp(den);
-  rd = fma(rd, fma(-den, rd, 1.0), rd);
-  rd = fma(rd, fma(-den, rd, 1.0), rd);
-  beta = ident ? alpha : mkz(b, 0.0);
-  tau = ident ? mkz(0, 0) : mkz(-dr * rb, -alpha.im * rb);
-  scale = ident ? mkz(0, 0) : mkz(dr * rd, -alpha.im * rd);
-}
-
-// One element by a buffer load or store that the caches of other XCDs see (sc1), 16 bytes at
-// once; loads past the buffer's end give zero.  Aux bit 4 is sc1 on gfx94x and gfx950.
-__device__ inline __amdgpu_buffer_rsrc_t dev_buffer(void* p, size_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(bytes > 0xFFFFFFF0ull ? 0xFFFFFFF0ull : bytes), 0x00027000);
-}
-__device__ inline zc ld_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff) {
-  return __builtin_bit_cast(zc, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 16));
-}
-__device__ inline void st_buf(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff, zc v) {
-  typedef unsigned u4 __attribute__((ext_vector_type(4)));
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rs, voff, soff, 16);
 }
 
 __device__ inline double first_lane(double x) {
@@ -1435,6 +1910,12 @@ __global__ void k_zero_ints(int* p, int n) {
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+// the exchange slots of one panel parity: k_qr_panel's, then k_qr_w's
+template <int B>
+static size_t qr_ex_elems(int nwg_max) {
+  return qr_slots<B>(nwg_max) + (size_t)nwg_max * B * B;
+}
+
 size_t band_work_bytes(int N, int b, int nrhs) {
   const size_t nwg = (N + PR - 1) / PR + 1;
   const size_t LB = 2 * (size_t)b + 1;
@@ -1460,6 +1941,7 @@ size_t band_work_bytes(int N, int b, int nrhs) {
   add(sizeof(int) * ((size_t)N + 1));         // prog
   add(sizeof(int) * 64);                      // err
   add(sizeof(int) * ((size_t)N / b + 2) * (BMAX + 1));   // panel column counters
+  add(sizeof(zc) * 2 * qr_ex_elems<BMAX>((int)std::min<size_t>(nwg, QP_WG)));   // exchange slots
   return s + 4096;
 }
 
@@ -1501,23 +1983,41 @@ int band_bind(BandWork& w, void* base, int N, int b, int nrhs) {
   w.prog = (int*)take(sizeof(int) * ((size_t)N + 1));
   w.err = (int*)take(sizeof(int) * 64);
   w.bar = (int*)take(sizeof(int) * ((size_t)N / b + 2) * (BMAX + 1));
+  w.ex = (zc*)take(sizeof(zc) * 2 * qr_ex_elems<BMAX>((int)std::min<size_t>(nwg, QP_WG)));
+  w.panel_wg = QP_WG;
   return WTB_OK;
 }
 
-// X = A22 Y (m x B) with enough workgroups to fill the chip: K slices until the grid
-// holds ~1024 workgroups (at most HB_SMAX slices), partials summed in slice order
+// A22 -= V W^H + W V^H
 template <class T, int B>
-static void hmm_band(hipStream_t s, BandWork& w, int m, const T* A, int ld, const zc* Y, zc* X) {
+static void her2k_band(hipStream_t s, BandWork& w, T* H, int ld, int m, int r0, int k) {
+  const int nt = (m + 63) / 64;
+  const bool tev = w.kev && w.kev_used < w.kev_cap;
+  if (tev) hipEventRecord(w.kev[2 * w.kev_used], s);
+  hipLaunchKernelGGL((k_her2k_full<T, B>), dim3(nt * (nt + 1) / 2), dim3(256), 0, s, H, ld, m, r0, w.N, w.V, w.X);
+  if (tev) {
+    hipEventRecord(w.kev[2 * w.kev_used++ + 1], s);
+    w.kev_flops += 8.0 * 0.5 * (double)m * (double)(m + 1) * (2.0 * k);   // lower triangle, 2k products each
+  }
+}
+
+// X = A22 Y (m x B) with enough workgroups to fill the chip: K slices until the grid
+// holds ~1024 workgroups (at most HB_SMAX slices), partials summed in slice order, or (sum
+// false) left to the caller: returns their number, 0 when X holds the product
+template <class T, int B>
+static int hmm_band(hipStream_t s, BandWork& w, int m, const T* A, int ld, const zc* Y, zc* X, bool sum = true) {
   const int rb = (m + HB_R - 1) / HB_R;
   int ns = std::max(1, std::min(HB_SMAX, (1024 + rb - 1) / rb));
   const int kc = ((m + ns - 1) / ns + 31) / 32 * 32;   // a multiple of either K step
   ns = (m + kc - 1) / kc;
   hipLaunchKernelGGL((k_hmm_b<T, B>), dim3(rb, ns), dim3(256), 0, s, m, A, ld, Y, w.N, kc, ns > 1 ? w.hb : nullptr,
                      X, w.N);
+  if (ns > 1 && !sum) return ns;
   if (ns > 1) {
     const size_t tot = (size_t)m * B;
     hipLaunchKernelGGL(k_hmm_sum<B>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, m, ns, w.hb, X, w.N);
   }
+  return 0;
 }
 
 // out0 = A^H Y0 (B x B) and out1 = A^H Y1 (B x n1) over m rows, ld B
@@ -1534,6 +2034,15 @@ static void gram(hipStream_t s, BandWork& w, int m, const zc* A, const zc* Y0, i
 template <class T, int B>
 static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   const int N = w.N, b = B;
+  const int exw = min(w.nwg_max, QP_WG);               // workgroups that the slots hold
+  const size_t exn = qr_ex_elems<B>(exw);
+  // COMPLEX*16 panels of at most QP_WG workgroups: one launch for the panel and one for W
+  // (4 launches a panel).  The limit does not depend on how many streams run, so that the
+  // results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
+  // its stored matrix amplifies.
+  const bool qr = std::is_same<T, zc>::value && B == 16 && w.panel_wg >= (N - b + PR - 1) / PR;
+  if (qr)
+    hipLaunchKernelGGL(k_fill_empty, dim3((unsigned)((2 * exn + 255) / 256)), dim3(256), 0, s, w.ex, 2 * exn);
   for (int p = 0;; ++p) {
     const int c0 = p * b, r0 = c0 + b;
     if (r0 >= N) break;
@@ -1555,6 +2064,18 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
     a.tau = w.tau;
     a.nwg = (m + PR - 1) / PR;
     const dim3 g(a.nwg), blk(PR);
+    if constexpr (std::is_same<T, zc>::value && B == 16)
+      if (qr) {
+        zc *ex = w.ex + (size_t)(p & 1) * exn, *exo = w.ex + (size_t)((p + 1) & 1) * exn;
+        const size_t wo = qr_slots<B>(exw);
+        QrPanelArgs q{H, ld, N, c0, r0, m, k, w.V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20};
+        hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, q);
+        const int ns = hmm_band<T, B>(s, w, m, H + r0 + (size_t)ld * r0, ld, w.Y, w.X, false);
+        QrWArgs x{m, N, ns, w.hb, w.V, w.T, w.X, ex + wo, exo + wo, a.nwg, w.err + 8, 1 << 20};
+        hipLaunchKernelGGL((k_qr_w<B>), g, blk, 0, s, x);
+        her2k_band<T, B>(s, w, H, ld, m, r0, k);
+        continue;
+      }
     if (w.panel_resident > 0 && a.nwg <= w.panel_resident) {
       hipLaunchKernelGGL((k_panel<T, B>), g, blk, 0, s, a, w.V, w.bar + (size_t)p * (BMAX + 1), w.err + 8,
                          (long long)1 << 20);
@@ -1569,15 +2090,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
     hmm_band<T, B>(s, w, m, H + r0 + (size_t)ld * r0, ld, w.Y, w.X);
     gram<B>(s, w, m, w.V, w.X, N, nullptr, 0, w.M, nullptr);
     hipLaunchKernelGGL((k_pW<B>), g, blk, 0, s, m, N, w.V, w.T, w.M, w.X);
-    const int nt = (m + 63) / 64;
-    const bool tev = w.kev && w.kev_used < w.kev_cap;
-    if (tev) hipEventRecord(w.kev[2 * w.kev_used], s);
-    hipLaunchKernelGGL((k_her2k_full<T, B>), dim3(nt * (nt + 1) / 2), dim3(256), 0, s, H, ld, m, r0, N, w.V,
-                       w.X);
-    if (tev) {
-      hipEventRecord(w.kev[2 * w.kev_used++ + 1], s);
-      w.kev_flops += 8.0 * 0.5 * (double)m * (double)(m + 1) * (2.0 * k);   // lower triangle, 2k products each
-    }
+    her2k_band<T, B>(s, w, H, ld, m, r0, k);
   }
   WTB_LAUNCH_CHECK();
   return WTB_OK;
