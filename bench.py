@@ -463,7 +463,7 @@ def main():
     ap.add_argument("--cpu-threads", type=int, default=16)
     ap.add_argument("--reduction", choices=["auto", "one", "two"], default="auto",
                     help="tridiagonal reduction: one-stage Householder, two-stage (dense -> band -> "
-                         "tridiagonal), or by size (auto: two-stage from N = 8192 on, one-stage where "
+                         "tridiagonal), or by type and size (auto: FP64 two-stage, precision form from N = 8192 on; one-stage where "
                          "exciton vectors are formed)")
     ap.add_argument("--band", type=int, default=32, choices=[16, 32], help="two-stage reduction: band width")
     ap.add_argument("--no-graph", action="store_true",

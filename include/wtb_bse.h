@@ -406,7 +406,9 @@ int wtb_bse_plan_set_vectors(wtb_bse_plan* plan, int first, int count);
  * bse_solver-tool-diel.f90:485-492; no counterpart in the reference's arithmetic):
  * two_stage = 0: one-stage blocked Householder; two_stage = 1: dense -> band of width
  * `band` (16 or 32, MFMA panel updates, lower triangle only) -> tridiagonal by bulge
- * chasing; two_stage = -1 (default): the two-stage form for N >= 8192, else one-stage.
+ * chasing; two_stage = -1 (default): the faster one by type and size (WTB_FP64: two-stage
+ * from N = 32 on; WTB_MIXED: from N = 8192 on), with the band width of 16 or 32 that goes
+ * with it when band = 32.
  * Executes that form exciton vectors (BSE_WF, the refinement) always take the one-stage
  * form, whose reflectors they need.                                                    */
 int wtb_bse_plan_set_reduction(wtb_bse_plan* plan, int two_stage, int band);

@@ -519,8 +519,9 @@ class BSEPlan:
 
     def set_reduction(self, two_stage=None, band=32):
         """Tridiagonal reduction: two-stage (True: dense -> band -> tridiagonal), one-stage
-        Householder (False), or by size (None, the default: two-stage from N = 8192 on);
-        band width 16 or 32."""
+        Householder (False), or the faster one by type and size (None, the default: plain form
+        two-stage from N = 32 on, precision form from N = 8192 on); band width 16 or 32 (with
+        None and 32 the one that goes with the size)."""
         mode = -1 if two_stage is None else int(bool(two_stage))
         _check(lib().wtb_bse_plan_set_reduction(self.h, mode, int(band)))
 

@@ -1916,6 +1916,8 @@ static size_t qr_ex_elems(int nwg_max) {
   return qr_slots<B>(nwg_max) + (size_t)nwg_max * B * B;
 }
 
+int band_panel_rows() { return QP_WG * PR + 16; }
+
 size_t band_work_bytes(int N, int b, int nrhs) {
   const size_t nwg = (N + PR - 1) / PR + 1;
   const size_t LB = 2 * (size_t)b + 1;

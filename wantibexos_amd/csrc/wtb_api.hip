@@ -35,6 +35,9 @@ __global__ void k_upper_to_lower(int n, const zc* __restrict__ a, int lda, zc* _
   zc v = a[(size_t)j + (size_t)lda * i];      // a(j,i), j <= i
   v = conj(v);
   if (i == j) v.im = 0.0;
+  // any NaN by the usual bits: all bits set mark an empty slot of the panels' exchange
+  if (v.re != v.re) v.re = __builtin_nan("");
+  if (v.im != v.im) v.im = __builtin_nan("");
   h[(size_t)i + (size_t)ldh * j] = v;
 }
 
@@ -105,6 +108,8 @@ struct wtb_ctx {
   hipStream_t stream = nullptr;
 };
 
+static int plan_default_band(bool mixed, int N);
+
 struct wtb_bse_plan {
   wtb_ctx* ctx = nullptr;
   wtb_bse_params prm{};
@@ -168,8 +173,8 @@ struct wtb_bse_plan {
   // back-transformed vectors, HXr = H Xr, rq_res the residual norms |H x - theta x| / |x|
   // stage (d1) form: two-stage (dense -> band -> tridiagonal) when the path needs no
   // eigenvectors, one-stage Householder otherwise (its reflectors feed the back-transform)
-  int two_stage = -1;          // -1: two-stage from kTwoStageMinN on, 0: one-stage, 1: two-stage
-  int band_b = 32;
+  int two_stage = -1;          // -1: by type and size (plan_two_stage), 0: one-stage, 1: two-stage
+  int band_b = 32;             // its band width (plan_default_band unless set)
   BandWork bw;
   void* bandwork = nullptr;
   int nref = 0;
@@ -582,6 +587,7 @@ static int plan_create_impl(wtb_ctx* c, const wtb_tb_model* m, const wtb_bse_par
     return rc;
   }
   tridiag_bind(p->tw, p->triwork, N, nb_panel, p->nrhs);
+  p->band_b = plan_default_band(p->mixed, N);
   if (N >= 2 && ((rc = dmalloc((char**)&p->bandwork, band_work_bytes(N, p->band_b, p->nrhs))) ||
                  (rc = band_bind(p->bw, p->bandwork, N, p->band_b, p->nrhs)))) {
     plan_free(p);
@@ -643,16 +649,29 @@ static void plan_drop_graph(wtb_bse_plan* p);
 // tridiagonal tw.d, tw.e, with Q^T applied to g (may be NULL).  Two-stage when nothing
 // downstream needs the Householder reflectors (exciton vectors, the refinement); its
 // bulge chase reports a stalled wait through status.
-// Matrices of at least this size take the two-stage reduction by default: its MFMA panel
-// updates overtake the one-stage GEMV chain between N = 5184 (one-stage faster) and
-// N = 36864 (two-stage 3.4x to 4.4x faster) on MI355X.
-constexpr int kTwoStageMinN = 8192;
+//
+// By default (two_stage = -1) the COMPLEX*16 matrix takes the two-stage reduction at every
+// size that has a panel.  Whole plan, one-stage / two-stage with band 16, MI355X:
+//   N = 36: 1.11 / 0.77 ms   144: 3.14 / 1.93   576: 11.2 / 6.7   2116: 41.8 / 26.4
+//   5184: 161 / 82           8100: 445 / 186    14400: 2187 / 665
+// Band 16 while the panels run in one launch (band_panel_rows), where its shorter chase
+// outweighs the smaller updates (band 32 with that launch's kernels apart: 5.8 ms at
+// N = 256, 140 at 5184, 261 at 8100, 699 at 14400); band 32 above, where the MFMA updates
+// are most of the time.  The COMPLEX*8 matrix keeps the one-stage form below 8192, where
+// its GEMV chain reads half the bytes, and band 32 above.
+constexpr int kTwoStageMinN64 = 32, kTwoStageMinN = 8192;
+
+static int plan_default_band(bool mixed, int N) { return !mixed && N <= band_panel_rows() ? 16 : 32; }
+
+static bool plan_two_stage(const wtb_bse_plan* p) {
+  if (p->wf_count > 0 || (p->mixed && p->nref > 0) || !p->bandwork) return false;   // the reflectors are needed
+  if (p->two_stage >= 0) return p->two_stage == 1;
+  return p->N >= (!p->mixed && p->band_b == 16 ? kTwoStageMinN64 : kTwoStageMinN);
+}
 
 static int plan_reduce(wtb_bse_plan* p, zc* g, int* status) {
   hipStream_t s = p->stream;
-  const bool vectors = p->wf_count > 0 || (p->mixed && p->nref > 0);
-  const bool two = p->two_stage == 1 || (p->two_stage < 0 && p->N >= kTwoStageMinN);
-  if (two && !vectors && p->bandwork) {
+  if (plan_two_stage(p)) {
     p->bw.kev = p->kernel_timing ? p->kev.data() : nullptr;
     p->bw.kev_cap = p->kernel_timing ? p->N : 0;
     // the band reduction reads and updates the lower triangle only
@@ -792,9 +811,7 @@ static int plan_enqueue_pre(wtb_bse_plan* p, bool build_only, bool after_b = fal
 // whether the plan's reduction is the one-stage form, which a batch runs in lockstep
 static bool plan_one_stage(const wtb_bse_plan* p) {
   if (p->qmode || p->sp_only) return false;
-  const bool vectors = p->wf_count > 0 || (p->mixed && p->nref > 0);
-  const bool two = p->two_stage == 1 || (p->two_stage < 0 && p->N >= kTwoStageMinN);
-  return !(two && !vectors && p->bandwork);
+  return !plan_two_stage(p);
 }
 
 // stages (d2)-(e): everything after the reduction
@@ -1065,37 +1082,56 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
   zc *da = nullptr, *dh = nullptr, *dx = nullptr;
   void *tri = nullptr, *dcw = nullptr, *btw = nullptr;
   double *dl = nullptr, *dz = nullptr;
-  int rc;
-  if ((rc = dmalloc(&da, (size_t)lda * n)) || (rc = dmalloc(&dh, (size_t)n * n)) ||
-      (rc = dmalloc((char**)&tri, tridiag_work_bytes(n, 32, 0))) ||
+  int* dst = nullptr;
+  int rc, st = 0;
+  // eigenvalues alone take the two-stage reduction, as a plan's do (plan_two_stage)
+  const bool two = !vec && n >= kTwoStageMinN64;
+  const int band = plan_default_band(false, n);
+  if ((rc = dmalloc(&da, (size_t)lda * n)) || (rc = dmalloc(&dh, (size_t)n * n)) || (rc = dmalloc(&dst, 1)) ||
+      (rc = dmalloc((char**)&tri, two ? band_work_bytes(n, band, 0) + sizeof(double) * 2 * n : tridiag_work_bytes(n, 32, 0))) ||
       (rc = dmalloc((char**)&dcw, dc_work_bytes(n, 0, vec))) || (rc = dmalloc(&dl, n)) ||
       (vec && ((rc = dmalloc(&dz, (size_t)n * n)) || (rc = dmalloc(&dx, (size_t)n * n)) ||
                (rc = dmalloc((char**)&btw, backtr_work_bytes(n, n)))))) {
   } else {
     TridiagWork tw;
+    BandWork bw;
     DCTree tree;
-    tridiag_bind(tw, tri, n, 32, 0);
-    tw.store_v = vec;
-    rc = dc_prepare(dcw, n, 0, tree, vec);
+    if (two) {
+      tw.d = static_cast<double*>(tri);
+      tw.e = tw.d + n;
+      rc = band_bind(bw, tw.e + n, n, band, 0);
+      int cus = 0;
+      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 0;
+      bw.panel_resident = cus;
+    } else {
+      tridiag_bind(tw, tri, n, 32, 0);
+      tw.store_v = vec;
+    }
+    if (!rc) rc = dc_prepare(dcw, n, 0, tree, vec);
     if (!rc) {
       hipMemcpyAsync(da, a, sizeof(zc) * lda * n, hipMemcpyHostToDevice, s);
       hipLaunchKernelGGL(k_upper_to_lower, dim3((n + 255) / 256, n), dim3(256), 0, s, n, da, lda, dh, n);
-      rc = run_tridiag(s, tw, dh, n, nullptr);
+      hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, s, dst, 1);
+      rc = two ? run_band_tridiag(s, bw, dh, n, nullptr, tw.d, tw.e, dst) : run_tridiag(s, tw, dh, n, nullptr);
     }
     if (!rc) rc = run_dc(s, dcw, tree, tw.d, tw.e, nullptr, dl, dz);
     if (!rc && vec) rc = run_backtr(s, dh, n, n, tw.tau, dz, 0, n, dx, n, btw);
     if (!rc) {
       hipMemcpyAsync(w, dl, sizeof(double) * n, hipMemcpyDeviceToHost, s);
+      hipMemcpyAsync(&st, dst, sizeof(int), hipMemcpyDeviceToHost, s);
       if (vec)
         hipMemcpy2DAsync(a, sizeof(zc) * lda, dx, sizeof(zc) * n, sizeof(zc) * n, n, hipMemcpyDeviceToHost, s);
       if (hipStreamSynchronize(s) != hipSuccess) {
         set_error("wtb_zheev: stream error");
         rc = WTB_ERR_HIP;
+      } else if ((rc = status_to_code(st))) {
+        set_error(status_text(rc));
       }
     }
   }
   hipFree(da);
   hipFree(dh);
+  hipFree(dst);
   hipFree(dx);
   hipFree(tri);
   hipFree(dcw);
@@ -2030,6 +2066,7 @@ int wtb_bse_plan_set_reduction(wtb_bse_plan* p, int two_stage, int band) {
     set_error("wtb_bse_plan_set_reduction: the two-stage reduction needs N >= 2");
     return WTB_ERR_ARG;
   }
+  if (two_stage < 0 && band == 32) band = plan_default_band(p->mixed, p->N);
   if (band != p->band_b && p->N >= 2) {
     WTB_HIP(hipSetDevice(p->ctx->device));
     WTB_HIP(hipStreamSynchronize(p->stream));

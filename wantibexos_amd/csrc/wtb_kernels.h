@@ -155,6 +155,7 @@ struct BandWork {
   double kev_flops = 0.0;       // summed over the timed launches
 };
 size_t band_work_bytes(int N, int b, int nrhs);
+int band_panel_rows();            // largest N whose COMPLEX*16 panels run in one launch (band 16)
 int band_bind(BandWork& w, void* base, int N, int b, int nrhs);
 int run_band_tridiag(hipStream_t s, BandWork& w, zc* H, int ld, zc* g, double* d, double* e, int* status);
 int run_band_tridiag_f32(hipStream_t s, BandWork& w, zf* H, int ld, zc* g, double* d, double* e, int* status);
