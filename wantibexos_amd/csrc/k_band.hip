@@ -1369,14 +1369,15 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   }
 }
 
-// W = X - 1/2 V (T^H (V^H X)) with X the sum of the K slices of A22 Y, in one launch:
-// workgroup w takes rows 256 w .., its part of M = V^H X on FP64 MFMA (operands straight
-// from memory in the MFMA's layout), one exchange of the B x B parts as above (slots
-// [workgroup][B B]), then Z = T^H M and its rows of W.
+// W = X - 1/2 V (T^H (V^H X)) with X = A22 Y, in one launch: workgroup w takes rows 256 w ..,
+// its part of M = V^H X on FP64 MFMA (operands straight from memory in the MFMA's layout),
+// one exchange of the B x B parts as above (slots [workgroup][B B]), then Z = T^H M and its
+// rows of W.  Latency-bound (17 us at N = 5184); summing the K slices of X here too, on the
+// few workgroups of this launch, took 30 us against 17 + 5 with k_hmm_sum.
 struct QrWArgs {
-  int m, N, ns;          // rows; slices of part (0: X holds the product)
-  const zc *part, *V, *Tm;
-  zc* X;                 // in (ns = 0), out: W
+  int m, N;
+  const zc *V, *Tm;
+  zc* X;                 // in: X, out: W
   zc *ex, *ex_next;
   int nwg;
   int* err;
@@ -1395,18 +1396,12 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   const size_t N = a.N;
-  const int row0 = blockIdx.x * 256, i = row0 + t;
+  const int row0 = blockIdx.x * 256;
   const __amdgpu_buffer_rsrc_t ex = dev_buffer(a.ex, (size_t)a.nwg * B * B * sizeof(zc));
   if (t == 0) bad = 0;
   const zc empty = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
 #pragma unroll
   for (int u = 0; u < NE; ++u) a.ex_next[(size_t)blockIdx.x * B * B + t + 256 * u] = empty;
-  if (a.ns > 0 && i < a.m)
-    for (int c = 0; c < B; ++c) {
-      const zc* pp = a.part + (size_t)c * a.m + i;
-      a.X[i + N * c] = strided_sum(pp, (size_t)a.m * B, 0, a.ns, 1, mkz(0, 0));
-    }
-  __syncthreads();
   // this wave's 64 rows of M = V^H X
   d4 mr[TI][TI], mi[TI][TI];
 #pragma unroll
@@ -1414,15 +1409,16 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
 #pragma unroll
     for (int y = 0; y < TI; ++y) mr[x][y] = mi[x][y] = d4{0, 0, 0, 0};
   const int w0 = row0 + 64 * wave;
-#pragma unroll 4
+#pragma unroll
   for (int k0 = 0; k0 < 64; k0 += 4) {
     const int rr = w0 + k0 + lk;
     const bool on = rr < a.m;
     zc av[TI], xv[TI];
 #pragma unroll
     for (int x = 0; x < TI; ++x) {
-      av[x] = on ? a.V[rr + N * (16 * x + lr)] : mkz(0, 0);
-      xv[x] = on ? a.X[rr + N * (16 * x + lr)] : mkz(0, 0);
+      av[x] = a.V[min(rr, a.m - 1) + N * (16 * x + lr)];
+      xv[x] = a.X[min(rr, a.m - 1) + N * (16 * x + lr)];
+      if (!on) av[x] = mkz(0, 0);
     }
     // conj(v) x = (vr xr + vi xi) + i (vr xi - vi xr)
 #pragma unroll
@@ -2004,22 +2000,19 @@ static void her2k_band(hipStream_t s, BandWork& w, T* H, int ld, int m, int r0, 
 }
 
 // X = A22 Y (m x B) with enough workgroups to fill the chip: K slices until the grid
-// holds ~1024 workgroups (at most HB_SMAX slices), partials summed in slice order, or (sum
-// false) left to the caller: returns their number, 0 when X holds the product
+// holds ~1024 workgroups (at most HB_SMAX slices), partials summed in slice order
 template <class T, int B>
-static int hmm_band(hipStream_t s, BandWork& w, int m, const T* A, int ld, const zc* Y, zc* X, bool sum = true) {
+static void hmm_band(hipStream_t s, BandWork& w, int m, const T* A, int ld, const zc* Y, zc* X) {
   const int rb = (m + HB_R - 1) / HB_R;
   int ns = std::max(1, std::min(HB_SMAX, (1024 + rb - 1) / rb));
   const int kc = ((m + ns - 1) / ns + 31) / 32 * 32;   // a multiple of either K step
   ns = (m + kc - 1) / kc;
   hipLaunchKernelGGL((k_hmm_b<T, B>), dim3(rb, ns), dim3(256), 0, s, m, A, ld, Y, w.N, kc, ns > 1 ? w.hb : nullptr,
                      X, w.N);
-  if (ns > 1 && !sum) return ns;
   if (ns > 1) {
     const size_t tot = (size_t)m * B;
     hipLaunchKernelGGL(k_hmm_sum<B>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, m, ns, w.hb, X, w.N);
   }
-  return 0;
 }
 
 // out0 = A^H Y0 (B x B) and out1 = A^H Y1 (B x n1) over m rows, ld B
@@ -2039,7 +2032,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   const int exw = min(w.nwg_max, QP_WG);               // workgroups that the slots hold
   const size_t exn = qr_ex_elems<B>(exw);
   // COMPLEX*16 panels of at most QP_WG workgroups: one launch for the panel and one for W
-  // (4 launches a panel).  The limit does not depend on how many streams run, so that the
+  // (5 launches a panel).  The limit does not depend on how many streams run, so that the
   // results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
   // its stored matrix amplifies.
   const bool qr = std::is_same<T, zc>::value && B == 16 && w.panel_wg >= (N - b + PR - 1) / PR;
@@ -2072,8 +2065,8 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
         const size_t wo = qr_slots<B>(exw);
         QrPanelArgs q{H, ld, N, c0, r0, m, k, w.V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20};
         hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, q);
-        const int ns = hmm_band<T, B>(s, w, m, H + r0 + (size_t)ld * r0, ld, w.Y, w.X, false);
-        QrWArgs x{m, N, ns, w.hb, w.V, w.T, w.X, ex + wo, exo + wo, a.nwg, w.err + 8, 1 << 20};
+        hmm_band<T, B>(s, w, m, H + r0 + (size_t)ld * r0, ld, w.Y, w.X);
+        QrWArgs x{m, N, w.V, w.T, w.X, ex + wo, exo + wo, a.nwg, w.err + 8, 1 << 20};
         hipLaunchKernelGGL((k_qr_w<B>), g, blk, 0, s, x);
         her2k_band<T, B>(s, w, H, ld, m, r0, k);
         continue;
