@@ -375,10 +375,11 @@ def bench_bands(args, cfg, model):
     avg_s = k_ms * 1e-3 / max(k_n, 1)
     if k_flops > 0:
         per_launch = k_flops / max(k_n, 1)
+        kname = "k_her2k_full" if args.precision == "mixed" or (args.reduction == "two" and args.band == 32) else "k_update_mul"
         ach = per_launch / avg_s / 1e12
         peak = FP32_PEAK if args.precision == "mixed" else FP64_PEAK
         roofline = dict(bound="mfma", achieved=round(ach, 2), peak=peak, unit="TFLOP/s", frac=round(ach / peak, 4),
-                        traffic=None, kernel="k_her2k_full", launches=k_n, avg_launch_us=round(avg_s * 1e6, 3),
+                        traffic=None, kernel=kname, launches=k_n, avg_launch_us=round(avg_s * 1e6, 3),
                         flops_per_launch=round(per_launch))
     else:
         per_launch = hemv_b / max(k_n, 1)
@@ -633,11 +634,12 @@ def main():
     if k_flops > 0:
         # two-stage reduction: the dense -> band stage's trailing update, MFMA-bound
         per_launch = k_flops / max(k_n, 1)
+        kname = "k_her2k_full" if args.precision == "mixed" or (args.reduction == "two" and args.band == 32) else "k_update_mul"
         ach = per_launch / avg_s / 1e12
         peak = FP32_PEAK if args.precision == "mixed" else FP64_PEAK
-        log(f"k_her2k_full: {k_n} launches, avg {avg_s * 1e6:.2f} us, {per_launch / 1e9:.3f} GFLOP/launch")
+        log(f"{kname}: {k_n} launches, avg {avg_s * 1e6:.2f} us, {per_launch / 1e9:.3f} GFLOP/launch")
         roofline = dict(bound="mfma", achieved=round(ach, 2), peak=peak, unit="TFLOP/s", frac=round(ach / peak, 4),
-                        traffic=None, kernel="k_her2k_full", launches=k_n, avg_launch_us=round(avg_s * 1e6, 3),
+                        traffic=None, kernel=kname, launches=k_n, avg_launch_us=round(avg_s * 1e6, 3),
                         flops_per_launch=round(per_launch))
     else:
         per_launch = hemv_b / max(k_n, 1)

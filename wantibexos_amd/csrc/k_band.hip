@@ -20,6 +20,11 @@
 //   k_gram, k_gram_sum         M = V^H X
 //   k_pW                       W = X - 1/2 V (T^H M)
 //   k_her2k_full               A22 -= V W^H + W V^H (MFMA, the tiles on and below the diagonal)
+// COMPLEX*16 with b = 16 (up to band_panel_rows() rows) has its own form of the same steps:
+//   k_strip                    the panel's columns take the update of the panel before
+//   k_qr_panel                 reflectors, T, Y = V T and the tracked vectors, in one launch
+//   k_update_mul, k_um_sum     A22 takes the update of the panel before; X = A22 Y in that pass
+//   k_qr_w                     W = X - 1/2 V (T^H (V^H X))
 // The tracked vectors are carried conjugated (gc = conj(g)): Q^H gc = conj(Q^T g).
 //
 // Stage 2 (bulge chasing, FP64, band storage BD[c][d] = A(c + d, c), d <= 2b): sweep s
@@ -1373,7 +1378,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
 // its part of M = V^H X on FP64 MFMA (operands straight from memory in the MFMA's layout),
 // one exchange of the B x B parts as above (slots [workgroup][B B]), then Z = T^H M and its
 // rows of W.  Latency-bound (17 us at N = 5184); summing the K slices of X here too, on the
-// few workgroups of this launch, took 30 us against 17 + 5 with k_hmm_sum.
+// few workgroups of this launch, took 30 us against 17 + 5 with a launch of its own.
 struct QrWArgs {
   int m, N;
   const zc *V, *Tm;
@@ -1518,6 +1523,254 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
           a.X[at] = mkz(v.re - 0.5 * cr[x][r], v.im - 0.5 * ci[x][r]);
         }
   }
+}
+
+// The 16 columns of the next panel, ahead of k_update_mul (5.4 us, latency-bound): A(:, 0:16) -= (V W^H + W V^H)(:, 0:16)
+// on and below the diagonal, rows 0 .. m - 1 of the trailing matrix at A.  One 16 x 16 MFMA
+// tile a wave, rows over the MFMA's columns as in k_her2k_full.
+template <int B>
+__global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m, int N, const zc* __restrict__ V,
+                                               const zc* __restrict__ W) {
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int r = blockIdx.x * 64 + (threadIdx.x >> 6) * 16 + lr, rc = min(r, m - 1), c = min(lr, m - 1);
+  zc av[B / 2], bv[B / 2], h[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) h[q] = A[(size_t)rc + (size_t)ld * min(lk + 4 * q, m - 1)];
+#pragma unroll
+  for (int s = 0; s < B / 2; ++s) {            // [V | W](c, k) and [W | V](r, k), k = 4 s + lk
+    const int k = 4 * s + lk;
+    av[s] = (k < B) ? V[(size_t)k * N + c] : W[(size_t)(k - B) * N + c];
+    bv[s] = (k < B) ? W[(size_t)k * N + rc] : V[(size_t)(k - B) * N + rc];
+  }
+  d4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < B / 2; ++s) {
+    cr = mfma16x16x4(av[s].re, bv[s].re, cr);
+    ci = mfma16x16x4(av[s].im, bv[s].re, ci);
+    cr = mfma16x16x4(av[s].im, bv[s].im, cr);
+    ci = mfma16x16x4(-av[s].re, bv[s].im, ci);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int cc = lk + 4 * q;
+    if (r < m && cc <= r) A[(size_t)r + (size_t)ld * cc] = mkz(h[q].re - cr[q], h[q].im + ci[q]);
+  }
+}
+
+// One pass over the trailing matrix A (m x m, lower triangle): the update of the panel before,
+// A -= V W^H + W V^H (UPD), and the product of the updated values with this panel's Y, X = A Y.
+// A workgroup takes 128 rows (block I) and 32 n columns of block J <= I, a wave 32 rows of
+// them, and goes through the columns in steps of 32.  Every element is read and written once
+// and serves both A(I, J) Y(J) -> X(I), accumulated over the steps, and A(I, J)^H Y(I) -> X(J),
+// summed over the waves: the update, accumulated onto the elements, leaves a 16 x 16 tile in
+// the MFMA's result layout, which is its layout for an operand whose sum runs over the tile's
+// columns, so the first product needs no data movement, and the second one transposes the
+// tile through LDS.  The parts go to part[slot][col][row], the rows of block K in the slots
+// 0 .. um_parts(K) - 1 (first the 4 (K + 1) / n column groups left of and in block K, then the
+// row blocks from K on); k_um_sum adds them in order.
+//
+// 256 m^2 flops over 16 m^2 bytes and 2 m^2 of parts: at m = 14400 0.73 ms of the matrix cores
+// and 0.73 ms of memory, and the kernel takes 1.15 ms (46 TFLOP/s, 3.7 TB/s with the operands
+// that miss the L2; the matrix cores are busy 63 % of the time).  Two kernels, a product over
+// 16 m^2 bytes and an update over 16 m^2, took 483 ms of a reduction at N = 14400 where this
+// one and k_um_sum take 385, and 27 ms of one at N = 5184 (20 here).  64 x 64 tiles, three
+// waves per SIMD with spills, and an order of the tiles by XCD were no faster.
+#define UM_R 128
+__host__ __device__ inline int um_parts(int K, int n, int nt) { return 4 / n * (K + 1) + nt - K; }
+template <int B, bool UPD>
+__global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int ld, int m, int N,
+                                                       const zc* __restrict__ V, const zc* __restrict__ W,
+                                                       const zc* __restrict__ Y, zc* __restrict__ part, int nt, int n) {
+  static_assert(B == 16, "one MFMA tile of Y columns");
+  __shared__ zc tr[4][16 * 17];                // a wave's tile on its way through
+  __shared__ zc red[4][2][4][64];              // the waves' parts of A^H Y
+  const int ng = 4 / n, t = blockIdx.x / ng;
+  int ti = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
+  while (ti * (ti + 1) / 2 > t) --ti;
+  const int tj = t - ti * (ti + 1) / 2, g = tj * ng + (int)blockIdx.x % ng;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int r0 = ti * UM_R + wave * 32;
+  d4 ar[2], ai[2];                             // (A Y)^T of this wave's rows [y]
+#pragma unroll
+  for (int y = 0; y < 2; ++y) ar[y] = ai[y] = d4{0, 0, 0, 0};
+#pragma unroll 1
+  for (int u = 0; u < n; ++u) {
+    const int c0 = (g * n + u) * 32;
+    if (c0 >= m) break;
+    int l = lane;
+    __asm__ volatile("" : "+v"(l));            // no addresses kept from step to step
+    const int lr = l & 15, lk = l >> 4;
+    const unsigned lao = (unsigned)(lk * ld + lr);
+    const bool on = r0 >= c0 && r0 < m;        // not above the diagonal or outside
+    const bool diag = r0 == c0, edge = diag || r0 + 32 > m || c0 + 32 > m;
+    zc* const Aw = A + (size_t)ld * c0 + r0;
+    if (u > 0) lds_barrier();                  // the sums of the step before are taken
+    if (on) {
+      // h[x][y][2 e], [2 e + 1]: re and im of column c0 + 8 x + 4 e + lk, row r0 + 16 y + lr,
+      // which are rows lk + 8 e and lk + 8 e + 4 of the MFMA's result: 16 bytes go to and come
+      // from four registers next to each other
+      d4 h[4][2];
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const zc v = A[(size_t)min(r0 + 16 * y + lr, m - 1) + (size_t)ld * min(c0 + 8 * x + 4 * e + lk, m - 1)];
+            h[x][y][2 * e] = v.re;
+            h[x][y][2 * e + 1] = v.im;
+          }
+      if constexpr (UPD) {
+        unsigned cc[4], rr[2];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) cc[x] = (unsigned)(lk * N + min(c0 + 8 * x + (lr & 3) + 4 * (lr >> 3), m - 1));
+#pragma unroll
+        for (int y = 0; y < 2; ++y) rr[y] = (unsigned)(lk * N + min(r0 + 16 * y + lr, m - 1));
+        const bool im = (lr & 4) != 0;
+#pragma unroll
+        for (int s = 0; s < B / 2; ++s) {      // h -= conj(a) b, a: [V | W](c, k), b: [W | V](r, k)
+          const zc* pa = (s < B / 4) ? V + (size_t)(4 * s) * N : W + (size_t)(4 * s - B) * N;
+          const zc* pb = (s < B / 4) ? W + (size_t)(4 * s) * N : V + (size_t)(4 * s - B) * N;
+          double a1[4], a2[4];
+          zc b[2];
+#pragma unroll
+          for (int y = 0; y < 2; ++y) b[y] = pb[rr[y]];
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const zc a = pa[cc[x]];
+            a1[x] = im ? a.im : -a.re;
+            a2[x] = im ? -a.re : -a.im;
+          }
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) h[x][y] = mfma16x16x4(a1[x], b[y].re, h[x][y]);
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) h[x][y] = mfma16x16x4(a2[x], b[y].im, h[x][y]);
+        }
+      }
+      if (edge) {                              // nothing above the diagonal or outside
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const int c = c0 + 8 * x + 4 * e + lk, r = r0 + 16 * y + lr;
+              if (r >= m || c > r) h[x][y][2 * e] = h[x][y][2 * e + 1] = 0.0;
+            }
+      }
+      // A Y: the sum runs over the columns
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        zc yv[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) yv[e] = Y[(size_t)min(c0 + 8 * x + 4 * e + lk, m - 1) + (size_t)N * lr];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            ar[y] = mfma16x16x4(yv[e].re, h[x][y][2 * e], ar[y]);
+            ai[y] = mfma16x16x4(yv[e].re, h[x][y][2 * e + 1], ai[y]);
+          }
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            ar[y] = mfma16x16x4(-yv[e].im, h[x][y][2 * e + 1], ar[y]);
+            ai[y] = mfma16x16x4(yv[e].im, h[x][y][2 * e], ai[y]);
+          }
+        }
+      }
+      // A^H Y: the sum runs over the rows; the diagonal itself is in A Y already
+      __builtin_amdgcn_sched_barrier(0);
+      d4 br[2], bi[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) br[x] = bi[x] = d4{0, 0, 0, 0};
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        zc yv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) yv[q] = Y[(size_t)min(r0 + 16 * y + lk + 4 * q, m - 1) + (size_t)N * lr];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            tr[wave][(lk + 4 * q) * 17 + lr] = mkz(h[2 * x + q / 2][y][2 * (q & 1)], h[2 * x + q / 2][y][2 * (q & 1) + 1]);
+          if (diag && x == y && lane < 16) tr[wave][lane * 18] = mkz(0, 0);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const zc b = tr[wave][lr * 17 + lk + 4 * q];
+            br[x] = mfma16x16x4(yv[q].re, b.re, br[x]);
+            bi[x] = mfma16x16x4(yv[q].im, b.re, bi[x]);
+            br[x] = mfma16x16x4(yv[q].im, b.im, br[x]);
+            bi[x] = mfma16x16x4(-yv[q].re, b.im, bi[x]);
+          }
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[wave][x][q][lane] = mkz(br[x][q], bi[x][q]);
+      // the stores last: a later load's wait would wait for them too
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (UPD) {
+        __asm__ volatile("" : "+v"(l));
+        const int lr = l & 15, lk = l >> 4;
+        const unsigned lao = (unsigned)(lk * ld + lr);
+        auto put = [&](auto masked) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const int c = c0 + 8 * x + 4 * e + lk;
+              zc* pc = Aw + (size_t)ld * (8 * x + 4 * e);
+#pragma unroll
+              for (int y = 0; y < 2; ++y)
+                if (!decltype(masked)::value || (r0 + 16 * y + lr < m && c <= r0 + 16 * y + lr))
+                  (pc + 16 * y)[lao] = mkz(h[x][y][2 * e], h[x][y][2 * e + 1]);
+            }
+        };
+        if (edge) put(std::true_type{});
+        else put(std::false_type{});
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[wave][x][q][lane] = mkz(0, 0);
+    }
+    lds_barrier();
+    const int row = c0 + 16 * (wave >> 1) + lr;
+    zc* const pp = part + (size_t)(ng * (c0 / UM_R + 1) + ti - c0 / UM_R) * B * m + row;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int q = 2 * (wave & 1) + e;
+      zc v = red[0][wave >> 1][q][lane];
+#pragma unroll
+      for (int o = 1; o < 4; ++o) v = v + red[o][wave >> 1][q][lane];
+      if (row < m) pp[(size_t)(lk + 4 * q) * m] = v;
+    }
+  }
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    const int row = r0 + 16 * y + (lane & 15);
+    if (row < m)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) part[((size_t)g * B + (lane >> 4) + 4 * q) * m + row] = mkz(ar[y][q], ai[y][q]);
+  }
+}
+
+// X(row, col) = the sum of the parts of k_update_mul, in slot order
+template <int B>
+__global__ __launch_bounds__(256) void k_um_sum(int m, int n, int nt, const zc* __restrict__ part, zc* __restrict__ X,
+                                                int ldx) {
+  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= (size_t)m * B) return;
+  const int row = (int)(e % m), col = (int)(e / m);
+  X[(size_t)row + (size_t)ldx * col] = strided_sum(part + e, (size_t)m * B, 0, um_parts(row / UM_R, n, nt), 1, mkz(0, 0));
 }
 
 __global__ void k_fill_empty(zc* p, size_t n) {
@@ -1914,6 +2167,19 @@ static size_t qr_ex_elems(int nwg_max) {
 
 int band_panel_rows() { return QP_WG * PR + 16; }
 
+// steps of k_update_mul: fewer parts with more steps, more workgroups with fewer (at these
+// sizes about 1200 workgroups either way, 512 run at once; lines at half and one and a half
+// times these sizes measured within 1 %)
+constexpr int UM_4 = 6144, UM_2 = 3072;
+static int um_steps(int m) { return m > UM_4 ? 4 : m > UM_2 ? 2 : 1; }
+
+// slots of the partial products for at most N rows: k_hmm_b's K slices, k_update_mul's parts
+static size_t hb_slots(int N, int b) {
+  if (b != 16 || N > band_panel_rows()) return HB_SMAX;
+  auto slots = [](int m) { const int nt = (m + UM_R - 1) / UM_R; return um_parts(nt - 1, um_steps(m), nt); };
+  return std::max({(int)HB_SMAX, slots(N), slots(std::min(N, UM_4)), slots(std::min(N, UM_2))});
+}
+
 size_t band_work_bytes(int N, int b, int nrhs) {
   const size_t nwg = (N + PR - 1) / PR + 1;
   const size_t LB = 2 * (size_t)b + 1;
@@ -1933,7 +2199,8 @@ size_t band_work_bytes(int N, int b, int nrhs) {
   add(sizeof(zc) * BMAX * BMAX);              // M
   add(sizeof(zc) * nwg * BMAX * BMAX);        // K slices of the small products
   add(sizeof(zc) * GRAM_PMAX * BMAX * (BMAX + 16));   // partials of the tall-skinny products
-  add(sizeof(zc) * HB_SMAX * (size_t)N * b);           // K-slice partials of X = A22 Y
+  add(sizeof(zc) * hb_slots(N, b) * (size_t)N * b);    // partials of X = A22 Y
+  add(sizeof(zc) * 2 * (size_t)N * b);                 // V2, X2
   add(sizeof(zc) * (size_t)N * LB);           // band
   add(sizeof(zc) * (size_t)N * (nrhs > 0 ? nrhs : 1));   // gc
   add(sizeof(int) * ((size_t)N + 1));         // prog
@@ -1975,7 +2242,9 @@ int band_bind(BandWork& w, void* base, int N, int b, int nrhs) {
   w.gw = (zc*)take(sizeof(zc) * nwg * BMAX * BMAX);
   w.gw_elems = nwg * BMAX * BMAX;
   w.gp = (zc*)take(sizeof(zc) * GRAM_PMAX * BMAX * (BMAX + 16));
-  w.hb = (zc*)take(sizeof(zc) * HB_SMAX * (size_t)N * b);
+  w.hb = (zc*)take(sizeof(zc) * hb_slots(N, b) * (size_t)N * b);
+  w.V2 = (zc*)take(sizeof(zc) * 2 * (size_t)N * b);
+  w.X2 = w.V2 + (size_t)N * b;
   w.BD = (zc*)take(sizeof(zc) * (size_t)N * w.LB);
   w.gc = (zc*)take(sizeof(zc) * (size_t)N * (nrhs > 0 ? nrhs : 1));
   w.prog = (int*)take(sizeof(int) * ((size_t)N + 1));
@@ -2032,8 +2301,9 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   const int exw = min(w.nwg_max, QP_WG);               // workgroups that the slots hold
   const size_t exn = qr_ex_elems<B>(exw);
   // COMPLEX*16 panels of at most QP_WG workgroups: one launch for the panel and one for W
-  // (5 launches a panel).  The limit does not depend on how many streams run, so that the
-  // results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
+  // (5 launches a panel, one of them a pass over the trailing matrix that updates it for the
+  // panel before and multiplies it with this one's Y).  The limit does not depend on how many
+  // streams run, so that the results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
   // its stored matrix amplifies.
   const bool qr = std::is_same<T, zc>::value && B == 16 && w.panel_wg >= (N - b + PR - 1) / PR;
   if (qr)
@@ -2063,12 +2333,33 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
       if (qr) {
         zc *ex = w.ex + (size_t)(p & 1) * exn, *exo = w.ex + (size_t)((p + 1) & 1) * exn;
         const size_t wo = qr_slots<B>(exw);
-        QrPanelArgs q{H, ld, N, c0, r0, m, k, w.V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20};
+        zc *V = p & 1 ? w.V2 : w.V, *X = p & 1 ? w.X2 : w.X;          // this panel's; the one's before:
+        const zc *Vo = p & 1 ? w.V : w.V2, *Xo = p & 1 ? w.X : w.X2;
+        zc* A22 = H + r0 + (size_t)ld * r0;
+        if (p > 0)
+          hipLaunchKernelGGL((k_strip<B>), dim3((m + B + 63) / 64), blk, 0, s, H + c0 + (size_t)ld * c0, ld, m + B, N, Vo, Xo);
+        QrPanelArgs q{H, ld, N, c0, r0, m, k, V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20};
         hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, q);
-        hmm_band<T, B>(s, w, m, H + r0 + (size_t)ld * r0, ld, w.Y, w.X);
-        QrWArgs x{m, N, w.V, w.T, w.X, ex + wo, exo + wo, a.nwg, w.err + 8, 1 << 20};
+        const int n = um_steps(m), nt = (m + UM_R - 1) / UM_R;
+        const dim3 gt(4 / n * (nt * (nt + 1) / 2));
+        auto um = p > 0 ? k_update_mul<B, true> : k_update_mul<B, false>;
+        const bool tev = w.kev && w.kev_used < w.kev_cap;
+        if (tev) hipEventRecord(w.kev[2 * w.kev_used], s);
+        hipLaunchKernelGGL(um, gt, blk, 0, s, A22, ld, m, N, Vo + B, Xo + B, w.Y, w.hb, nt, n);
+        if (tev) {
+          hipEventRecord(w.kev[2 * w.kev_used++ + 1], s);
+          // the update's two products of B reflectors on the lower triangle, the product with Y
+          w.kev_flops += (p > 0 ? 8.0 * 0.5 * (double)m * (double)(m + 1) * (2.0 * B) : 0.0) + 8.0 * (double)m * m * k;
+        }
+        const size_t tot = (size_t)m * B;
+        hipLaunchKernelGGL(k_um_sum<B>, dim3((unsigned)((tot + 255) / 256)), blk, 0, s, m, n, nt, w.hb, X, N);
+        QrWArgs x{m, N, V, w.T, X, ex + wo, exo + wo, a.nwg, w.err + 8, 1 << 20};
         hipLaunchKernelGGL((k_qr_w<B>), g, blk, 0, s, x);
-        her2k_band<T, B>(s, w, H, ld, m, r0, k);
+        // the last panel's update, which no further product waits for
+        if (m - B <= 0 || min(b, m - B - 1) <= 0) {
+          const int nu = (m + 63) / 64;
+          hipLaunchKernelGGL((k_her2k_full<T, B>), dim3(nu * (nu + 1) / 2), blk, 0, s, H, ld, m, r0, N, V, X);
+        }
         continue;
       }
     if (w.panel_resident > 0 && a.nwg <= w.panel_resident) {

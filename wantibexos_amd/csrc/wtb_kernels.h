@@ -147,7 +147,9 @@ struct BandWork {
   int panel_resident = 0;       // one-launch panels up to this many workgroups (0: per column)
   int panel_wg = 0;             // COMPLEX*16: panel and W in one launch each up to this many workgroups
   zc* ex = nullptr;             // their exchange slots, two panel parities
-  // optional per-launch timing of the trailing-update kernel (k_her2k_full): launch c is
+  zc *V2 = nullptr, *X2 = nullptr;   // every other panel's V and W
+  // optional per-launch timing of the trailing-update kernel (k_update_mul with COMPLEX*16 and
+  // band 16, else k_her2k_full): launch c is
   // bracketed by kev[2c], kev[2c+1] (c < kev_cap); kev_flops[c] its flop count
   hipEvent_t* kev = nullptr;
   int kev_cap = 0;
