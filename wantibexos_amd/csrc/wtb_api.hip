@@ -1119,8 +1119,11 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
     if (!rc) {
       hipMemcpyAsync(w, dl, sizeof(double) * n, hipMemcpyDeviceToHost, s);
       hipMemcpyAsync(&st, dst, sizeof(int), hipMemcpyDeviceToHost, s);
+      // one block where the array has no gaps: the strided copy to pageable memory goes column
+      // by column (10 ms more at n = 1290)
       if (vec)
-        hipMemcpy2DAsync(a, sizeof(zc) * lda, dx, sizeof(zc) * n, sizeof(zc) * n, n, hipMemcpyDeviceToHost, s);
+        lda == n ? hipMemcpyAsync(a, dx, sizeof(zc) * n * n, hipMemcpyDeviceToHost, s)
+                 : hipMemcpy2DAsync(a, sizeof(zc) * lda, dx, sizeof(zc) * n, sizeof(zc) * n, n, hipMemcpyDeviceToHost, s);
       if (hipStreamSynchronize(s) != hipSuccess) {
         set_error("wtb_zheev: stream error");
         rc = WTB_ERR_HIP;
