@@ -94,17 +94,31 @@ struct SmallEig {
   void* btw = nullptr;
   double* lam = nullptr;
   double* Z = nullptr;   // mmax x mmax
+  int* status = nullptr; // set when a reduction stalls
+  int cus = 0;
 };
+
+// room for either reduction of up to m rows
+size_t small_tri_bytes(int m) {
+  const size_t one = tridiag_work_bytes(m, 32, 0);
+  const int mt = std::min(m, band_vec_rows());
+  return std::max(one, sizeof(zc) * ((size_t)mt + band_tau_elems(mt)) + band_work_bytes(mt, 16, 0));
+}
 
 int small_alloc(SmallEig& e, int mmax, int kmax) {
   e.mmax = mmax;
   e.kmax = kmax;
   WTB_HIP(hipMalloc(&e.A, sizeof(zc) * (size_t)mmax * mmax));
-  WTB_HIP(hipMalloc(&e.tri, tridiag_work_bytes(mmax, 32, 0)));
+  WTB_HIP(hipMalloc(&e.tri, small_tri_bytes(mmax)));
   WTB_HIP(hipMalloc(&e.dcw, dc_work_bytes(mmax, 0, 1)));
   WTB_HIP(hipMalloc(&e.btw, backtr_work_bytes(mmax, kmax)));
   WTB_HIP(hipMalloc(&e.lam, sizeof(double) * mmax));
   WTB_HIP(hipMalloc(&e.Z, sizeof(double) * (size_t)mmax * mmax));
+  WTB_HIP(hipMalloc(&e.status, sizeof(int)));
+  int dev = 0, none = 0;
+  WTB_HIP(hipMemcpy(e.status, &none, sizeof(int), hipMemcpyHostToDevice));
+  WTB_HIP(hipGetDevice(&dev));
+  WTB_HIP(hipDeviceGetAttribute(&e.cus, hipDeviceAttributeMultiprocessorCount, dev));
   return WTB_OK;
 }
 
@@ -115,6 +129,13 @@ void small_free(SmallEig& e) {
   hipFree(e.btw);
   hipFree(e.lam);
   hipFree(e.Z);
+  hipFree(e.status);
+}
+
+int small_status(int st) {
+  if (!st) return WTB_OK;
+  set_error("davidson: a small eigensolve stalled");
+  return WTB_ERR_EIG;
 }
 
 // eigenpairs of the m x m Hermitian G (lower triangle used): all eigenvalues into
@@ -122,12 +143,23 @@ void small_free(SmallEig& e) {
 int small_heev(hipStream_t s, SmallEig& e, int m, const zc* G, int ldg, double* theta, zc* S, int lds, int k) {
   WTB_HIP(hipMemcpy2DAsync(e.A, sizeof(zc) * m, G, sizeof(zc) * ldg, sizeof(zc) * m, m,
                            hipMemcpyDeviceToDevice, s));
-  TridiagWork tw;
-  tridiag_bind(tw, e.tri, m, 32, 0);
-  tw.store_v = 1;
   DCTree tree;
   int rc = dc_prepare(e.dcw, m, 0, tree, 1);
   if (rc) return rc;
+  if (band_vec_two_stage(m, k)) {
+    double *d = static_cast<double*>(e.tri), *off = d + m;
+    BandWork bw;
+    zc* tau = reinterpret_cast<zc*>(off + m);
+    if ((rc = band_bind(bw, tau + band_tau_elems(m), m, 16, 0))) return rc;
+    bw.tau1 = tau;
+    bw.tau2 = tau + m;
+    if ((rc = run_band_tridiag(s, bw, e.A, m, nullptr, d, off, e.status))) return rc;
+    if ((rc = run_dc(s, e.dcw, tree, d, off, nullptr, theta, e.Z, k))) return rc;
+    return run_band_backtr(s, bw, e.A, m, e.Z, 0, k, S, lds, e.cus, e.btw);
+  }
+  TridiagWork tw;
+  tridiag_bind(tw, e.tri, m, 32, 0);
+  tw.store_v = 1;
   if ((rc = run_tridiag(s, tw, e.A, m, nullptr))) return rc;
   if ((rc = run_dc(s, e.dcw, tree, tw.d, tw.e, nullptr, theta, e.Z, k))) return rc;
   return run_backtr(s, e.A, m, m, tw.tau, e.Z, 0, k, S, lds, e.btw);
@@ -262,6 +294,7 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
   const zc one = mkz(1, 0), zero = mkz(0, 0), mone = mkz(-1, 0);
   // start: unit vectors at the nk smallest diagonal entries
   double Dmin = 0.0, fp32_floor = 0.0;
+  int h_st = 0;          // a small reduction's status
   {
     std::vector<double> hD(N);
     DAV_TRY(hipStreamSynchronize(s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);   // D comes from stream s
@@ -280,6 +313,9 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
       DAV_TRY(hipMemcpy(crow, order.data(), sizeof(int) * M, hipMemcpyHostToDevice) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
       hipLaunchKernelGGL(k_gather_block, dim3((M + 255) / 256, M), dim3(256), 0, s, M, crow, H, ldh, CS);
       DAV_TRY(small_heev(s, sc, M, CS, M, lamS, QS, M, M));
+      DAV_TRY(hipMemcpyAsync(&h_st, sc.status, sizeof(int), hipMemcpyDeviceToHost, s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
+      DAV_TRY(hipStreamSynchronize(s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
+      DAV_TRY(small_status(h_st));
     }
     order.resize(nk);
     DAV_TRY(hipMemcpy(idx, order.data(), sizeof(int) * nk, hipMemcpyHostToDevice) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
@@ -310,7 +346,9 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
     DAV_TRY(zgemm(s, 'N', 'N', N, nk, m, one, HV, N, S, msub, zero, HU, N));
     DAV_TRY(launch_residual(s, N, nk, U, HU, N, theta, R, rn));
     DAV_TRY(hipMemcpyAsync(h_rn.data(), rn, sizeof(double) * nk, hipMemcpyDeviceToHost, s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
+    DAV_TRY(hipMemcpyAsync(&h_st, se.status, sizeof(int), hipMemcpyDeviceToHost, s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
     DAV_TRY(hipStreamSynchronize(s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
+    DAV_TRY(small_status(h_st));
     double mx = 0.0;
     for (int c = 0; c < nev; ++c) mx = std::max(mx, h_rn[c]);
     info.max_resid = mx;

@@ -2,7 +2,7 @@
 // X = Q Z, with Q = H(0) H(1) ... H(N-2) the product of the reduction's
 // reflectors H(j) = I - tau_j v_j v_j^H (v_j(j+1) = 1, v_j(r) for r > j+1 kept in
 // the lower triangle of the reduced matrix, column j; the layout of ZHETRD with
-// UPLO = 'L').  Panels of nb reflectors are applied last to first in compact WY
+// UPLO = 'L'; off = 1 below, or the band width for the first stage of a two-stage reduction).  Panels of nb reflectors are applied last to first in compact WY
 // form, I - V T V^H, with T upper triangular as ZLARFT ('F', 'C') builds it:
 //   T(i,i) = tau_i,  T(0:i-1, i) = -tau_i T(0:i-1, 0:i-1) V(:, 0:i-1)^H v_i.
 // Per panel: Y = V^H X (row chunks on FP64 MFMA, partial sums), Y <- T Y, and
@@ -21,10 +21,10 @@ constexpr int kBtPairs = (BT_NB * (BT_NB - 1) / 2 + 255) / 256;   // Gram pairs 
 constexpr int kBtSteps = 4;   // V^H X: MFMA steps (4 rows each) per group of loads
 
 template <class T>
-__device__ inline zc vref(const T* H, int ld, int r, int j) {
-  // v_j(r): 0 above row j+1, 1 at row j+1, the stored entry below
-  if (r <= j) return mkz(0, 0);
-  if (r == j + 1) return mkz(1, 0);
+__device__ inline zc vref(const T* H, int ld, int r, int j, int off) {
+  // v_j(r): 0 above row j + off, 1 at row j + off, the stored entry below
+  if (r < j + off) return mkz(0, 0);
+  if (r == j + off) return mkz(1, 0);
   return ldz(H[(size_t)r + (size_t)ld * j]);
 }
 
@@ -44,15 +44,16 @@ __device__ inline void bt_pair(int t, int& pi, int& pj) {
   pj = i;
 }
 template <class T>
-__global__ __launch_bounds__(256) void k_bt_gram(const T* __restrict__ H, int ld, int N, zc* __restrict__ Gp) {
+__global__ __launch_bounds__(256) void k_bt_gram(const T* __restrict__ H, int ld, int N, int off,
+                                                 zc* __restrict__ Gp) {
   __shared__ zc Vs[kBtVR][BT_NB + 1];
   const int p = blockIdx.x * BT_NB;
-  const int kp = min(BT_NB, N - 1 - p);
+  const int kp = min(BT_NB, N - off - p);
   const int tid = threadIdx.x;
   const int npair = kp * (kp - 1) / 2;
-  const int rtot = N - 1 - p;
+  const int rtot = N - off - p;
   const int per = ((rtot + kBtSplit - 1) / kBtSplit + kBtVR - 1) / kBtVR * kBtVR;
-  const int rlo = p + 1 + (int)blockIdx.y * per, rhi = min(N, rlo + per);
+  const int rlo = p + off + (int)blockIdx.y * per, rhi = min(N, rlo + per);
   zc acc[kBtPairs];
   int pi[kBtPairs], pj[kBtPairs];
   for (int s = 0; s < kBtPairs; ++s) {
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(256) void k_bt_gram(const T* __restrict__ H, int ld
     for (int e = tid; e < kBtVR * BT_NB; e += 256) {
       const int rl = e % kBtVR, c = e / kBtVR;
       const int r = r0 + rl;
-      Vs[rl][c] = (r < rhi && c < kp) ? vref(H, ld, r, p + c) : mkz(0, 0);
+      Vs[rl][c] = (r < rhi && c < kp) ? vref(H, ld, r, p + c, off) : mkz(0, 0);
     }
     __syncthreads();
 #pragma unroll
@@ -80,12 +81,12 @@ __global__ __launch_bounds__(256) void k_bt_gram(const T* __restrict__ H, int ld
 
 // T factor of block blockIdx.x from its Gram partials (summed in range order), one
 // workgroup per block
-__global__ __launch_bounds__(256) void k_bt_tfactor(int N, const zc* __restrict__ tau, const zc* __restrict__ Gp,
+__global__ __launch_bounds__(256) void k_bt_tfactor(int N, int off, const zc* __restrict__ tau, const zc* __restrict__ Gp,
                                                     zc* __restrict__ Tf) {
   __shared__ zc G[BT_NB][BT_NB + 1];
   __shared__ zc Ts[BT_NB][BT_NB + 1];
   const int p = blockIdx.x * BT_NB;
-  const int kp = min(BT_NB, N - 1 - p);
+  const int kp = min(BT_NB, N - off - p);
   const int tid = threadIdx.x;
   const int npair = kp * (kp - 1) / 2;
   const zc* gp = Gp + (size_t)blockIdx.x * kBtSplit * kBtPairSlots;
@@ -121,11 +122,11 @@ __global__ __launch_bounds__(256) void k_bt_tfactor(int N, const zc* __restrict_
 // Ypart[chunk][c][col] = sum over the chunk's rows of conj(V(r, c)) X(r, col).
 // Workgroup: 64 reflectors x 64 columns; wave w: reflectors 16w .. 16w + 15, all 64 columns.
 template <class T>
-__global__ __launch_bounds__(256) void k_bt_vhx(const T* __restrict__ H, int ld, int N, int p, int kp,
+__global__ __launch_bounds__(256) void k_bt_vhx(const T* __restrict__ H, int ld, int N, int off, int p, int kp,
                                                 const zc* __restrict__ X, int ldx, int m, int chunk,
                                                 zc* __restrict__ Ypart) {
   const int col0 = blockIdx.x * 64;
-  const int rbeg = p + 1 + blockIdx.y * chunk;
+  const int rbeg = p + off + blockIdx.y * chunk;
   const int rend = min(N, rbeg + chunk);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(256) void k_bt_vhx(const T* __restrict__ H, int ld,
 #pragma unroll
     for (int t = 0; t < kBtSteps; ++t) {
       const int r = g0 + 4 * t + lk;
-      v[t] = (r < rend && c < kp) ? vref(H, ld, r, p + c) : mkz(0, 0);
+      v[t] = (r < rend && c < kp) ? vref(H, ld, r, p + c, off) : mkz(0, 0);
 #pragma unroll
       for (int y = 0; y < YC; ++y) {
         const int col = nb0 + y * 16 + lr;
@@ -208,12 +209,12 @@ static int bt_chunk(int rows, int ncol) {
   return std::max(64, std::min(256, (ch + 3) & ~3));
 }
 
-// X(r, col) -= sum_c V(r, c) Y(c, col) for rows r > p; 64 x 64 tiles, waves of 32 x 32
+// X(r, col) -= sum_c V(r, c) Y(c, col) for rows r >= p + off; 64 x 64 tiles, waves of 32 x 32
 template <class T>
-__global__ __launch_bounds__(256) void k_bt_update(const T* __restrict__ H, int ld, int N, int p, int kp,
+__global__ __launch_bounds__(256) void k_bt_update(const T* __restrict__ H, int ld, int N, int off, int p, int kp,
                                                    const zc* __restrict__ Y, zc* __restrict__ X, int ldx,
                                                    int m) {
-  const int rt = p + 1 + blockIdx.x * 64, col0 = blockIdx.y * 64;
+  const int rt = p + off + blockIdx.x * 64, col0 = blockIdx.y * 64;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lk = lane >> 4;
   const int rb = rt + (wave >> 1) * 32, cb = col0 + (wave & 1) * 32;
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(256) void k_bt_update(const T* __restrict__ H, int 
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         const int r = rb + x * 16 + lr;
-        v[t][x] = (k < kp && r < N) ? vref(H, ld, r, p + k) : mkz(0, 0);
+        v[t][x] = (k < kp && r < N) ? vref(H, ld, r, p + k, off) : mkz(0, 0);
       }
 #pragma unroll
       for (int y = 0; y < 2; ++y) {
@@ -304,12 +305,12 @@ size_t backtr_work_bytes(int N, int m) {
          4 * 256;
 }
 
+// X <- H(0) H(1) ... X, v_j with its 1 at row j + off; then the phases
 template <class T>
-static int run_backtr_t(hipStream_t s, const T* H, int ld, int N, const zc* tau, const double* Z, int c0,
-                        int m, zc* X, int ldx, void* work) {
-  if (N < 1 || m < 1) return WTB_OK;
+static int backtr_apply(hipStream_t s, const T* H, int ld, int N, int off, const zc* tau, int m, zc* X, int ldx,
+                        void* work) {
   char* w = static_cast<char*>(work);
-  const int np = (N - 1 + BT_NB - 1) / BT_NB;   // panels of reflectors 0 .. N-2
+  const int np = (max(N - off, 0) + BT_NB - 1) / BT_NB;   // panels of reflectors 0 .. N - off - 1
   zc* Tf = (zc*)w;
   w += ((sizeof(zc) * (size_t)(np + 1) * BT_NB * BT_NB + 255) & ~size_t(255));
   zc* Ypart = (zc*)w;
@@ -318,23 +319,21 @@ static int run_backtr_t(hipStream_t s, const T* H, int ld, int N, const zc* tau,
   zc* Y = (zc*)w;
   w += ((sizeof(zc) * BT_NB * (size_t)m + 255) & ~size_t(255));
   zc* Gp = (zc*)w;                                // Gram partials, kBtSplit per block
-  const int gl = (int)std::min<size_t>(((size_t)N * m + 255) / 256, 65536);
-  hipLaunchKernelGGL(k_bt_load, dim3(gl), dim3(256), 0, s, N, m, Z, c0, X, ldx);
   if (np > 0) {
-    hipLaunchKernelGGL(k_bt_gram<T>, dim3(np, kBtSplit), dim3(256), 0, s, H, ld, N, Gp);
-    hipLaunchKernelGGL(k_bt_tfactor, dim3(np), dim3(256), 0, s, N, tau, Gp, Tf);
+    hipLaunchKernelGGL(k_bt_gram<T>, dim3(np, kBtSplit), dim3(256), 0, s, H, ld, N, off, Gp);
+    hipLaunchKernelGGL(k_bt_tfactor, dim3(np), dim3(256), 0, s, N, off, tau, Gp, Tf);
     const int ncol = (m + 63) / 64;
     for (int b = np - 1; b >= 0; --b) {
       const int p = b * BT_NB;
-      const int kp = std::min(BT_NB, N - 1 - p);
-      const int rows = N - p - 1;
+      const int kp = std::min(BT_NB, N - off - p);
+      const int rows = N - p - off;
       const int chunk = bt_chunk(rows, ncol);
       const int nch = (rows + chunk - 1) / chunk;
-      hipLaunchKernelGGL(k_bt_vhx<T>, dim3(ncol, nch), dim3(256), 0, s, H, ld, N, p, kp, X, ldx, m, chunk,
+      hipLaunchKernelGGL(k_bt_vhx<T>, dim3(ncol, nch), dim3(256), 0, s, H, ld, N, off, p, kp, X, ldx, m, chunk,
                          Ypart);
       hipLaunchKernelGGL(k_bt_ty, dim3((m + kBtTyCols - 1) / kBtTyCols), dim3(256), 0, s, Ypart, nch, m, kp,
                          Tf + (size_t)b * BT_NB * BT_NB, Y);
-      hipLaunchKernelGGL(k_bt_update<T>, dim3((rows + 63) / 64, ncol), dim3(256), 0, s, H, ld, N, p, kp,
+      hipLaunchKernelGGL(k_bt_update<T>, dim3((rows + 63) / 64, ncol), dim3(256), 0, s, H, ld, N, off, p, kp,
                          Y, X, ldx, m);
     }
   }
@@ -343,6 +342,20 @@ static int run_backtr_t(hipStream_t s, const T* H, int ld, int N, const zc* tau,
   return WTB_OK;
 }
 
+template <class T>
+static int run_backtr_t(hipStream_t s, const T* H, int ld, int N, const zc* tau, const double* Z, int c0,
+                        int m, zc* X, int ldx, void* work) {
+  if (N < 1 || m < 1) return WTB_OK;
+  const int gl = (int)std::min<size_t>(((size_t)N * m + 255) / 256, 65536);
+  hipLaunchKernelGGL(k_bt_load, dim3(gl), dim3(256), 0, s, N, m, Z, c0, X, ldx);
+  return backtr_apply(s, H, ld, N, 1, tau, m, X, ldx, work);
+}
+
+// the panels' reflectors of a two-stage reduction (1 at row j + b of column j), onto X = Q2 Z
+int run_backtr_band(hipStream_t s, const zc* H, int ld, int N, int b, const zc* tau, int m, zc* X, int ldx,
+                    void* work) {
+  return backtr_apply(s, H, ld, N, b, tau, m, X, ldx, work);
+}
 int run_backtr(hipStream_t s, const zc* H, int ld, int N, const zc* tau, const double* Z, int c0, int m,
                zc* X, int ldx, void* work) {
   return run_backtr_t<zc>(s, H, ld, N, tau, Z, c0, m, X, ldx, work);

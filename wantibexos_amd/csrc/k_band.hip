@@ -1104,6 +1104,7 @@ struct QrPanelArgs {
   int nwg;
   int* err;
   int spin_limit;
+  zc* tau;               // where column q's tau goes; V is kept below R then (null: neither)
 };
 
 __device__ inline bool is_empty(zc v) {
@@ -1299,7 +1300,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
 #pragma unroll
   for (int j = 0; j < B; ++j) {
     const zc p = row[j];
-    if (live && i <= j) a.A[(size_t)(a.r0 + i) + (size_t)a.ld * (a.c0 + j)] = p;
+    if (live && (i <= j || a.tau)) a.A[(size_t)(a.r0 + i) + (size_t)a.ld * (a.c0 + j)] = p;
     const zc x = (j < a.k) ? (i == j ? mkz(1, 0) : (i > j ? p : mkz(0, 0))) : mkz(0, 0);
     row[j] = x;
     if (live) a.V[i + N * j] = x;
@@ -1329,8 +1330,10 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   }
   lds_barrier();
   if (bad) return;
-  if (blockIdx.x == 0)
+  if (blockIdx.x == 0) {
     for (int e = t; e < B * B; e += 256) a.Tm[e] = Ts[e % B][e / B];
+    if (a.tau && t < a.k) a.tau[t] = Ts[t][t];
+  }
   // t2 = T^H t1, gc -= V t2
 #pragma unroll
   for (int r = 0; r < 6; ++r) {
@@ -1799,6 +1802,10 @@ struct ChaseArgs {
   int* prog;         // [group] tasks that the group's last sweep has finished
   int* ctl;          // [0] error flag, [32] next group to claim
   long long spin_limit;
+  zc* Vc;            // the reflectors kept (VEC): row r of sweep s at (N - 1 - r) + ld (N - 1 - s)
+  int ld;
+  zc* tau;           // [sweep][task], kt tasks
+  int kt;
 };
 
 __host__ __device__ inline int chase_ntasks(int N, int b, int s) { return 1 + (N - 2 - s) / b; }
@@ -1890,7 +1897,7 @@ __device__ inline int lds_get(int* f) {
 // 50.8 ms for band 32, whose wave holds four times the elements; a sweep per workgroup of
 // four waves that met at barriers and moved every block through memory took 62 ms (band 32,
 // 12 us a sweep).  With eight waves a sweep and barriers, band 16 took 28 ms.
-template <int B>
+template <int B, bool VEC>
 __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseArgs a) {
   typedef ChaseDim<B> C;
   constexpr int SW = C::SW, R = C::R, NC = C::NC, P = C::P;
@@ -2052,6 +2059,10 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
       larfg_fast(first_lane(x0), xn2, beta, tau, scale);
       const zc vr = (r == 0) ? mkz(1, 0) : scale * x0;
       if (hg == 0) xv[r] = vr;
+      if constexpr (VEC) {
+        if (hg == 0 && rin) a.Vc[(size_t)(N - 1 - st - r) + (size_t)a.ld * (N - 1 - s)] = vr;
+        if (lane == 0) a.tau[(size_t)s * a.kt + k] = tau;
+      }
 #pragma unroll
       for (int q = 0; q < NC; ++q) vp[q] = xv[c0 + q];
       // (iii) z = v^H O, row quarter u summing columns u NC / 4 ..
@@ -2146,6 +2157,102 @@ __global__ void k_band_finish(const zc* __restrict__ BD, int N, int LB, double* 
 
 // control block of the chase: its error flag and sweep counter 0 (the panel's flag, [8],
 // is kept)
+// X = Q2 Z: the chase's reflectors, sweeps last to first, onto columns kept in LDS.  Bound by
+// the vector ALU: 8 N^2 flops a column as short dot products.  The wpc waves of a pair of
+// columns take its 64-row pieces (four reflectors of B rows) in turn, lane = row; the four
+// sums of a piece's two columns share their reduction over the 16 lanes (one column a wave
+// took 3.3 ms where two take 2.5, N = 1290 with all vectors).  v and tau of a wave's next
+// pieces are loaded while it works on the present ones, SB sweeps ahead where few pieces
+// make a sweep short (288 vectors of N = 1000: 0.45 ms, 3.5 with one sweep ahead), and a
+// barrier that leaves those loads in flight ends a sweep.
+struct ChaseBackArgs {
+  const zc* Vc;
+  int ld;
+  const zc* tau;
+  int kt, N;
+  const double* Z;       // N x ., columns c0 ..
+  int c0, m;
+  zc* X;
+  int ldx, pairs, wpc;   // pairs of columns of a workgroup, waves of a pair
+};
+template <int B, int U, int SB>
+__global__ __launch_bounds__(768) void k_chase_back(ChaseBackArgs a) {
+  static_assert(B == 16, "a reflector on a row of 16 lanes");
+  extern __shared__ zc xcol[];
+  const int N = a.N, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int pair = wave / a.wpc, part = wave % a.wpc, c = 2 * (blockIdx.x * a.pairs + pair);
+  const bool on = c < a.m, two = c + 1 < a.m;
+  zc* const x0 = xcol + (size_t)2 * pair * N;
+  zc* const x1 = x0 + N;
+  for (int r = part * 64 + lane; r < N; r += a.wpc * 64) {
+    x0[r] = mkz(on ? a.Z[(size_t)r + (size_t)N * (a.c0 + c)] : 0.0, 0.0);
+    x1[r] = mkz(two ? a.Z[(size_t)r + (size_t)N * (a.c0 + c + 1)] : 0.0, 0.0);
+  }
+  const bool h8 = (lane & 8) != 0, h4 = (lane & 4) != 0;
+  zc v[SB][U], t[SB][U], vn[SB][U], tn[SB][U];
+  // pieces part + wpc (u0 .. u0 + U - 1) of sweeps s, s - 1, .. (SB of them)
+  auto load = [&](int s, int u0, zc (&lv)[SB][U], zc (&lt)[SB][U]) {
+#pragma unroll
+    for (int h = 0; h < SB; ++h)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int o = 64 * (part + a.wpc * (u0 + u)) + lane, r = s - h + 1 + o;
+        const bool ok = s >= h && r < N;
+        lv[h][u] = ok ? a.Vc[(size_t)(N - 1 - r) + (size_t)a.ld * (N - 1 - s + h)] : mkz(0, 0);
+        lt[h][u] = ok ? a.tau[(size_t)(s - h) * a.kt + o / B] : mkz(0, 0);
+      }
+  };
+  load(N - 2, 0, v, t);
+  lds_barrier();
+  for (int s = N - 2; s >= 0; s -= SB) {
+    for (int u0 = 0;; u0 += U) {
+      const bool more = SB == 1 && part + a.wpc * (u0 + U) < (N - 1 - s + 63) / 64;
+      if (more) load(s, u0 + U, vn, tn);
+      else if (s >= SB) load(s - SB, 0, vn, tn);
+#pragma unroll
+      for (int h = 0; h < SB; ++h) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int rp = s - h + 1 + 64 * (part + a.wpc * (u0 + u)), r = rp + lane;
+          if (s < h || rp >= N) break;
+          const zc xa = x0[min(r, N - 1)], xb = x1[min(r, N - 1)];
+          const zc da = fma_conj(v[h][u], xa, mkz(0, 0)), db = fma_conj(v[h][u], xb, mkz(0, 0));
+          // the four sums over the 16 lanes: lanes with bit 8 keep xb's, with bit 4 the
+          // imaginary part, two more steps, then a lane of each quarter gives its sum back
+          const zc keep = h8 ? db : da;
+          zc d = h8 ? da : db;
+          d = keep + dpp_z<0x128>(d);            // row_ror:8
+          double e = h4 ? d.im : d.re;
+          const double f = h4 ? d.re : d.im;
+          e += xchg<4>(f);
+          e += dpp_d<0x4E>(e);                   // quad_perm ^2, ^1
+          e += dpp_d<0xB1>(e);
+          const zc sa = mkz(dpp_d<0x150>(e), dpp_d<0x154>(e));       // row_newbcast of lanes 0, 4, 8, 12
+          const zc sb = mkz(dpp_d<0x158>(e), dpp_d<0x15C>(e));
+          if (r < N) {
+            x0[r] = fnma_z(t[h][u] * sa, v[h][u], xa);
+            x1[r] = fnma_z(t[h][u] * sb, v[h][u], xb);
+          }
+        }
+        if (h < SB - 1) lds_barrier();
+      }
+#pragma unroll
+      for (int h = 0; h < SB; ++h)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          v[h][u] = vn[h][u];
+          t[h][u] = tn[h][u];
+        }
+      if (!more) break;
+    }
+    lds_barrier();
+  }
+  for (int r = part * 64 + lane; r < N; r += a.wpc * 64) {
+    if (on) a.X[(size_t)r + (size_t)a.ldx * c] = x0[r];
+    if (two) a.X[(size_t)r + (size_t)a.ldx * (c + 1)] = x1[r];
+  }
+}
+
 __global__ void k_chase_init(int* ctl) {
   const int i = threadIdx.x;
   if (i == 0 || i == 32) ctl[i] = 0;
@@ -2338,7 +2445,8 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
         zc* A22 = H + r0 + (size_t)ld * r0;
         if (p > 0)
           hipLaunchKernelGGL((k_strip<B>), dim3((m + B + 63) / 64), blk, 0, s, H + c0 + (size_t)ld * c0, ld, m + B, N, Vo, Xo);
-        QrPanelArgs q{H, ld, N, c0, r0, m, k, V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20};
+        QrPanelArgs q{H, ld, N, c0, r0, m, k, V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20,
+                      w.tau1 ? w.tau1 + c0 : nullptr};
         hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, q);
         const int n = um_steps(m), nt = (m + UM_R - 1) / UM_R;
         const dim3 gt(4 / n * (nt * (nt + 1) / 2));
@@ -2390,6 +2498,11 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
     return WTB_ERR_ARG;
   }
   if (nrhs > 6) return WTB_ERR_LIMIT;
+  if (w.tau1) {
+    // the kept reflectors are those of the one-launch panels of the COMPLEX*16 matrix
+    if (!std::is_same<T, zc>::value || b != 16 || N > band_vec_rows()) return WTB_ERR_LIMIT;
+    hipLaunchKernelGGL(k_zero_ints, dim3((4 * N + 255) / 256), dim3(256), 0, s, (int*)w.tau1, 4 * N);
+  }
   if (nrhs > 0)
     hipLaunchKernelGGL(k_conj_vec, dim3((unsigned)(((size_t)nrhs * N + 255) / 256)), dim3(256), 0, s, nrhs * N, g,
                        w.gc);
@@ -2418,12 +2531,46 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
   const int sw = (b == 16) ? ChaseDim<16>::SW : ChaseDim<32>::SW;
   const int ngrp = (N - 1 + sw - 1) / sw;
   const int P = min(ngrp, min(256, chase_ntasks(N, b, 0) / (2 * sw) + 4));
-  if (b == 16) hipLaunchKernelGGL(k_chase<16>, dim3(P), dim3((sw + 1) * 64), 0, s, ca);
-  else hipLaunchKernelGGL(k_chase<32>, dim3(P), dim3((sw + 1) * 64), 0, s, ca);
+  ca.Vc = nullptr;
+  if constexpr (std::is_same<T, zc>::value)
+    if (w.tau1) ca.Vc = H;
+  ca.ld = ld;
+  ca.tau = w.tau2;
+  ca.kt = chase_ntasks(N, b, 0);
+  auto chase = b == 32 ? k_chase<32, false> : ca.Vc ? k_chase<16, true> : k_chase<16, false>;
+  hipLaunchKernelGGL(chase, dim3(P), dim3((sw + 1) * 64), 0, s, ca);
   hipLaunchKernelGGL(k_band_finish, dim3((N + 255) / 256), dim3(256), 0, s, w.BD, N, w.LB, d, e, w.gc, g, nrhs,
                      w.err, status);
   WTB_LAUNCH_CHECK();
   return WTB_OK;
+}
+
+// two columns of X fit the LDS of a compute unit
+int band_vec_rows() { return 160 * 1024 / (2 * (int)sizeof(zc)); }
+// Whether a solve with m eigenvectors takes the two-stage reduction (COMPLEX*16).  It saves
+// 8 to 16 us a column of the one-stage form and pays N^2 m for the chase's reflectors.
+// zheev with all vectors, two-stage / one-stage: N = 256 4.4 / 6.4 ms, 640 8.5 / 13.7, 1290 21
+// / 29, 2049 45 / 52, 2500 62 / 69, 3000 86 / 91: the line lies where N m is 3000^2.
+bool band_vec_two_stage(int N, int m) {
+  return N >= 32 && N <= band_vec_rows() && (double)N * m <= 9e6;
+}
+size_t band_tau_elems(int N) { return (size_t)N + (size_t)N * (N / 16 + 1); }
+
+int run_band_backtr(hipStream_t s, const BandWork& w, const zc* H, int ld, const double* Z, int c0, int m, zc* X,
+                    int ldx, int cus, void* work) {
+  const int N = w.N;
+  if (N < 2 || m < 1 || !w.tau1 || N > band_vec_rows()) return WTB_ERR_ARG;
+  // every pair of columns at work at once where the LDS holds them, 12 waves a workgroup,
+  // fewer where the pieces do not need them
+  const int pieces = (N + 63) / 64, np = (m + 1) / 2;
+  const int pairs = std::max(1, std::min({(np + std::max(cus, 1) - 1) / std::max(cus, 1), band_vec_rows() / N, 12}));
+  const int wpc = std::max(1, std::min(12 / pairs, pieces));
+  // pieces of a wave and sweeps ahead: few pieces need more sweeps to cover a load
+  auto kern = pieces <= 2 * wpc ? k_chase_back<16, 2, 3> : k_chase_back<16, 4, 1>;
+  WTB_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+  ChaseBackArgs a{H, ld, w.tau2, chase_ntasks(N, 16, 0), N, Z, c0, m, X, ldx, pairs, wpc};
+  hipLaunchKernelGGL(kern, dim3((np + pairs - 1) / pairs), dim3(64 * pairs * wpc), 2 * pairs * N * (int)sizeof(zc), s, a);
+  return run_backtr_band(s, H, ld, N, 16, w.tau1, m, X, ldx, work);
 }
 
 int run_band_tridiag(hipStream_t s, BandWork& w, zc* H, int ld, zc* g, double* d, double* e, int* status) {

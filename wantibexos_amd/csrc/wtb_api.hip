@@ -1085,10 +1085,12 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
   int* dst = nullptr;
   int rc, st = 0;
   // eigenvalues alone take the two-stage reduction, as a plan's do (plan_two_stage)
-  const bool two = !vec && n >= kTwoStageMinN64;
+  const bool two = vec ? band_vec_two_stage(n, n) : n >= kTwoStageMinN64;
   const int band = plan_default_band(false, n);
+  const size_t ntau = two && vec ? band_tau_elems(n) : 0;
   if ((rc = dmalloc(&da, (size_t)lda * n)) || (rc = dmalloc(&dh, (size_t)n * n)) || (rc = dmalloc(&dst, 1)) ||
-      (rc = dmalloc((char**)&tri, two ? band_work_bytes(n, band, 0) + sizeof(double) * 2 * n : tridiag_work_bytes(n, 32, 0))) ||
+      (rc = dmalloc((char**)&tri, two ? band_work_bytes(n, band, 0) + sizeof(double) * 2 * n + sizeof(zc) * ntau
+                                      : tridiag_work_bytes(n, 32, 0))) ||
       (rc = dmalloc((char**)&dcw, dc_work_bytes(n, 0, vec))) || (rc = dmalloc(&dl, n)) ||
       (vec && ((rc = dmalloc(&dz, (size_t)n * n)) || (rc = dmalloc(&dx, (size_t)n * n)) ||
                (rc = dmalloc((char**)&btw, backtr_work_bytes(n, n)))))) {
@@ -1096,12 +1098,16 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
     TridiagWork tw;
     BandWork bw;
     DCTree tree;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 0;
     if (two) {
       tw.d = static_cast<double*>(tri);
       tw.e = tw.d + n;
-      rc = band_bind(bw, tw.e + n, n, band, 0);
-      int cus = 0;
-      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 0;
+      rc = band_bind(bw, tw.e + n + 2 * ntau, n, band, 0);
+      if (vec) {
+        bw.tau1 = reinterpret_cast<zc*>(tw.e + n);
+        bw.tau2 = bw.tau1 + n;
+      }
       bw.panel_resident = cus;
     } else {
       tridiag_bind(tw, tri, n, 32, 0);
@@ -1115,7 +1121,9 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
       rc = two ? run_band_tridiag(s, bw, dh, n, nullptr, tw.d, tw.e, dst) : run_tridiag(s, tw, dh, n, nullptr);
     }
     if (!rc) rc = run_dc(s, dcw, tree, tw.d, tw.e, nullptr, dl, dz);
-    if (!rc && vec) rc = run_backtr(s, dh, n, n, tw.tau, dz, 0, n, dx, n, btw);
+    if (!rc && vec)
+      rc = two ? run_band_backtr(s, bw, dh, n, dz, 0, n, dx, n, cus, btw)
+               : run_backtr(s, dh, n, n, tw.tau, dz, 0, n, dx, n, btw);
     if (!rc) {
       hipMemcpyAsync(w, dl, sizeof(double) * n, hipMemcpyDeviceToHost, s);
       hipMemcpyAsync(&st, dst, sizeof(int), hipMemcpyDeviceToHost, s);

@@ -148,6 +148,11 @@ struct BandWork {
   int panel_wg = 0;             // COMPLEX*16: panel and W in one launch each up to this many workgroups
   zc* ex = nullptr;             // their exchange slots, two panel parities
   zc *V2 = nullptr, *X2 = nullptr;   // every other panel's V and W
+  // COMPLEX*16, band 16: keep the reflectors for run_band_backtr, the panels' below the band,
+  // the chase's in the strict upper triangle of H (row r of sweep s at row N - 1 - r, column
+  // N - 1 - s), and their tau here (null: not kept)
+  zc* tau1 = nullptr;           // N
+  zc* tau2 = nullptr;           // N (N / 16 + 1)
   // optional per-launch timing of the trailing-update kernel (k_update_mul with COMPLEX*16 and
   // band 16, else k_her2k_full): launch c is
   // bracketed by kev[2c], kev[2c+1] (c < kev_cap); kev_flops[c] its flop count
@@ -157,6 +162,13 @@ struct BandWork {
   double kev_flops = 0.0;       // summed over the timed launches
 };
 size_t band_work_bytes(int N, int b, int nrhs);
+// eigenvectors from Z (N x ., real) after a reduction that kept its reflectors: columns
+// c0 .. c0 + m - 1; N <= band_vec_rows()
+bool band_vec_two_stage(int N, int m);   // the faster form for m vectors
+size_t band_tau_elems(int N);     // tau1 and tau2 together
+int band_vec_rows();
+int run_band_backtr(hipStream_t s, const BandWork& w, const zc* H, int ld, const double* Z, int c0, int m, zc* X,
+                    int ldx, int cus, void* work);
 int band_panel_rows();            // largest N whose COMPLEX*16 panels run in one launch (band 16)
 int band_bind(BandWork& w, void* base, int N, int b, int nrhs);
 int run_band_tridiag(hipStream_t s, BandWork& w, zc* H, int ld, zc* g, double* d, double* e, int* status);
@@ -181,6 +193,8 @@ int run_dc(hipStream_t s, void* work, const DCTree& tree, const double* d_d, con
 size_t backtr_work_bytes(int N, int m);
 int run_backtr(hipStream_t s, const zc* H, int ld, int N, const zc* tau, const double* Z, int c0, int m,
                zc* X, int ldx, void* work);
+int run_backtr_band(hipStream_t s, const zc* H, int ld, int N, int b, const zc* tau, int m, zc* X, int ldx,
+                    void* work);
 int run_backtr_f32(hipStream_t s, const zf* H, int ld, int N, const zc* tau, const double* Z, int c0,
                    int m, zc* X, int ldx, void* work);
 
