@@ -59,23 +59,13 @@ __device__ inline zc zdiv(zc a, zc b) {
 
 __device__ inline zc shfl_xor_z(zc v, int off) { return mkz(__shfl_xor(v.re, off), __shfl_xor(v.im, off)); }
 
-// x of another lane by a DPP lane permutation (within rows of 16 lanes) or a swizzle
-// (within 32 lanes); both halves of the double move
-template <int CTRL>
-__device__ inline double dpp_d(double x) {
-  const long long v = __builtin_bit_cast(long long, x);
-  const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xF, 0xF, false);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
-}
-__device__ inline double swz16_d(double x) {   // lane ^ 16 within 32 lanes
+// lane ^ 16 within 32 lanes, by a swizzle
+__device__ inline double swz16_d(double x) {
   const long long v = __builtin_bit_cast(long long, x);
   const int lo = __builtin_amdgcn_ds_swizzle((int)v, 0x401F);
   const int hi = __builtin_amdgcn_ds_swizzle((int)(v >> 32), 0x401F);
   return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
 }
-template <int CTRL>
-__device__ inline zc dpp_z(zc v) { return mkz(dpp_d<CTRL>(v.re), dpp_d<CTRL>(v.im)); }
 
 // The value of the partner lane that differs from this one in lane bit OFF and agrees in
 // the bits above it: ^1 and ^2 by quad permutations, i <-> 7 - i (row half mirror) for 4,
@@ -982,33 +972,6 @@ __global__ void k_band_extract(const T* __restrict__ A, int ld, int N, int b, in
 __global__ void k_conj_vec(int n, const zc* __restrict__ x, zc* __restrict__ y) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = conj(x[i]);
-}
-
-// Lane halves and 16-lane rows by the swap instructions (VALU, no LDS round trip): after
-// swap32(a, b) lane l < 32 holds a(l) and a(l + 32), lane l >= 32 b(l - 32) and b(l); swap16
-// does the same within each pair of 16-lane rows.  a + b is then a sum over that lane bit,
-// of a in the lanes where the bit is clear and of b where it is set.
-__device__ inline void swap32(double& a, double& b) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
-  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-  a = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
-  b = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-}
-__device__ inline void swap16(double& a, double& b) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
-  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-  a = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
-  b = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-}
-__device__ inline double add32(double a, double b) {
-  swap32(a, b);
-  return a + b;
-}
-__device__ inline double add16(double a, double b) {
-  swap16(a, b);
-  return a + b;
 }
 
 // sum over groups of SUB (8 or 16) consecutive lanes, the same bits in each: ^1, ^2, then

@@ -61,84 +61,89 @@ struct TriArgs {
   int nblk;
 };
 
-__device__ inline zc wave_sum(zc v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    v.re += __shfl_xor(v.re, off);
-    v.im += __shfl_xor(v.im, off);
-  }
+// The value of lane ^ OFF: rotations and permutations of the vector ALU (4 is a mirror of 8
+// lanes, ^7, and a reversal of quads, ^3), without the LDS round trip of a shuffle
+template <int CTRL>
+__device__ inline float dpp_f(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
+}
+template <int OFF>
+__device__ inline double lane_xor(double x) {
+  if constexpr (OFF == 8) return dpp_d<0x128>(x);
+  else if constexpr (OFF == 4) return dpp_d<0x1B>(dpp_d<0x141>(x));
+  else if constexpr (OFF == 2) return dpp_d<0x4E>(x);
+  else return dpp_d<0xB1>(x);
+}
+template <int OFF>
+__device__ inline float lane_xor(float x) {
+  if constexpr (OFF == 8) return dpp_f<0x128>(x);
+  else if constexpr (OFF == 4) return dpp_f<0x1B>(dpp_f<0x141>(x));
+  else if constexpr (OFF == 2) return dpp_f<0x4E>(x);
+  else return dpp_f<0xB1>(x);
+}
+template <int OFF>
+__device__ inline zc lane_xor(zc v) { return mkz(lane_xor<OFF>(v.re), lane_xor<OFF>(v.im)); }
+template <int OFF>
+__device__ inline zf lane_xor(zf v) { return zf{lane_xor<OFF>(v.re), lane_xor<OFF>(v.im)}; }
+// sum over the 16 lanes of a row, 4 lanes of a quad, the wave: the partners lane ^ OFF in
+// falling order
+__device__ inline zc row_sum(zc v) {
+  v += lane_xor<8>(v);
+  v += lane_xor<4>(v);
+  v += lane_xor<2>(v);
+  v += lane_xor<1>(v);
   return v;
 }
+__device__ inline zc quad_sum(zc v) {
+  v += lane_xor<2>(v);
+  v += lane_xor<1>(v);
+  return v;
+}
+__device__ inline zc wave_sum(zc v) {
+  v = mkz(add32(v.re, v.re), add32(v.im, v.im));
+  v = mkz(add16(v.re, v.re), add16(v.im, v.im));
+  return row_sum(v);
+}
 
-// Sum of each of 16 values over the 64 lanes of a wave (pv: a zc[16] in registers):
-// every butterfly step halves the set a lane keeps; afterwards lane l holds the sum for
-// index (l >> 2) & 15.  A macro, so that the array is never addressed through memory.
-#define BUTTERFLY16(pv, lane)                                             \
-  do {                                                                    \
-    int n_ = 16;                                                          \
-    for (int off_ = 32; off_ >= 4; off_ >>= 1) {                          \
-      n_ >>= 1;                                                           \
-      const bool up_ = ((lane) & off_) != 0;                              \
-      for (int i_ = 0; i_ < n_; ++i_) {                                   \
-        const zc send_ = up_ ? pv[i_] : pv[i_ + n_];                      \
-        zc recv_;                                                         \
-        recv_.re = __shfl_xor(send_.re, off_);                            \
-        recv_.im = __shfl_xor(send_.im, off_);                            \
-        pv[i_] = (up_ ? pv[i_ + n_] : pv[i_]) + recv_;                    \
-      }                                                                   \
-    }                                                                     \
-    for (int off_ = 2; off_ > 0; off_ >>= 1) {                            \
-      pv[0].re += __shfl_xor(pv[0].re, off_);                             \
-      pv[0].im += __shfl_xor(pv[0].im, off_);                             \
-    }                                                                     \
-  } while (0)
-
-// the same for 8 values: lane holds the sum for value (lane >> 3) & 7
-#define BUTTERFLY8(pv, lane)                                              \
-  do {                                                                    \
-    int n_ = 8;                                                           \
-    for (int off_ = 32; off_ >= 8; off_ >>= 1) {                          \
-      n_ >>= 1;                                                           \
-      const bool up_ = ((lane) & off_) != 0;                              \
-      for (int i_ = 0; i_ < n_; ++i_) {                                   \
-        const zc send_ = up_ ? pv[i_] : pv[i_ + n_];                      \
-        zc recv_;                                                         \
-        recv_.re = __shfl_xor(send_.re, off_);                            \
-        recv_.im = __shfl_xor(send_.im, off_);                            \
-        pv[i_] = (up_ ? pv[i_ + n_] : pv[i_]) + recv_;                    \
-      }                                                                   \
-    }                                                                     \
-    for (int off_ = 4; off_ > 0; off_ >>= 1) {                            \
-      pv[0].re += __shfl_xor(pv[0].re, off_);                             \
-      pv[0].im += __shfl_xor(pv[0].im, off_);                             \
-    }                                                                     \
-  } while (0)
-
-// the same on COMPLEX*8 values (FP32 sums over the 64 rows of a tile)
 __device__ inline zf operator+(zf a, zf b) {
   zf c;
   c.re = a.re + b.re;
   c.im = a.im + b.im;
   return c;
 }
-#define BUTTERFLY16F(pv, lane)                                            \
-  do {                                                                    \
-    int n_ = 16;                                                          \
-    for (int off_ = 32; off_ >= 4; off_ >>= 1) {                          \
-      n_ >>= 1;                                                           \
-      const bool up_ = ((lane) & off_) != 0;                              \
-      for (int i_ = 0; i_ < n_; ++i_) {                                   \
-        const zf send_ = up_ ? pv[i_] : pv[i_ + n_];                      \
-        zf recv_;                                                         \
-        recv_.re = __shfl_xor(send_.re, off_);                            \
-        recv_.im = __shfl_xor(send_.im, off_);                            \
-        pv[i_] = (up_ ? pv[i_ + n_] : pv[i_]) + recv_;                    \
-      }                                                                   \
-    }                                                                     \
-    for (int off_ = 2; off_ > 0; off_ >>= 1) {                            \
-      pv[0].re += __shfl_xor(pv[0].re, off_);                             \
-      pv[0].im += __shfl_xor(pv[0].im, off_);                             \
-    }                                                                     \
-  } while (0)
+// Sum of each of E = 16 or 8 values over the 64 lanes of a wave: every step halves the set a
+// lane keeps; afterwards lane l holds the sum for index (l >> 2) & 15 (E = 16) or
+// (l >> 3) & 7 in pv[0].  COMPLEX*8 values are summed in FP32.  The sums are
+// those of shuffles through LDS, whose round trips they save: k_tri_hemv 12.3 -> 11.1 us a
+// launch on the COMPLEX*8 matrix at N = 5184 (k_tri_rowstep 8.3 -> 7.9).  Loading what x~
+// needs ahead of the tile, or up to 24 partial sums at a time, changed nothing.
+template <int E, class Z>
+__device__ __forceinline__ void butterfly(Z (&pv)[E], int lane) {
+#pragma unroll
+  for (int i = 0; i < E / 2; ++i) {
+    pv[i].re = add32(pv[i].re, pv[i + E / 2].re);
+    pv[i].im = add32(pv[i].im, pv[i + E / 2].im);
+  }
+#pragma unroll
+  for (int i = 0; i < E / 4; ++i) {
+    pv[i].re = add16(pv[i].re, pv[i + E / 4].re);
+    pv[i].im = add16(pv[i].im, pv[i + E / 4].im);
+  }
+  const bool h8 = (lane & 8) != 0, h4 = (lane & 4) != 0;
+#pragma unroll
+  for (int i = 0; i < E / 8; ++i) {
+    const Z send = h8 ? pv[i] : pv[i + E / 8];
+    pv[i] = (h8 ? pv[i + E / 8] : pv[i]) + lane_xor<8>(send);
+  }
+  if constexpr (E == 16) {
+    const Z send = h4 ? pv[0] : pv[1];
+    pv[0] = (h4 ? pv[1] : pv[0]) + lane_xor<4>(send);
+  } else {
+    pv[0] = pv[0] + lane_xor<4>(pv[0]);
+  }
+  pv[0] = pv[0] + lane_xor<2>(pv[0]);
+  pv[0] = pv[0] + lane_xor<1>(pv[0]);
+}
 
 // alpha' = -1/2 |tau|^2 sum_b puv[b] over the np partials of the previous rowstep, in a
 // fixed order (every thread of the workgroup returns it)
@@ -190,10 +195,7 @@ __device__ void reflector_scalars(const TriArgs<T>& a, int jm, int jjh, zc* sums
       }
       acc = strided_sum(base, stride, b0h + sub, a.nblk, 4, acc);
     }
-    for (int off = 2; off > 0; off >>= 1) {
-      acc.re += __shfl_xor(acc.re, off, 4);
-      acc.im += __shfl_xor(acc.im, off, 4);
-    }
+    acc = quad_sum(acc);
     if (sub == 0 && q < nq) sums[q] = acc;
   }
   __syncthreads();
@@ -317,10 +319,7 @@ __device__ __forceinline__ void tri_rowstep(const TriArgs<T>& a, int bx, int j, 
         acc = acc - w2[k] * st2[c];
       }
     }
-    for (int off = 8; off > 0; off >>= 1) {
-      acc.re += __shfl_xor(acc.re, off, 16);
-      acc.im += __shfl_xor(acc.im, off, 16);
-    }
+    acc = row_sum(acc);
     return acc;
   };
   // u(j): every workgroup needs it for the column update; the same lanes publish
@@ -372,10 +371,7 @@ __device__ __forceinline__ void tri_rowstep(const TriArgs<T>& a, int bx, int j, 
         acc = acc + vc * conj(sWj[c]) + wc * conj(sVj[c]);
       }
     }
-    for (int off = 8; off > 0; off >>= 1) {
-      acc.re += __shfl_xor(acc.re, off, 16);
-      acc.im += __shfl_xor(acc.im, off, 16);
-    }
+    acc = row_sum(acc);
     if (sub == 0) a.xp[r] = hcol - acc;
   }
   __syncthreads();
@@ -481,11 +477,11 @@ __device__ __forceinline__ void hemv_quant_pass(const TriArgs<T>& a, HemvPV<hemv
   int q;
   bool head;
   if constexpr (EPQ == 8) {
-    BUTTERFLY8(pv, lane);
+    butterfly(pv, lane);
     q = q0 + ((lane >> 3) & 7);
     head = (lane & 7) == 0;
   } else {
-    BUTTERFLY16(pv, lane);
+    butterfly(pv, lane);
     q = q0 + ((lane >> 2) & 15);
     head = (lane & 3) == 0;
   }
@@ -627,7 +623,7 @@ __device__ __forceinline__ void tri_hemv_tile(const TriArgs<T>& a, int ti, int t
       hf[k].im = low ? t.im : 0.0f;
     }
     y1s[w][lane] = ldz(y1f);
-    BUTTERFLY16F(hf, lane);
+    butterfly(hf, lane);
     if ((lane & 3) == 0) y2s[0][16 * w + ((lane >> 2) & 15)] = ldz(hf[0]);
   } else {
 #pragma unroll
@@ -640,7 +636,7 @@ __device__ __forceinline__ void tri_hemv_tile(const TriArgs<T>& a, int ti, int t
     }
     y1s[w][lane] = y1;
     // transpose-reduce the 16 column sums over the 64 lanes: halve the set per butterfly step
-    BUTTERFLY16(hv, lane);
+    butterfly(hv, lane);
     // lane holds the sum for column 16w + ((lane >> 2) & 15)
     if ((lane & 3) == 0) y2s[0][16 * w + ((lane >> 2) & 15)] = hv[0];
   }
@@ -708,7 +704,7 @@ __device__ __forceinline__ void tri_hemv_tile(const TriArgs<T>& a, int ti, int t
         if (q == 0) v = mkz(xr2, 0.0);
         pv[k] = (q < nq && rok) ? v : mkz(0, 0);
       }
-      BUTTERFLY16(pv, lane);
+      butterfly(pv, lane);
       const int q = q0 + ((lane >> 2) & 15);
       if ((lane & 3) == 0 && q < nq) {
         if (q == 0) a.pn[bi] = pv[0].re;
@@ -882,7 +878,7 @@ __device__ __forceinline__ void tri_hemv_pair(const TriArgs<T>& a, int pb, int n
       hf[k].im = on ? t.im : 0.0f;
     }
     y1s[u][w][lane] = ldz(y1f);
-    BUTTERFLY16F(hf, lane);
+    butterfly(hf, lane);
     if ((lane & 3) == 0) y2s[u][16 * w + ((lane >> 2) & 15)] = ldz(hf[0]);
   }
   __syncthreads();

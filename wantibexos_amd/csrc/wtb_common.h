@@ -51,6 +51,55 @@ __device__ inline zc fma_z(zc a, zc b, zc acc) {
   return acc;
 }
 
+// x of another lane by a DPP lane permutation (within rows of 16 lanes); both halves of the
+// double move
+template <int CTRL>
+__device__ inline double dpp_d(double x) {
+  const long long v = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
+}
+template <int CTRL>
+__device__ inline zc dpp_z(zc v) { return mkz(dpp_d<CTRL>(v.re), dpp_d<CTRL>(v.im)); }
+
+// Lane halves and 16-lane rows by the swap instructions (VALU, no LDS round trip): after
+// swap32(a, b) lane l < 32 holds a(l) and a(l + 32), lane l >= 32 b(l - 32) and b(l); swap16
+// does the same within each pair of 16-lane rows.  a + b is then a sum over that lane bit,
+// of a in the lanes where the bit is clear and of b where it is set.
+__device__ inline void swap32(double& a, double& b) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
+  b = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline void swap16(double& a, double& b) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]);
+  b = __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline double add32(double a, double b) {
+  swap32(a, b);
+  return a + b;
+}
+__device__ inline double add16(double a, double b) {
+  swap16(a, b);
+  return a + b;
+}
+__device__ inline float add32(float a, float b) {
+  const auto v = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned x = v[0], y = v[1];           // (bit_cast of a vector's element reads element 0)
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+__device__ inline float add16(float a, float b) {
+  const auto v = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned x = v[0], y = v[1];
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+
 // sum of p[b * stride] over b = b0, b0 + step, ... < b1, added in that order, with the loads
 // issued eight at a time (a plain loop waits for each load before the next).  The last
 // group loads from clamped indices (b1 - 1 is in range whenever the group runs) and adds
