@@ -77,7 +77,8 @@ __global__ void k_quantize(int n, const double* __restrict__ src, double* __rest
 }
 
 // avgsme (optics.f90:302-324): sequential sum of successive differences, in the
-// reference's order; the energies are staged through LDS in chunks
+// reference's order; the energies are staged through LDS in chunks and read 16 ahead of the
+// chain of additions, which is all that is left to wait for (8.5 -> 7.5 us at N = 576, 133 us at 14400)
 __global__ __launch_bounds__(256) void k_avgsme(int N, const double* __restrict__ E, double* __restrict__ out) {
   __shared__ double buf[4097];
   double s = 0.0, prev = 0.0;
@@ -87,9 +88,20 @@ __global__ __launch_bounds__(256) void k_avgsme(int N, const double* __restrict_
     for (int i = threadIdx.x; i < m; i += 256) buf[i] = E[c0 + i];
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (int i = 0; i < m; ++i) {
-        const int gi = c0 + i;
-        if (gi > 0) s = s + buf[i] - prev;
+      int i = 0;
+      if (c0 == 0) prev = buf[i++];
+      for (; i + 16 <= m; i += 16) {
+        double b[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) b[u] = buf[i + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          s = s + b[u] - prev;
+          prev = b[u];
+        }
+      }
+      for (; i < m; ++i) {
+        s = s + buf[i] - prev;
         prev = buf[i];
       }
     }
@@ -99,7 +111,10 @@ __global__ __launch_bounds__(256) void k_avgsme(int N, const double* __restrict_
 
 // optdiel for 4 photon energies per workgroup and all six components:
 //   eps2 = caux sum f g/((w-E)^2+g^2),  eps1 = delta + caux sum f (E-w)/((w-E)^2+g^2)
-// with g = sme + avgsme; partial sums reduced in a fixed tree order.
+// with g = sme + avgsme; partial sums reduced in a fixed tree order: threads t and t + 128,
+// t + 64, .. t + 1.  The sums of a part go through LDS together, a quarter to each wave, which
+// finishes the tree by lane exchanges (a barrier for each step of each sum's tree took 55 us
+// at 1001 energies and N = 576, this takes 7.3).
 #define OMB 4
 __global__ __launch_bounds__(256) void k_optdiel(int N, const double* __restrict__ E,
                                                  const double* __restrict__ f6, double caux,
@@ -107,7 +122,8 @@ __global__ __launch_bounds__(256) void k_optdiel(int N, const double* __restrict
                                                  const double* __restrict__ smeavg,
                                                  double* __restrict__ eps) {
 #pragma clang fp contract(off)
-  __shared__ double red[256];
+  constexpr int NV = OMB * 6;                  // sums of either part
+  __shared__ double red[NV][256];
   const int j0 = blockIdx.x * OMB;
   const double smef = smeavg[0] + sme;
   double om[OMB];
@@ -133,64 +149,70 @@ __global__ __launch_bounds__(256) void k_optdiel(int N, const double* __restrict
       }
     }
   }
-  for (int q = 0; q < OMB; ++q)
-    for (int c = 0; c < 6; ++c)
-      for (int part = 0; part < 2; ++part) {
-        double v = part ? si[q][c] : sr[q][c];
-        red[threadIdx.x] = v;
-        __syncthreads();
-        for (int s = 128; s > 0; s >>= 1) {
-          if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-          __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-          int j = j0 + q;
-          if (j < numbse) {
-            double out = part ? red[0] * caux : (c < 3 ? 1.0 : 0.0) + red[0] * caux;
-            eps[j + (size_t)numbse * (part + 2 * c)] = out;
-          }
-        }
-        __syncthreads();
-      }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int part = 0; part < 2; ++part) {
+    if (part) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < OMB; ++q)
+#pragma unroll
+      for (int c = 0; c < 6; ++c) red[q * 6 + c][threadIdx.x] = part ? si[q][c] : sr[q][c];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NV / 4; u += 2) {
+      auto waves = [&](int v) { return (red[v][lane] + red[v][lane + 128]) + (red[v][lane + 64] + red[v][lane + 192]); };
+      // the one sum in lanes 0 .. 31, the next in the others
+      const int v0 = wave * (NV / 4) + u, v = v0 + (lane >> 5), j = j0 + v / 6, c = v % 6;
+      double x = add32(waves(v0), waves(v0 + 1));
+      x = add16(x, x);
+      x += dpp_d<0x128>(x);                    // lane ^ 8, ^ 4, ^ 2, ^ 1
+      x += dpp_d<0x1B>(dpp_d<0x141>(x));
+      x += dpp_d<0x4E>(x);
+      x += dpp_d<0xB1>(x);
+      if (j < numbse && (lane & 31) == 0)
+        eps[j + (size_t)numbse * (part + 2 * c)] = part ? x * caux : (c < 3 ? 1.0 : 0.0) + x * caux;
+    }
+  }
 }
 
 // imagrenorm (optics.f90:327-390) on eps2 of each component
 __global__ __launch_bounds__(256) void k_imagrenorm(const double* __restrict__ E, double ebse0, double ebsef,
                                                     int numbse, double* __restrict__ eps) {
 #pragma clang fp contract(off)
-  __shared__ int sib;
-  __shared__ double saux3;
+  // the last grid point of the leading ones at or below aux: one before the first that is
+  // not, found by all threads (one thread's search took 20 us of the kernel's 28, now
+  // 9.1)
+  __shared__ int sfail;
   const double factor = (double)0.15f;
   const double aux = E[0] - factor;
   if (aux <= 0.0) return;
-  if (threadIdx.x == 0) {
-    int ib = 0;
-    for (int j = 0; j < numbse; ++j) {
-      double w = ebse0 + ((ebsef - ebse0) * (double)j) / ((double)numbse - 1.0);
-      if (w <= aux) ib = j;
-      else break;
+  if (threadIdx.x == 0) sfail = numbse;
+  __syncthreads();
+  for (int j = threadIdx.x; j < numbse; j += 256) {
+    const double w = ebse0 + ((ebsef - ebse0) * (double)j) / ((double)numbse - 1.0);
+    if (!(w <= aux)) {
+      atomicMin(&sfail, j);
+      break;
     }
-    sib = ib;
   }
   __syncthreads();
-  const int ib = sib;
-  for (int c = 0; c < 6; ++c) {
-    double* im = eps + (size_t)numbse * (1 + 2 * c);
-    if (threadIdx.x == 0) saux3 = (ib + 1 < numbse) ? im[ib + 1] : 0.0;
-    __syncthreads();
-    const double aux3 = saux3;
-    for (int j = threadIdx.x; j < numbse; j += 256) {
+  const int ib = max(sfail - 1, 0);
+  double aux3[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) aux3[c] = (ib + 1 < numbse) ? eps[(size_t)numbse * (1 + 2 * c) + ib + 1] : 0.0;
+  __syncthreads();
+  for (int j = threadIdx.x; j < numbse; j += 256)
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      double* im = eps + (size_t)numbse * (1 + 2 * c);
       double v;
       if (ib + 1 >= numbse) v = 0.0;          // the reference would read past the grid; zero it all
       else if (j <= ib) v = 0.0;
       else {
-        v = im[j] - aux3;
+        v = im[j] - aux3[c];
         v = v < 0.0 ? 0.0 : v;
       }
       im[j] = v;
     }
-    __syncthreads();
-  }
 }
 
 // t_i = sum_j X(j,i) h(j) for up to two vectors (dielbsev / dielbsep), one wave per column i
