@@ -1536,11 +1536,13 @@ __global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m
 // row blocks from K on); k_um_sum adds them in order.
 //
 // 256 m^2 flops over 16 m^2 bytes and 2 m^2 of parts: at m = 14400 0.73 ms of the matrix cores
-// and 0.73 ms of memory, and the kernel takes 1.15 ms (46 TFLOP/s, 3.7 TB/s with the operands
-// that miss the L2; the matrix cores are busy 63 % of the time).  Two kernels, a product over
+// and 0.73 ms of memory, and the kernel takes 1.11 ms (48 TFLOP/s, 3.8 TB/s with the operands
+// that miss the L2; the matrix cores are busy 65 % of the time).  Two kernels, a product over
 // 16 m^2 bytes and an update over 16 m^2, took 483 ms of a reduction at N = 14400 where this
-// one and k_um_sum take 385, and 27 ms of one at N = 5184 (20 here).  64 x 64 tiles, three
-// waves per SIMD with spills, and an order of the tiles by XCD were no faster.
+// one and k_um_sum take 373, and 27 ms of one at N = 5184 (19 here).  Y ahead of the products
+// that use it took 14 ms of that, their wave's priority 1 ms of a plan at N = 5184 (a higher
+// priority for the loads instead cost 68 ms at 14400).  64 x 64 tiles, three waves per SIMD
+// with spills, and an order of the tiles by XCD were no faster.
 #define UM_R 128
 __host__ __device__ inline int um_parts(int K, int n, int nt) { return 4 / n * (K + 1) + nt - K; }
 template <int B, bool UPD>
@@ -1587,6 +1589,11 @@ __global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int l
             h[x][y][2 * e] = v.re;
             h[x][y][2 * e + 1] = v.im;
           }
+      zc ya[4][2], yb[2][4];                   // Y of the step's columns and of the rows
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) ya[x][e] = Y[(size_t)min(c0 + 8 * x + 4 * e + lk, m - 1) + (size_t)N * lr];
       if constexpr (UPD) {
         unsigned cc[4], rr[2];
 #pragma unroll
@@ -1629,13 +1636,17 @@ __global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int l
               if (r >= m || c > r) h[x][y][2 * e] = h[x][y][2 * e + 1] = 0.0;
             }
       }
-      // A Y: the sum runs over the columns
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) yb[y][q] = Y[(size_t)min(r0 + 16 * y + lk + 4 * q, m - 1) + (size_t)N * lr];
+      // A Y: the sum runs over the columns.  The wave that has its operands goes before one
+      // that still loads.
+      __builtin_amdgcn_s_setprio(2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
-        zc yv[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) yv[e] = Y[(size_t)min(c0 + 8 * x + 4 * e + lk, m - 1) + (size_t)N * lr];
+        const zc* yv = ya[x];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
 #pragma unroll
@@ -1657,9 +1668,7 @@ __global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int l
       for (int x = 0; x < 2; ++x) br[x] = bi[x] = d4{0, 0, 0, 0};
 #pragma unroll
       for (int y = 0; y < 2; ++y) {
-        zc yv[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) yv[q] = Y[(size_t)min(r0 + 16 * y + lk + 4 * q, m - 1) + (size_t)N * lr];
+        const zc* yv = yb[y];
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
 #pragma unroll
@@ -1681,6 +1690,7 @@ __global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int l
 #pragma unroll
         for (int q = 0; q < 4; ++q) red[wave][x][q][lane] = mkz(br[x][q], bi[x][q]);
       // the stores last: a later load's wait would wait for them too
+      __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (UPD) {
         __asm__ volatile("" : "+v"(l));
