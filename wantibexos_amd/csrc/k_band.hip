@@ -1086,8 +1086,9 @@ __host__ __device__ constexpr size_t qr_slots(int nwg_max) { return (size_t)(B +
 // scale conj(d_j)), the latter while the next column's sums are on their way; thread
 // (i, j sub) holds T(i, j).
 //
-// Bound by latency: about 4300 cycles a column, of which the exchange (store, first load
-// that sees it) takes about half.  The launch needs every workgroup resident, so it is used
+// Bound by latency: 60 us a panel of 16 columns, about 7100 cycles a column, of which the
+// exchange (store, first load that sees it) takes 2700 and the sums, the reflector and the
+// update of the rows the rest; the launches that it replaces took about 10 us a column.  The launch needs every workgroup resident, so it is used
 // for at most QP_WG of them: eight streams' launches fit at two workgroups per compute unit.
 template <int B>
 __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {

@@ -652,12 +652,12 @@ static void plan_drop_graph(wtb_bse_plan* p);
 //
 // By default (two_stage = -1) the COMPLEX*16 matrix takes the two-stage reduction at every
 // size that has a panel.  Whole plan, one-stage / two-stage with band 16, MI355X:
-//   N = 36: 1.11 / 0.77 ms   144: 3.14 / 1.93   576: 11.2 / 6.7   2116: 41.8 / 26.4
-//   5184: 161 / 82           8100: 445 / 186    14400: 2187 / 665
-// Band 16 while the panels run in one launch (band_panel_rows), where its shorter chase
-// outweighs the smaller updates (band 32 with that launch's kernels apart: 5.8 ms at
-// N = 256, 140 at 5184, 261 at 8100, 699 at 14400); band 32 above, where the MFMA updates
-// are most of the time.  The COMPLEX*8 matrix keeps the one-stage form below 8192, where
+//   N = 36: 1.00 / 0.70 ms   144: 2.95 / 1.82   576: 10.3 / 6.2   2116: 39.7 / 23.3
+//   5184: 160 / 74           8100: 445 / 162    14400: 2187 / 544
+// Band 16 while the panels run in one launch (band_panel_rows), where its shorter chase and
+// its pass over the trailing matrix outweigh the smaller updates (band 32 with the separate
+// kernels: 5.8 ms at N = 256 against 2.9, 142 at 5184, 261 at 8100, 703 at 14400); band 32
+// above, where the MFMA updates are most of the time.  The COMPLEX*8 matrix keeps the one-stage form below 8192, where
 // its GEMV chain reads half the bytes, and band 32 above.
 constexpr int kTwoStageMinN64 = 32, kTwoStageMinN = 8192;
 
