@@ -1086,8 +1086,8 @@ __host__ __device__ constexpr size_t qr_slots(int nwg_max) { return (size_t)(B +
 // scale conj(d_j)), the latter while the next column's sums are on their way; thread
 // (i, j sub) holds T(i, j).
 //
-// Bound by latency: 60 us a panel of 16 columns, about 7100 cycles a column, of which the
-// exchange (store, first load that sees it) takes 2700 and the sums, the reflector and the
+// Bound by latency: 54 us a panel of 16 columns (61 with more than 15 workgroups), about
+// 6400 cycles a column, of which the exchange (store, first load that sees it) takes 2700 and the sums, the reflector and the
 // update of the rows the rest; the launches that it replaces took about 10 us a column.  The launch needs every workgroup resident, so it is used
 // for at most QP_WG of them: eight streams' launches fit at two workgroups per compute unit.
 template <int B>
@@ -1144,9 +1144,8 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   };
   // value q of rounds c .. c + nr - 1 summed over the workgroups, and entry nwg of round c
   // (row c); all loads of a pass at once, repeated until every value is there (bounded)
-  auto gather = [&](auto nrc, int c, int nr, bool with_row, zc* tot, zc& rowv) {
-    constexpr int NR = decltype(nrc)::value, U = NR == 1 ? 4 : 2;
-    const int n = a.nwg + (with_row ? 1 : 0);
+  auto gather_u = [&](auto nrc, auto uc, int n, int c, int nr, bool with_row, zc* tot, zc& rowv) {
+    constexpr int NR = decltype(nrc)::value, U = decltype(uc)::value;
     zc s[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) s[r] = mkz(0, 0);
@@ -1188,6 +1187,13 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
 #pragma unroll
     for (int r = 0; r < NR; ++r)
       if (r < nr) tot[r] = sub_sum<SUB>(s[r]);
+  };
+  // one slot a thread where that covers them (with four loads a poll throughout, a panel took
+  // 60 us at N = 2116, with one 54)
+  auto gather = [&](auto nrc, int c, int nr, bool with_row, zc* tot, zc& rowv) {
+    const int n = a.nwg + (with_row ? 1 : 0);
+    if (n <= SUB) gather_u(nrc, std::integral_constant<int, 1>{}, n, c, nr, with_row, tot, rowv);
+    else gather_u(nrc, std::integral_constant<int, decltype(nrc)::value == 1 ? 4 : 2>{}, n, c, nr, with_row, tot, rowv);
   };
 
   zc T[NT], gcol[NT], taup = mkz(0, 0);
@@ -1344,8 +1350,9 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
 // W = X - 1/2 V (T^H (V^H X)) with X = A22 Y, in one launch: workgroup w takes rows 256 w ..,
 // its part of M = V^H X on FP64 MFMA (operands straight from memory in the MFMA's layout),
 // one exchange of the B x B parts as above (slots [workgroup][B B]), then Z = T^H M and its
-// rows of W.  Latency-bound (17 us at N = 5184); summing the K slices of X here too, on the
-// few workgroups of this launch, took 30 us against 17 + 5 with a launch of its own.
+// rows of W, whose V and X are loaded during the exchange (13.0 us without that, now 10.2
+// at N = 2116).  Latency-bound; summing the parts of X here too, on the few workgroups of this
+// launch, took 30 us against 17 + 5 with a launch of its own.
 struct QrWArgs {
   int m, N;
   const zc *V, *Tm;
@@ -1374,6 +1381,9 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
   const zc empty = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
 #pragma unroll
   for (int u = 0; u < NE; ++u) a.ex_next[(size_t)blockIdx.x * B * B + t + 256 * u] = empty;
+  zc tm[NE];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) tm[u] = a.Tm[t + 256 * u];
   // this wave's 64 rows of M = V^H X
   d4 mr[TI][TI], mi[TI][TI];
 #pragma unroll
@@ -1418,8 +1428,21 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
     st_buf(ex, (unsigned)((size_t)blockIdx.x * B * B + e) * (unsigned)sizeof(zc), 0,
            p);
   }
+  // while the sums are on their way: the rows of V and X that become W
+  zc vv[4][B / 4], xx[4][TI][4];
+#pragma unroll
+  for (int rt = 0; rt < 4; ++rt) {
+    const int rr = min(w0 + 16 * rt + lr, a.m - 1);
+#pragma unroll
+    for (int k = 0; k < B / 4; ++k) vv[rt][k] = a.V[rr + N * (4 * k + lk)];
+#pragma unroll
+    for (int x = 0; x < TI; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) xx[rt][x][r] = a.X[rr + N * (16 * x + lk + 4 * r)];
+  }
   lds_barrier();                               // red is read
-  for (int e = t; e < B * B; e += 256) Ts[e % B][e / B] = a.Tm[e];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) Ts[(t + 256 * u) % B][(t + 256 * u) / B] = tm[u];
 #pragma unroll
   for (int u = 0; u < NE; ++u) {
     const int e = t + 256 * u;
@@ -1463,6 +1486,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
   __syncthreads();
   // (V Z)^T by 16 x 16 tiles: MFMA rows over the columns of W, MFMA columns over its rows,
   // so that a lane's results lie next to its neighbours' in memory
+#pragma unroll
   for (int rt = 0; rt < 4; ++rt) {
     const int rr = w0 + 16 * rt + lr;
     d4 cr[TI], ci[TI];
@@ -1470,14 +1494,14 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
     for (int x = 0; x < TI; ++x) cr[x] = ci[x] = d4{0, 0, 0, 0};
 #pragma unroll
     for (int k0 = 0; k0 < B; k0 += 4) {
-      const zc vv = rr < a.m ? a.V[rr + N * (k0 + lk)] : mkz(0, 0);
+      const zc vk = vv[rt][k0 / 4];
 #pragma unroll
       for (int x = 0; x < TI; ++x) {
         const zc zz = Zs[k0 + lk][16 * x + lr];
-        cr[x] = mfma16x16x4(zz.re, vv.re, cr[x]);
-        ci[x] = mfma16x16x4(zz.re, vv.im, ci[x]);
-        cr[x] = mfma16x16x4(-zz.im, vv.im, cr[x]);
-        ci[x] = mfma16x16x4(zz.im, vv.re, ci[x]);
+        cr[x] = mfma16x16x4(zz.re, vk.re, cr[x]);
+        ci[x] = mfma16x16x4(zz.re, vk.im, ci[x]);
+        cr[x] = mfma16x16x4(-zz.im, vk.im, cr[x]);
+        ci[x] = mfma16x16x4(zz.im, vk.re, ci[x]);
       }
     }
     if (rr < a.m)
@@ -1486,7 +1510,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const size_t at = rr + N * (16 * x + lk + 4 * r);
-          const zc v = a.X[at];
+          const zc v = xx[rt][x][r];
           a.X[at] = mkz(v.re - 0.5 * cr[x][r], v.im - 0.5 * ci[x][r]);
         }
   }
