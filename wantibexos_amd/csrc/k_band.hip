@@ -1561,10 +1561,10 @@ __global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m
 // row blocks from K on); k_um_sum adds them in order.
 //
 // 256 m^2 flops over 16 m^2 bytes and 2 m^2 of parts: at m = 14400 0.73 ms of the matrix cores
-// and 0.73 ms of memory, and the kernel takes 1.11 ms (48 TFLOP/s, 3.8 TB/s with the operands
-// that miss the L2; the matrix cores are busy 65 % of the time).  Two kernels, a product over
+// and 0.73 ms of memory, and the kernel takes 1.15 ms (46 TFLOP/s, 3.7 TB/s with the operands
+// that miss the L2; the matrix cores are busy 63 % of the time).  Two kernels, a product over
 // 16 m^2 bytes and an update over 16 m^2, took 483 ms of a reduction at N = 14400 where this
-// one and k_um_sum take 373, and 27 ms of one at N = 5184 (19 here).  Y ahead of the products
+// one and k_um_sum take 377, and 29 ms of one at N = 5184 (22 here).  Y ahead of the products
 // that use it took 14 ms of that, their wave's priority 1 ms of a plan at N = 5184 (a higher
 // priority for the loads instead cost 68 ms at 14400).  64 x 64 tiles, three waves per SIMD
 // with spills, and an order of the tiles by XCD were no faster.

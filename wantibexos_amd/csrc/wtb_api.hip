@@ -652,11 +652,11 @@ static void plan_drop_graph(wtb_bse_plan* p);
 //
 // By default (two_stage = -1) the COMPLEX*16 matrix takes the two-stage reduction at every
 // size that has a panel.  Whole plan, one-stage / two-stage with band 16, MI355X:
-//   N = 36: 1.00 / 0.70 ms   144: 2.95 / 1.82   576: 10.3 / 6.2   2116: 39.7 / 23.3
-//   5184: 160 / 74           8100: 445 / 162    14400: 2187 / 544
+//   N = 36: 1.00 / 0.68 ms   144: 2.95 / 1.73   576: 10.3 / 5.8   2116: 39.7 / 22.1
+//   5184: 160 / 72           8100: 445 / 160    14400: 2187 / 540
 // Band 16 while the panels run in one launch (band_panel_rows), where its shorter chase and
 // its pass over the trailing matrix outweigh the smaller updates (band 32 with the separate
-// kernels: 5.8 ms at N = 256 against 2.9, 142 at 5184, 261 at 8100, 703 at 14400); band 32
+// kernels: 5.8 ms at N = 256 against 2.7, 142 at 5184, 261 at 8100, 703 at 14400); band 32
 // above, where the MFMA updates are most of the time.  The COMPLEX*8 matrix keeps the one-stage form below 8192, where
 // its GEMV chain reads half the bytes, and band 32 above.
 constexpr int kTwoStageMinN64 = 32, kTwoStageMinN = 8192;
@@ -1916,7 +1916,7 @@ int wtb_bse_batch_create(wtb_ctx* c, int n, const wtb_tb_model* models, const wt
     return rc;
   }
   // longest processing time first: the longest goes to the least loaded lane.  A plan takes
-  // about 11 us N + 1.3e-10 ms N^3 (6.2 ms at N = 576, 23 at 2116, 74 at 5184, 543 at 14400);
+  // about 11 us N + 1.3e-10 ms N^3 (5.8 ms at N = 576, 22 at 2116, 72 at 5184, 540 at 14400);
   // with N^3 alone eight models of N = 576 .. 2304 took 44 ms on four lanes, 38 with this
   std::vector<int> order(n);
   for (int i = 0; i < n; ++i) order[i] = i;
