@@ -255,7 +255,8 @@ int wtb_bse_plan_set_timing(wtb_bse_plan* plan, int on);
 int wtb_bse_plan_kernel_ms(const wtb_bse_plan* plan, double* total_ms, int* launches);
 /* With the two-stage reduction the timed kernel is instead the trailing update of the
  * dense -> band stage (one launch per panel); flops = their algorithmic flop count
- * (8 m^2 2k per launch: m trailing rows, k reflectors); 0 for the one-stage GEMV. */
+ * (about 8 m^2 k per launch: m trailing rows, k reflectors; where the launch also forms the
+ * next product, twice that); 0 for the one-stage GEMV. */
 int wtb_bse_plan_kernel_flops(const wtb_bse_plan* plan, double* flops);
 /* execute() captures the pipeline into a HIP graph on its first call and
  * replays it afterwards (default on); off launches the kernels directly.
