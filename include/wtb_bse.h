@@ -121,6 +121,11 @@ int wtb_version(void);
 void* wtb_stream(wtb_ctx* ctx);             /* the context's hipStream_t             */
 int wtb_sync(wtb_ctx* ctx);                 /* wait for all work on the context      */
 
+/* Workgroups of one launch wait for each other inside the two-stage reduction.  A wait gives
+ * up after this many polls (0, the default: about a second's worth), so that a reduction
+ * ends whatever else holds the device.  Plans take it over when they enqueue or capture. */
+int wtb_set_wait_limit(wtb_ctx* ctx, int polls);
+
 /* ---- single stages ---------------------------------------------------------- */
 
 /* monhkhorst_pack (subroutines/mhkpack_subs.f90:359-407, recvec :409-432):

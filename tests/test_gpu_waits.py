@@ -1,0 +1,51 @@
+"""GPU: the bounded waits between the workgroups of the two-stage reduction.  With a limit of
+one poll every wait gives up at once; a call may then fail with its error or give the right
+values, never wrong ones."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import ctx  # noqa: F401  (fixture)
+
+pytestmark = pytest.mark.gpu
+
+WTB_ERR_EIG = 8
+
+
+@pytest.fixture
+def hasty():
+    """a context whose waits give up after one poll"""
+    from wantibexos_amd import bse
+    with bse.Context(0) as c:
+        c.set_wait_limit(1)
+        yield c
+
+
+def case(n1, n2):
+    from wantibexos_amd import bse, tbmodel
+    m = tbmodel.hex2d(seed=9, nw=6, ngrid=(12, 12, 1))
+    return m, bse.BSEParams(ngrid=(n1, n2, 1), nc=2, nv=2, coultype="V2DRK", r0=40.0, cshift=0.05, ebse0=0.0,
+                            ebsef=6.0, numbse=101, dtfull=True, cpol=True, f154=False)
+
+
+# N = 4: the chase's only group of sweeps waits in LDS alone; 32: no panel at band 32; 144:
+# one workgroup a panel; 576: three
+@pytest.mark.parametrize("band", [16, 32])
+@pytest.mark.parametrize("grid", [(1, 1), (2, 4), (6, 6), (12, 12)])
+def test_stalled_plan_gives_no_wrong_values(ctx, hasty, grid, band):  # noqa: F811
+    from wantibexos_amd import bse
+    print(f"stalled plan {grid} band {band}", flush=True)
+    m, prm = case(*grid)
+    with bse.BSEPlan(ctx, m, prm) as plan:
+        plan.set_reduction(False)
+        plan.execute()
+        ref = plan.results()
+    with bse.BSEPlan(hasty, m, prm) as plan:
+        plan.set_reduction(True, band)
+        plan.execute()
+        try:
+            got = plan.results()
+        except bse.WTBError as e:
+            assert e.code == WTB_ERR_EIG
+            return
+    assert np.abs(got["W"] - ref["W"]).max() < 1e-12
+    assert np.abs(got["eps"] - ref["eps"]).max() <= 1e-9 * np.abs(ref["eps"]).max()

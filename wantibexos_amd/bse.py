@@ -91,6 +91,7 @@ def _load():
         "wtb_last_error": (C.c_char_p, []),
         "wtb_version": (ip, []),
         "wtb_stream": (vp, [vp]),
+        "wtb_set_wait_limit": (ip, [vp, ip]),
         "wtb_sync": (ip, [vp]),
         "wtb_monkhorst_pack": (ip, [vp, vp, vp, vp, vp]),
         "wtb_eigsys": (ip, [vp, vp, ip, vp, vp, vp, vp]),
@@ -276,6 +277,10 @@ class Context:
 
     def sync(self):
         _check(lib().wtb_sync(self.h))
+
+    def set_wait_limit(self, polls: int = 0):
+        """Polls after which a wait between the workgroups of a reduction gives up (0: default)."""
+        _check(lib().wtb_set_wait_limit(self.h, int(polls)))
 
 
 def monkhorst_pack(ctx: Context, ngrid, shift, rlat):

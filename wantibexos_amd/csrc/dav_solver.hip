@@ -96,6 +96,7 @@ struct SmallEig {
   double* Z = nullptr;   // mmax x mmax
   int* status = nullptr; // set when a reduction stalls
   int cus = 0;
+  int wait_limit = 0;
 };
 
 // room for either reduction of up to m rows
@@ -151,6 +152,7 @@ int small_heev(hipStream_t s, SmallEig& e, int m, const zc* G, int ldg, double* 
     BandWork bw;
     zc* tau = reinterpret_cast<zc*>(off + m);
     if ((rc = band_bind(bw, tau + band_tau_elems(m), m, 16, 0))) return rc;
+    bw.wait_limit = e.wait_limit;
     bw.tau1 = tau;
     bw.tau2 = tau + m;
     if ((rc = run_band_tridiag(s, bw, e.A, m, nullptr, d, off, e.status))) return rc;
@@ -285,6 +287,7 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
   double* lamS = work.lamS;
   SmallEig& se = work.se;
   SmallEig& sc = work.sc;
+  se.wait_limit = sc.wait_limit = cfg.wait_limit;
   auto cleanup = [&]() {};
 #define DAV_TRY(call)      \
   if ((rc = (call))) {     \

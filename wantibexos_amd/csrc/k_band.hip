@@ -35,8 +35,9 @@
 // order from a counter; task k of sweep s waits until sweep s - 1 has finished its tasks
 // 0..k+1 (its later tasks touch only rows below this task's), signalled through counters in
 // LDS inside a group and through a progress counter in memory between groups (device-scope
-// accesses, no cache maintenance).  Every wait is bounded: past the limit the kernel sets an
-// error flag that every waiting workgroup sees, and all of them return.
+// accesses, no cache maintenance).  Every wait is bounded, in memory and in LDS alike: past
+// the limit the kernel sets an error flag that every waiting workgroup sees, all of them
+// return, and what follows gets a zero tridiagonal and the status word.
 #include "wtb_kernels.h"
 
 namespace wtb {
@@ -1799,7 +1800,8 @@ struct ChaseArgs {
   int nrhs;
   int* prog;         // [group] tasks that the group's last sweep has finished
   int* ctl;          // [0] error flag, [32] next group to claim
-  long long spin_limit;
+  long long spin_limit;   // polls of a counter in memory
+  int lds_limit;          // polls of a counter in LDS
   zc* Vc;            // the reflectors kept (VEC): row r of sweep s at (N - 1 - r) + ld (N - 1 - s)
   int ld;
   zc* tau;           // [sweep][task], kt tasks
@@ -1914,13 +1916,21 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
   const __amdgpu_buffer_rsrc_t gb = dev_buffer(a.gc, (size_t)nrhs * N * sizeof(zc));
   for (int i = threadIdx.x; i < SW * R * C::SLOT; i += (SW + 1) * 64) (&slot[0][0][0])[i] = mkz(0, 0);
   if (threadIdx.x == 0) bad = 0;
+  // past a limit: the flags for this workgroup's waves (there before this one leaves) and
+  // for the other workgroups
+  auto give_up = [&]() {
+    lds_set(&bad, 1);
+    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
   // wait for *f >= need; seen keeps the last count read
   auto wait_lds = [&](int* f, int need, int& seen) {
     for (int n = 0; seen < need; ++n) {
       seen = lds_get(f);
       if (seen >= need) break;
-      if (lds_get(&bad) || n > (1 << 25)) {
-        bad = 1;
+      if (lds_get(&bad)) return false;
+      if (n > a.lds_limit) {
+        give_up();
         return false;
       }
     }
@@ -1928,6 +1938,9 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
   };
   for (;;) {
     __syncthreads();
+    // a wave that gave up has left (wave 0, which claims the groups, perhaps among them), so
+    // the others do not start another group
+    if (lds_get(&bad)) return;
     if (threadIdx.x == 0) group = atomicAdd(a.ctl + 32, 1);
     if ((int)threadIdx.x < SW) wrote[threadIdx.x] = read[threadIdx.x] = 0;
     __syncthreads();
@@ -1952,8 +1965,7 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
           if (have >= k + 1) break;
           if (n > a.spin_limit ||
               ((n & 63) == 63 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            lds_set(&bad, 1);
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            give_up();
             return;
           }
         }
@@ -2141,16 +2153,18 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
   }
 }
 
-// d, e of the tridiagonal from the band; g = conj(gc)
+// d, e of the tridiagonal from the band; g = conj(gc).  After a stalled wait the band is
+// unfinished and may hold anything: status is set and what follows works on zeros.
 __global__ void k_band_finish(const zc* __restrict__ BD, int N, int LB, double* __restrict__ d, double* __restrict__ e,
                               const zc* __restrict__ gc, zc* __restrict__ g, int nrhs, const int* __restrict__ err,
                               int* __restrict__ status) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j == 0 && status && (err[0] || err[8])) status[0] |= 1 << WTB_ERR_EIG;
+  const bool bad = err[0] || err[8];
+  if (j == 0 && status && bad) status[0] |= 1 << WTB_ERR_EIG;
   if (j >= N) return;
-  d[j] = BD[(size_t)j * LB].re;
-  e[j] = (j + 1 < N) ? BD[(size_t)j * LB + 1].re : 0.0;
-  for (int r = 0; r < nrhs; ++r) g[(size_t)r * N + j] = conj(gc[(size_t)r * N + j]);
+  d[j] = bad ? 0.0 : BD[(size_t)j * LB].re;
+  e[j] = (!bad && j + 1 < N) ? BD[(size_t)j * LB + 1].re : 0.0;
+  for (int r = 0; r < nrhs; ++r) g[(size_t)r * N + j] = bad ? mkz(0, 0) : conj(gc[(size_t)r * N + j]);
 }
 
 // control block of the chase: its error flag and sweep counter 0 (the panel's flag, [8],
@@ -2411,6 +2425,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   // streams run, so that the results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
   // its stored matrix amplifies.
   const bool qr = std::is_same<T, zc>::value && B == 16 && w.panel_wg >= (N - b + PR - 1) / PR;
+  const int spin = w.wait_limit > 0 ? w.wait_limit : 1 << 20;
   if (qr)
     hipLaunchKernelGGL(k_fill_empty, dim3((unsigned)((2 * exn + 255) / 256)), dim3(256), 0, s, w.ex, 2 * exn);
   for (int p = 0;; ++p) {
@@ -2443,7 +2458,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
         zc* A22 = H + r0 + (size_t)ld * r0;
         if (p > 0)
           hipLaunchKernelGGL((k_strip<B>), dim3((m + B + 63) / 64), blk, 0, s, H + c0 + (size_t)ld * c0, ld, m + B, N, Vo, Xo);
-        QrPanelArgs q{H, ld, N, c0, r0, m, k, V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, 1 << 20,
+        QrPanelArgs q{H, ld, N, c0, r0, m, k, V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, spin,
                       w.tau1 ? w.tau1 + c0 : nullptr};
         hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, q);
         const int n = um_steps(m), nt = (m + UM_R - 1) / UM_R;
@@ -2459,7 +2474,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
         }
         const size_t tot = (size_t)m * B;
         hipLaunchKernelGGL(k_um_sum<B>, dim3((unsigned)((tot + 255) / 256)), blk, 0, s, m, n, nt, w.hb, X, N);
-        QrWArgs x{m, N, V, w.T, X, ex + wo, exo + wo, a.nwg, w.err + 8, 1 << 20};
+        QrWArgs x{m, N, V, w.T, X, ex + wo, exo + wo, a.nwg, w.err + 8, spin};
         hipLaunchKernelGGL((k_qr_w<B>), g, blk, 0, s, x);
         // the last panel's update, which no further product waits for
         if (m - B <= 0 || min(b, m - B - 1) <= 0) {
@@ -2470,7 +2485,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
       }
     if (w.panel_resident > 0 && a.nwg <= w.panel_resident) {
       hipLaunchKernelGGL((k_panel<T, B>), g, blk, 0, s, a, w.V, w.bar + (size_t)p * (BMAX + 1), w.err + 8,
-                         (long long)1 << 20);
+                         (long long)spin);
     } else {
       for (int c = 0; c <= k; ++c) hipLaunchKernelGGL((k_pqr_col<T, B>), g, blk, 0, s, a, c);
       hipLaunchKernelGGL((k_pfin<T, B>), g, blk, 0, s, a, w.V);
@@ -2523,7 +2538,9 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
   ca.nrhs = nrhs;
   ca.prog = w.prog;
   ca.ctl = w.err;
-  ca.spin_limit = 1ll << 21;   // polls of about half a microsecond each: about a second
+  // polls of about half a microsecond each: about a second; in LDS about two seconds
+  ca.spin_limit = w.wait_limit > 0 ? w.wait_limit : 1 << 21;
+  ca.lds_limit = w.wait_limit > 0 ? w.wait_limit : 1 << 25;
   // groups of sweeps that can be at work at once: each follows the one before by more than
   // two tasks a sweep
   const int sw = (b == 16) ? ChaseDim<16>::SW : ChaseDim<32>::SW;

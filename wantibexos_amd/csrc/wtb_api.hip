@@ -106,6 +106,7 @@ using namespace wtb;
 struct wtb_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
+  int wait_limit = 0;            // BandWork::wait_limit of its reductions
 };
 
 static int plan_default_band(bool mixed, int N);
@@ -255,6 +256,15 @@ int wtb_destroy(wtb_ctx* c) {
 }
 
 void* wtb_stream(wtb_ctx* c) { return c ? (void*)c->stream : nullptr; }
+
+int wtb_set_wait_limit(wtb_ctx* c, int polls) {
+  if (!c || polls < 0) {
+    set_error("wtb_set_wait_limit: needs a context and polls >= 0");
+    return WTB_ERR_ARG;
+  }
+  c->wait_limit = polls;
+  return WTB_OK;
+}
 
 int wtb_sync(wtb_ctx* c) {
   if (!c) return WTB_ERR_ARG;
@@ -674,6 +684,7 @@ static int plan_reduce(wtb_bse_plan* p, zc* g, int* status) {
   if (plan_two_stage(p)) {
     p->bw.kev = p->kernel_timing ? p->kev.data() : nullptr;
     p->bw.kev_cap = p->kernel_timing ? p->N : 0;
+    p->bw.wait_limit = p->ctx->wait_limit;
     // the band reduction reads and updates the lower triangle only
     if (p->mixed) return run_band_tridiag_f32(s, p->bw, p->Hf, (int)p->ldh, g, p->tw.d, p->tw.e, status);
     return run_band_tridiag(s, p->bw, p->H, (int)p->ldh, g, p->tw.d, p->tw.e, status);
@@ -1109,6 +1120,7 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
         bw.tau2 = bw.tau1 + n;
       }
       bw.panel_resident = cus;
+      bw.wait_limit = c->wait_limit;
     } else {
       tridiag_bind(tw, tri, n, 32, 0);
       tw.store_v = vec;
@@ -1646,6 +1658,7 @@ int wtb_bse_plan_lowest(wtb_bse_plan* p, const wtb_davidson_params* dp, const wt
     cfg.max_iter = dp->max_iter;
     cfg.tol = dp->tol;
     cfg.coarse = dp->coarse;
+    cfg.wait_limit = p->ctx->wait_limit;
     MlpDev md;
     if (mlp) {
       md.w = mlp->P;

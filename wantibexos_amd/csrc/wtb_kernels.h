@@ -145,6 +145,7 @@ struct BandWork {
   int* err = nullptr;           // [0] the chase's error flag, [8] the panel's, [32] next sweep
   int* bar = nullptr;           // per panel and column: workgroups past the column
   int panel_resident = 0;       // one-launch panels up to this many workgroups (0: per column)
+  int wait_limit = 0;           // polls after which a wait inside a kernel gives up (0: the default)
   int panel_wg = 0;             // COMPLEX*16: panel and W in one launch each up to this many workgroups
   zc* ex = nullptr;             // their exchange slots, two panel parities
   zc *V2 = nullptr, *X2 = nullptr;   // every other panel's V and W
@@ -297,6 +298,7 @@ struct DavidsonCfg {
   // energy, whose block of H is inverted exactly (0: diagonal preconditioner only)
   int coarse = 0;
   double coarse_dmin = 1e-2;
+  int wait_limit = 0;     // of the small solves' reductions (BandWork)
 };
 struct DavidsonInfo {
   int iters = 0, matvecs = 0, converged = 0;
