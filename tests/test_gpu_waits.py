@@ -49,3 +49,20 @@ def test_stalled_plan_gives_no_wrong_values(ctx, hasty, grid, band):  # noqa: F8
             return
     assert np.abs(got["W"] - ref["W"]).max() < 1e-12
     assert np.abs(got["eps"] - ref["eps"]).max() <= 1e-9 * np.abs(ref["eps"]).max()
+
+
+def test_lowest_after_a_stalled_call(ctx):  # noqa: F811
+    """the solver's buffers live on in the plan; a stall of one call is not the next one's"""
+    from wantibexos_amd import bse
+    m, prm = case(12, 12)
+    prm.precision = bse.MIXED
+    with bse.BSEPlan(ctx, m, prm) as plan:
+        ref = plan.lowest(nev=16, tol=1e-8)["W"]
+    with bse.Context(0) as c, bse.BSEPlan(c, m, prm) as plan:
+        c.set_wait_limit(1)
+        try:
+            assert np.abs(plan.lowest(nev=16, tol=1e-8)["W"] - ref).max() < 1e-12
+        except bse.WTBError as e:
+            assert e.code == WTB_ERR_EIG
+        c.set_wait_limit(0)
+        assert np.abs(plan.lowest(nev=16, tol=1e-8)["W"] - ref).max() < 1e-12

@@ -84,6 +84,8 @@ __global__ void k_scatter_rows(int M, int nq, const int* rows, const zc* Z, zc* 
   T[(size_t)rows[i] + (size_t)ldt * q] = Z[(size_t)i + (size_t)M * q];
 }
 
+__global__ void k_clear_status(int* st) { *st = 0; }
+
 namespace {
 
 struct SmallEig {
@@ -94,7 +96,7 @@ struct SmallEig {
   void* btw = nullptr;
   double* lam = nullptr;
   double* Z = nullptr;   // mmax x mmax
-  int* status = nullptr; // set when a reduction stalls
+  int* status = nullptr; // set when a reduction stalls, cleared at the start of each solve
   int cus = 0;
   int wait_limit = 0;
 };
@@ -116,8 +118,7 @@ int small_alloc(SmallEig& e, int mmax, int kmax) {
   WTB_HIP(hipMalloc(&e.lam, sizeof(double) * mmax));
   WTB_HIP(hipMalloc(&e.Z, sizeof(double) * (size_t)mmax * mmax));
   WTB_HIP(hipMalloc(&e.status, sizeof(int)));
-  int dev = 0, none = 0;
-  WTB_HIP(hipMemcpy(e.status, &none, sizeof(int), hipMemcpyHostToDevice));
+  int dev = 0;
   WTB_HIP(hipGetDevice(&dev));
   WTB_HIP(hipDeviceGetAttribute(&e.cus, hipDeviceAttributeMultiprocessorCount, dev));
   return WTB_OK;
@@ -288,6 +289,8 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
   SmallEig& se = work.se;
   SmallEig& sc = work.sc;
   se.wait_limit = sc.wait_limit = cfg.wait_limit;
+  for (SmallEig* e : {&se, &sc})   // the buffers outlive a call; a stall of the last one's does not
+    if (e->status) hipLaunchKernelGGL(k_clear_status, dim3(1), dim3(1), 0, s, e->status);
   auto cleanup = [&]() {};
 #define DAV_TRY(call)      \
   if ((rc = (call))) {     \
