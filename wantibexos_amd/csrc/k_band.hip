@@ -2562,10 +2562,12 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
 
 // two columns of X fit the LDS of a compute unit
 int band_vec_rows() { return 160 * 1024 / (2 * (int)sizeof(zc)); }
-// Whether a solve with m eigenvectors takes the two-stage reduction (COMPLEX*16).  It saves
-// 8 to 16 us a column of the one-stage form and pays N^2 m for the chase's reflectors.
-// zheev with all vectors, two-stage / one-stage: N = 256 4.4 / 6.4 ms, 640 8.5 / 13.7, 1290 21
-// / 29, 2049 45 / 52, 2500 62 / 69, 3000 86 / 91: the line lies where N m is 3000^2.
+// Whether a solve with m eigenvectors that are corrected afterwards (the iterative solver's
+// small solves; its residuals are formed from the vectors) takes the two-stage reduction
+// (COMPLEX*16).  It saves 8 to 16 us a column of the one-stage form and pays N^2 m for the
+// chase's reflectors.  All vectors, two-stage / one-stage: N = 256 4.4 / 6.4 ms, 640 8.5 /
+// 13.7, 1290 21 / 29, 2049 45 / 52, 2500 62 / 69, 3000 86 / 91: the line lies where N m is
+// 3000^2.  wtb_zheev, whose vectors are the result, keeps the one-stage form's smaller error.
 bool band_vec_two_stage(int N, int m) {
   return N >= 32 && N <= band_vec_rows() && (double)N * m <= 9e6;
 }
