@@ -994,8 +994,9 @@ __device__ inline zc fnma_zc(zc a, zc b, zc c) {         // c - a conj(b)
 }
 
 // ZLARFG as above for latency chains: beta from one reciprocal square root
-// (two Newton steps, then a correction of the root), 1/(alpha - beta) from one reciprocal;
-// where squares near the range's ends would not do, as above
+// (two Newton steps, then a correction of the root), 1/(alpha - beta) from one reciprocal, each
+// quotient corrected by its remainder to the rounding of a division; where squares near the
+// range's ends would not do, as above
 __device__ inline void larfg_fast(zc alpha, double xn2, zc& beta, zc& tau, zc& scale) {
   const bool ident = xn2 == 0.0 && alpha.im == 0.0;
   const double n2 = ident ? 1.0 : alpha.re * alpha.re + alpha.im * alpha.im + xn2;
@@ -1016,9 +1017,13 @@ __device__ inline void larfg_fast(zc alpha, double xn2, zc& beta, zc& tau, zc& s
   double rd = __builtin_amdgcn_rcp(den);
   rd = fma(rd, fma(-den, rd, 1.0), rd);
   rd = fma(rd, fma(-den, rd, 1.0), rd);
+  auto quot = [](double x, double d, double r) {   // x / d with r about 1 / d
+    const double q = x * r;
+    return fma(fma(-d, q, x), r, q);
+  };
   beta = ident ? alpha : mkz(b, 0.0);
-  tau = ident ? mkz(0, 0) : mkz(-dr * rb, -alpha.im * rb);
-  scale = ident ? mkz(0, 0) : mkz(dr * rd, -alpha.im * rd);
+  tau = ident ? mkz(0, 0) : mkz(quot(-dr, b, rb), quot(-alpha.im, b, rb));
+  scale = ident ? mkz(0, 0) : mkz(quot(dr, den, rd), quot(-alpha.im, den, rd));
 }
 
 // One element by a buffer load or store that the caches of other XCDs see (sc1), 16 bytes at
