@@ -66,3 +66,71 @@ def test_lowest_after_a_stalled_call(ctx):  # noqa: F811
             assert e.code == WTB_ERR_EIG
         c.set_wait_limit(0)
         assert np.abs(plan.lowest(nev=16, tol=1e-8)["W"] - ref).max() < 1e-12
+
+
+# N = 36, 576: with any wait given up the one-stage form gives the values, to the bit
+@pytest.mark.parametrize("grid", [(3, 3), (12, 12)])
+def test_stalled_plan_is_solved_by_the_one_stage_form(ctx, hasty, grid):  # noqa: F811
+    from wantibexos_amd import bse
+    m, prm = case(*grid)
+    with bse.BSEPlan(ctx, m, prm) as plan:
+        plan.set_reduction(False)
+        plan.execute()
+        ref = plan.results()
+    with bse.BSEPlan(hasty, m, prm) as plan:
+        for _ in range(2):
+            plan.execute()
+            got = plan.results()
+            for k in ("W", "act", "eps"):
+                assert np.array_equal(got[k], ref[k]), k
+    with bse.BSEBatch(hasty, [m, m], [prm, prm], lanes=2) as batch:
+        batch.execute()
+        for i in range(2):
+            got = batch.results(i)
+            for k in ("W", "act", "eps"):
+                assert np.array_equal(got[k], ref[k]), k
+
+
+@pytest.mark.parametrize("n", [40, 300])
+def test_stalled_zheev_is_solved(hasty, n):
+    from wantibexos_amd import bse
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    a = a + a.conj().T
+    w = bse.zheev(hasty, np.triu(a))
+    assert np.linalg.norm(w - np.linalg.eigvalsh(a)) <= 8 * n * np.finfo(float).eps * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("lanes", [1, 3])
+def test_stalled_bands_are_solved(ctx, hasty, lanes):  # noqa: F811
+    from wantibexos_amd import bse
+    m, prm = case(6, 6)
+    q = np.array([[0.0, 0.0, 0.0, 0.0], [0.1, 0.05, 0.0, 0.0], [0.2, 0.1, 0.02, 0.0], [0.3, 0.1, 0.1, 0.0]])
+    with bse.BSEBands(ctx, m, prm, lanes=lanes) as b:
+        ref = b.run(q)
+    with bse.BSEBands(hasty, m, prm, lanes=lanes) as b:
+        got = b.run(q)
+    assert np.abs(got - ref).max() < 1e-12
+
+
+def test_stalled_lowest_is_solved(ctx, hasty):  # noqa: F811
+    from wantibexos_amd import bse
+    m, prm = case(12, 12)
+    prm.precision = bse.MIXED
+    with bse.BSEPlan(ctx, m, prm) as plan:
+        ref = plan.lowest(nev=16, tol=1e-8)["W"]
+    with bse.BSEPlan(hasty, m, prm) as plan:
+        assert np.abs(plan.lowest(nev=16, tol=1e-8)["W"] - ref).max() < 1e-12
+
+
+def test_the_launches_of_eight_streams(ctx):  # noqa: F811
+    """eight lanes at once, panels of one and of three workgroups"""
+    from wantibexos_amd import bse
+    for grid in ((6, 6), (12, 12)):
+        m, prm = case(*grid)
+        q = np.stack([np.linspace(0.0, 0.5, 16)] * 2 + [np.linspace(0.0, 0.2, 16), np.zeros(16)], axis=1)
+        with bse.BSEBands(ctx, m, prm, lanes=1) as b:
+            ref = b.run(q)
+        with bse.BSEBands(ctx, m, prm, lanes=8) as b:
+            for _ in range(3):
+                assert np.array_equal(b.run(q), ref), grid

@@ -97,6 +97,7 @@ struct SmallEig {
   double* lam = nullptr;
   double* Z = nullptr;   // mmax x mmax
   int* status = nullptr; // set when a reduction stalls, cleared at the start of each solve
+  bool one = false;      // the one-stage form only
   int cus = 0;
   int wait_limit = 0;
 };
@@ -134,8 +135,9 @@ void small_free(SmallEig& e) {
   hipFree(e.status);
 }
 
-int small_status(int st) {
+int small_status(int st, bool* stalled) {
   if (!st) return WTB_OK;
+  *stalled = true;
   set_error("davidson: a small eigensolve stalled");
   return WTB_ERR_EIG;
 }
@@ -148,7 +150,7 @@ int small_heev(hipStream_t s, SmallEig& e, int m, const zc* G, int ldg, double* 
   DCTree tree;
   int rc = dc_prepare(e.dcw, m, 0, tree, 1);
   if (rc) return rc;
-  if (band_vec_two_stage(m, k)) {
+  if (!e.one && band_vec_two_stage(m, k)) {
     double *d = static_cast<double*>(e.tri), *off = d + m;
     BandWork bw;
     zc* tau = reinterpret_cast<zc*>(off + m);
@@ -259,9 +261,10 @@ void davidson_work_delete(DavidsonWork* w) {
   delete w;
 }
 
-int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, const float* stats,
-                 const DavidsonCfg& cfg, const MlpDev* mlp, double* d_W, double* d_resid, zc* d_X,
-                 DavidsonInfo& info, DavidsonWork& work) {
+// one: the small solves by the one-stage reduction; stalled: one of them waited in vain
+static int davidson_solve(hipStream_t s, int N, const zf* H, int ldh, const double* D, const float* stats,
+                          const DavidsonCfg& cfg, const MlpDev* mlp, double* d_W, double* d_resid, zc* d_X,
+                          DavidsonInfo& info, DavidsonWork& work, bool one_stage, bool* stalled) {
   const int nev = cfg.nev;
   const int nk = std::min(N, nev + cfg.guard);
   const int msub = std::min(N, std::max(cfg.max_sub, 2 * nk));
@@ -289,6 +292,7 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
   SmallEig& se = work.se;
   SmallEig& sc = work.sc;
   se.wait_limit = sc.wait_limit = cfg.wait_limit;
+  se.one = sc.one = one_stage;
   for (SmallEig* e : {&se, &sc})   // the buffers outlive a call; a stall of the last one's does not
     if (e->status) hipLaunchKernelGGL(k_clear_status, dim3(1), dim3(1), 0, s, e->status);
   auto cleanup = [&]() {};
@@ -321,7 +325,7 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
       DAV_TRY(small_heev(s, sc, M, CS, M, lamS, QS, M, M));
       DAV_TRY(hipMemcpyAsync(&h_st, sc.status, sizeof(int), hipMemcpyDeviceToHost, s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
       DAV_TRY(hipStreamSynchronize(s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
-      DAV_TRY(small_status(h_st));
+      DAV_TRY(small_status(h_st, stalled));
     }
     order.resize(nk);
     DAV_TRY(hipMemcpy(idx, order.data(), sizeof(int) * nk, hipMemcpyHostToDevice) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
@@ -354,7 +358,7 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
     DAV_TRY(hipMemcpyAsync(h_rn.data(), rn, sizeof(double) * nk, hipMemcpyDeviceToHost, s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
     DAV_TRY(hipMemcpyAsync(&h_st, se.status, sizeof(int), hipMemcpyDeviceToHost, s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
     DAV_TRY(hipStreamSynchronize(s) == hipSuccess ? WTB_OK : WTB_ERR_HIP);
-    DAV_TRY(small_status(h_st));
+    DAV_TRY(small_status(h_st, stalled));
     double mx = 0.0;
     for (int c = 0; c < nev; ++c) mx = std::max(mx, h_rn[c]);
     info.max_resid = mx;
@@ -461,6 +465,16 @@ int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, co
 #undef DAV_TRY
   cleanup();
   return WTB_OK;
+}
+
+int run_davidson(hipStream_t s, int N, const zf* H, int ldh, const double* D, const float* stats,
+                 const DavidsonCfg& cfg, const MlpDev* mlp, double* d_W, double* d_resid, zc* d_X,
+                 DavidsonInfo& info, DavidsonWork& work) {
+  bool stalled = false;
+  int rc = davidson_solve(s, N, H, ldh, D, stats, cfg, mlp, d_W, d_resid, d_X, info, work, false, &stalled);
+  if (rc && stalled)
+    rc = davidson_solve(s, N, H, ldh, D, stats, cfg, mlp, d_W, d_resid, d_X, info, work, true, &stalled);
+  return rc;
 }
 
 }  // namespace wtb

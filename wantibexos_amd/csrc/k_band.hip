@@ -20,7 +20,7 @@
 //   k_gram, k_gram_sum         M = V^H X
 //   k_pW                       W = X - 1/2 V (T^H M)
 //   k_her2k_full               A22 -= V W^H + W V^H (MFMA, the tiles on and below the diagonal)
-// COMPLEX*16 with b = 16 (up to band_panel_rows() rows) has its own form of the same steps:
+// COMPLEX*16 with b = 16 (band_panel_fits) has its own form of the same steps:
 //   k_strip                    the panel's columns take the update of the panel before
 //   k_qr_panel                 reflectors, T, Y = V T and the tracked vectors, in one launch
 //   k_update_mul, k_um_sum     A22 takes the update of the panel before; X = A22 Y in that pass
@@ -39,6 +39,8 @@
 // the limit the kernel sets an error flag that every waiting workgroup sees, all of them
 // return, and what follows gets a zero tridiagonal and the status word.
 #include "wtb_kernels.h"
+#include <algorithm>
+#include <atomic>
 
 namespace wtb {
 
@@ -1094,8 +1096,8 @@ __host__ __device__ constexpr size_t qr_slots(int nwg_max) { return (size_t)(B +
 //
 // Bound by latency: 54 us a panel of 16 columns (61 with more than 15 workgroups), about
 // 6400 cycles a column, of which the exchange (store, first load that sees it) takes 2700 and the sums, the reflector and the
-// update of the rows the rest; the launches that it replaces took about 10 us a column.  The launch needs every workgroup resident, so it is used
-// for at most QP_WG of them: eight streams' launches fit at two workgroups per compute unit.
+// update of the rows the rest; the launches that it replaces took about 10 us a column.  The
+// launch needs every workgroup resident: band_panel_wg.
 template <int B>
 __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   constexpr int SUB = 256 / B;                 // threads per exchanged value
@@ -2165,7 +2167,7 @@ __global__ void k_band_finish(const zc* __restrict__ BD, int N, int LB, double* 
                               int* __restrict__ status) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   const bool bad = err[0] || err[8];
-  if (j == 0 && status && bad) status[0] |= 1 << WTB_ERR_EIG;
+  if (j == 0 && status && bad) status[0] |= 1 << WTB_ERR_EIG | kStalled;
   if (j >= N) return;
   d[j] = bad ? 0.0 : BD[(size_t)j * LB].re;
   e[j] = (!bad && j + 1 < N) ? BD[(size_t)j * LB + 1].re : 0.0;
@@ -2291,6 +2293,30 @@ static size_t qr_ex_elems(int nwg_max) {
 
 int band_panel_rows() { return QP_WG * PR + 16; }
 
+// Most workgroups of a panel's launch on the current device: an eighth of those resident at
+// once, so that the launches of eight streams (a set's lanes, or several threads' plans; a
+// process has four hardware queues by default) all get theirs, and at most QP_WG.  256
+// compute units hold two of these workgroups each: 64.  A chase beside them takes the LDS of
+// one of the two from up to 176 units, but ends by itself.  More launches than that at once,
+// or another process's, can keep each other waiting; then a wait ends at its limit and the
+// caller solves by the one-stage form (kStalled).
+static int band_panel_wg() {
+  static std::atomic<int> known[64];           // + 1; 0: not looked up yet
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (const int k = known[dev].load(std::memory_order_relaxed)) return k - 1;
+  int cus = 0, a = 0, b = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_qr_panel<16>, 256, 0) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_qr_w<16>, 256, 0) != hipSuccess)
+    return 0;
+  const int n = std::min(QP_WG, cus * std::min(a, b) / 8);
+  known[dev].store(n + 1, std::memory_order_relaxed);
+  return n;
+}
+
+bool band_panel_fits(int N) { return N <= band_panel_rows() && (N - 16 + PR - 1) / PR <= band_panel_wg(); }
+
 // steps of k_update_mul: fewer parts with more steps, more workgroups with fewer (at these
 // sizes about 1200 workgroups either way, 512 run at once; lines at half and one and a half
 // times these sizes measured within 1 %)
@@ -2375,7 +2401,7 @@ int band_bind(BandWork& w, void* base, int N, int b, int nrhs) {
   w.err = (int*)take(sizeof(int) * 64);
   w.bar = (int*)take(sizeof(int) * ((size_t)N / b + 2) * (BMAX + 1));
   w.ex = (zc*)take(sizeof(zc) * 2 * qr_ex_elems<BMAX>((int)std::min<size_t>(nwg, QP_WG)));
-  w.panel_wg = QP_WG;
+  w.panel_wg = band_panel_wg();
   return WTB_OK;
 }
 
@@ -2424,7 +2450,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   const int N = w.N, b = B;
   const int exw = min(w.nwg_max, QP_WG);               // workgroups that the slots hold
   const size_t exn = qr_ex_elems<B>(exw);
-  // COMPLEX*16 panels of at most QP_WG workgroups: one launch for the panel and one for W
+  // COMPLEX*16 panels of at most panel_wg workgroups: one launch for the panel and one for W
   // (5 launches a panel, one of them a pass over the trailing matrix that updates it for the
   // panel before and multiplies it with this one's Y).  The limit does not depend on how many
   // streams run, so that the results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
@@ -2518,7 +2544,7 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
   if (nrhs > 6) return WTB_ERR_LIMIT;
   if (w.tau1) {
     // the kept reflectors are those of the one-launch panels of the COMPLEX*16 matrix
-    if (!std::is_same<T, zc>::value || b != 16 || N > band_vec_rows()) return WTB_ERR_LIMIT;
+    if (!std::is_same<T, zc>::value || b != 16 || N > band_vec_rows() || !band_panel_fits(N)) return WTB_ERR_LIMIT;
     hipLaunchKernelGGL(k_zero_ints, dim3((4 * N + 255) / 256), dim3(256), 0, s, (int*)w.tau1, 4 * N);
   }
   if (nrhs > 0)
@@ -2574,7 +2600,7 @@ int band_vec_rows() { return 160 * 1024 / (2 * (int)sizeof(zc)); }
 // 13.7, 1290 21 / 29, 2049 45 / 52, 2500 62 / 69, 3000 86 / 91: the line lies where N m is
 // 3000^2.  wtb_zheev, whose vectors are the result, keeps the one-stage form's smaller error.
 bool band_vec_two_stage(int N, int m) {
-  return N >= 32 && N <= band_vec_rows() && (double)N * m <= 9e6;
+  return N >= 32 && N <= band_vec_rows() && (double)N * m <= 9e6 && band_panel_fits(N);
 }
 size_t band_tau_elems(int N) { return (size_t)N + (size_t)N * (N / 16 + 1); }
 

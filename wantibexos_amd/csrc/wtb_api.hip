@@ -48,6 +48,8 @@ static int status_to_code(int st) {
   if (st & (1 << WTB_ERR_EIG)) return WTB_ERR_EIG;
   return WTB_OK;
 }
+// a stalled reduction with nothing else wrong: worth solving again by the one-stage form
+static bool solve_stalled(int st) { return (st & kStalled) && status_to_code(st) == WTB_ERR_EIG; }
 static const char* status_text(int code) {
   switch (code) {
     case WTB_ERR_NOCP: return "no band above the Fermi level at some k (nocp undefined)";
@@ -178,6 +180,7 @@ struct wtb_bse_plan {
   int band_b = 32;             // its band width (plan_default_band unless set)
   BandWork bw;
   void* bandwork = nullptr;
+  bool redo = false;           // solving again by the one-stage form (plan_redo)
   int nref = 0;
   zc* Xr = nullptr;
   zc* HXr = nullptr;
@@ -604,8 +607,9 @@ static int plan_create_impl(wtb_ctx* c, const wtb_tb_model* m, const wtb_bse_par
     delete p;
     return rc;
   }
-  // one-launch panels need every workgroup resident: at most one per compute unit of a
-  // device the plan does not share (a batch sets 0: per-column launches)
+  // one-launch panels need every workgroup resident.  k_panel (COMPLEX*8, band 32): at most
+  // one per compute unit of a device the plan does not share (a set's lanes take per-column
+  // launches: 0); k_qr_panel (COMPLEX*16, band 16) goes by band_panel_fits on any stream
   {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 0;
@@ -664,17 +668,17 @@ static void plan_drop_graph(wtb_bse_plan* p);
 // size that has a panel.  Whole plan, one-stage / two-stage with band 16, MI355X:
 //   N = 36: 1.00 / 0.68 ms   144: 2.95 / 1.73   576: 10.3 / 5.8   2116: 39.7 / 22.1
 //   5184: 160 / 72           8100: 445 / 160    14400: 2187 / 540
-// Band 16 while the panels run in one launch (band_panel_rows), where its shorter chase and
+// Band 16 while the panels run in one launch (band_panel_fits), where its shorter chase and
 // its pass over the trailing matrix outweigh the smaller updates (band 32 with the separate
 // kernels: 5.8 ms at N = 256 against 2.7, 142 at 5184, 261 at 8100, 703 at 14400); band 32
 // above, where the MFMA updates are most of the time.  The COMPLEX*8 matrix keeps the one-stage form below 8192, where
 // its GEMV chain reads half the bytes, and band 32 above.
 constexpr int kTwoStageMinN64 = 32, kTwoStageMinN = 8192;
 
-static int plan_default_band(bool mixed, int N) { return !mixed && N <= band_panel_rows() ? 16 : 32; }
+static int plan_default_band(bool mixed, int N) { return !mixed && band_panel_fits(N) ? 16 : 32; }
 
 static bool plan_two_stage(const wtb_bse_plan* p) {
-  if (p->wf_count > 0 || (p->mixed && p->nref > 0) || !p->bandwork) return false;   // the reflectors are needed
+  if (p->redo || p->wf_count > 0 || (p->mixed && p->nref > 0) || !p->bandwork) return false;   // the reflectors are needed
   if (p->two_stage >= 0) return p->two_stage == 1;
   return p->N >= (!p->mixed && p->band_b == 16 ? kTwoStageMinN64 : kTwoStageMinN);
 }
@@ -933,6 +937,20 @@ int wtb_bse_plan_execute(wtb_bse_plan* p) {
   return WTB_OK;
 }
 
+// The plan's solve once more after one whose reduction stalled (kStalled: something else held
+// the device while its workgroups waited for each other), by the one-stage form and without
+// the graph; done when it returns.
+static int plan_redo(wtb_bse_plan* p) {
+  p->redo = true;
+  int rc = plan_enqueue(p);
+  p->redo = false;
+  if (hipStreamSynchronize(p->stream) != hipSuccess && !rc) {
+    set_error("one-stage solve after a stalled reduction: HIP error");
+    rc = WTB_ERR_HIP;
+  }
+  return rc;
+}
+
 int wtb_bse_plan_set_graph(wtb_bse_plan* p, int on) {
   if (!p) return WTB_ERR_ARG;
   p->use_graph = on != 0;
@@ -952,17 +970,10 @@ int wtb_bse_plan_build(wtb_bse_plan* p) {
   return WTB_OK;
 }
 
-int wtb_bse_plan_results(wtb_bse_plan* p, double* w, double* act, double* eps, double* egap) {
-  if (!p) {
-    set_error("wtb_bse_plan_results: null plan");
-    return WTB_ERR_ARG;
-  }
+// waits for the plan's solve and copies its results; status: the plan's status bits
+static int plan_read(wtb_bse_plan* p, double* w, double* act, double* eps, double* egap, int* status) {
   hipStream_t s = p->ctx->stream;
   const int N = p->N;
-  if (p->qmode && (act || eps || egap)) {
-    set_error("wtb_bse_plan_results: a finite-Q plan gives the exciton energies only (act, eps, egap NULL)");
-    return WTB_ERR_ARG;
-  }
   int st = 0, stq[2] = {0, 0};
   WTB_HIP(hipMemcpyAsync(p->qmode ? stq : &st, p->status, sizeof(int) * (p->qmode ? 2 : 1), hipMemcpyDeviceToHost,
                          s));
@@ -983,6 +994,23 @@ int wtb_bse_plan_results(wtb_bse_plan* p, double* w, double* act, double* eps, d
       if (v <= g) g = v;
     *egap = g;
   }
+  *status = p->qmode ? qmode_status(stq) : st;
+  return WTB_OK;
+}
+
+int wtb_bse_plan_results(wtb_bse_plan* p, double* w, double* act, double* eps, double* egap) {
+  if (!p) {
+    set_error("wtb_bse_plan_results: null plan");
+    return WTB_ERR_ARG;
+  }
+  if (p->qmode && (act || eps || egap)) {
+    set_error("wtb_bse_plan_results: a finite-Q plan gives the exciton energies only (act, eps, egap NULL)");
+    return WTB_ERR_ARG;
+  }
+  int st = 0;
+  int rc = plan_read(p, w, act, eps, egap, &st);
+  if (!rc && solve_stalled(st) && !(rc = plan_redo(p))) rc = plan_read(p, w, act, eps, egap, &st);
+  if (rc) return rc;
   if (p->timing) {
     // stage boundaries: [0]=start [1]=eig [2]=dip [3]=build [4]=tridiag [5]=dc [6]=end
     float t;
@@ -1002,8 +1030,7 @@ int wtb_bse_plan_results(wtb_bse_plan* p, double* w, double* act, double* eps, d
       if (hipEventElapsedTime(&t, p->kev[2 * c], p->kev[2 * c + 1]) == hipSuccess) p->kernel_ms += t;
     }
   }
-  if (p->qmode) st = qmode_status(stq);
-  int rc = status_to_code(st);
+  rc = status_to_code(st);
   if (rc) set_error(status_text(rc));
   return rc;
 }
@@ -1082,25 +1109,13 @@ int wtb_bsesolver(wtb_ctx* c, const wtb_tb_model* m, const wtb_bse_params* prm, 
 }
 
 // ---------------------------------------------------------------------------
-int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w) {
-  if (!c || !a || !w || n < 1 || lda < n) {
-    set_error("wtb_zheev: bad argument");
-    return WTB_ERR_ARG;
-  }
-  WTB_HIP(hipSetDevice(c->device));
+static int zheev_solve(wtb_ctx* c, int vec, bool two, int n, double* a, int lda, double* w, int* status) {
   hipStream_t s = c->stream;
-  const int vec = want_vectors ? 1 : 0;
   zc *da = nullptr, *dh = nullptr, *dx = nullptr;
   void *tri = nullptr, *dcw = nullptr, *btw = nullptr;
   double *dl = nullptr, *dz = nullptr;
   int* dst = nullptr;
-  int rc, st = 0;
-  // Eigenvalues alone take the two-stage reduction, as a plan's do (plan_two_stage).  With
-  // vectors it would be faster (24 ms against 32 at n = 1290), but the chase takes every row
-  // through n / 2 more transformations, whose roundings add up: |A X - X W| / |A| is 0.8 eps
-  // n^1/2 after it and stays at 6 eps without (n = 64 .. 1600), the vectors' largest error
-  // 1.1e-12 against 3.6e-13 at n = 1290.
-  const bool two = !vec && n >= kTwoStageMinN64;
+  int rc;
   const int band = plan_default_band(false, n);
   if ((rc = dmalloc(&da, (size_t)lda * n)) || (rc = dmalloc(&dh, (size_t)n * n)) || (rc = dmalloc(&dst, 1)) ||
       (rc = dmalloc((char**)&tri, two ? band_work_bytes(n, band, 0) + sizeof(double) * 2 * n
@@ -1135,7 +1150,7 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
     if (!rc && vec) rc = run_backtr(s, dh, n, n, tw.tau, dz, 0, n, dx, n, btw);
     if (!rc) {
       hipMemcpyAsync(w, dl, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-      hipMemcpyAsync(&st, dst, sizeof(int), hipMemcpyDeviceToHost, s);
+      hipMemcpyAsync(status, dst, sizeof(int), hipMemcpyDeviceToHost, s);
       // one block where the array has no gaps: the strided copy to pageable memory goes column
       // by column (10 ms more at n = 1290)
       if (vec)
@@ -1144,8 +1159,6 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
       if (hipStreamSynchronize(s) != hipSuccess) {
         set_error("wtb_zheev: stream error");
         rc = WTB_ERR_HIP;
-      } else if ((rc = status_to_code(st))) {
-        set_error(status_text(rc));
       }
     }
   }
@@ -1158,6 +1171,26 @@ int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w
   hipFree(btw);
   hipFree(dl);
   hipFree(dz);
+  return rc;
+}
+
+int wtb_zheev(wtb_ctx* c, int want_vectors, int n, double* a, int lda, double* w) {
+  if (!c || !a || !w || n < 1 || lda < n) {
+    set_error("wtb_zheev: bad argument");
+    return WTB_ERR_ARG;
+  }
+  WTB_HIP(hipSetDevice(c->device));
+  const int vec = want_vectors ? 1 : 0;
+  // Eigenvalues alone take the two-stage reduction, as a plan's do (plan_two_stage).  With
+  // vectors it would be faster (24 ms against 32 at n = 1290), but the chase takes every row
+  // through n / 2 more transformations, whose roundings add up: |A X - X W| / |A| is 0.8 eps
+  // n^1/2 after it and stays at 6 eps without (n = 64 .. 1600), the vectors' largest error
+  // 1.1e-12 against 3.6e-13 at n = 1290.
+  const bool two = !vec && n >= kTwoStageMinN64;
+  int st = 0;
+  int rc = zheev_solve(c, vec, two, n, a, lda, w, &st);
+  if (!rc && solve_stalled(st)) rc = zheev_solve(c, vec, false, n, a, lda, w, &st);
+  if (!rc && (rc = status_to_code(st))) set_error(status_text(rc));
   return rc;
 }
 
@@ -1698,13 +1731,11 @@ int wtb_bse_plan_lowest(wtb_bse_plan* p, const wtb_davidson_params* dp, const wt
       inf.used_fallback = 1;
       if (!p->H) rc = dmalloc(&p->H, p->ldh * N);
       if (!rc) {
+        std::vector<double> wall(N);
         p->mixed = false;
         rc = plan_enqueue(p);
+        if (!rc) rc = wtb_bse_plan_results(p, wall.data(), nullptr, eps, nullptr);
         p->mixed = true;
-      }
-      if (!rc) {
-        std::vector<double> wall(N);
-        rc = wtb_bse_plan_results(p, wall.data(), nullptr, eps, nullptr);
         if (!rc) {
           for (int i = 0; i < nev; ++i) {
             W[i] = wall[i];
@@ -2485,6 +2516,17 @@ int wtb_bse_bands_run_wf(wtb_bse_bands* b, int nq, const double* qauxv, double* 
       rc = WTB_ERR_HIP;
     }
   for (int iq = 0; iq < nq && !rc; ++iq) {
+    if (solve_stalled(qmode_status(b->hst + 2 * iq))) {
+      wtb_bse_plan* p = b->plans[iq % nl];
+      hipStream_t st = p->stream;
+      if (hipMemcpyAsync(p->dq, b->hq + 4 * iq, sizeof(double) * 4, hipMemcpyHostToDevice, st) != hipSuccess) rc = WTB_ERR_HIP;
+      if (!rc) rc = plan_redo(p);
+      if (!rc && (hipMemcpyAsync(b->hw + (size_t)N * iq, p->lambda, sizeof(double) * N, hipMemcpyDeviceToHost, st) != hipSuccess ||
+                  hipMemcpyAsync(b->hst + 2 * iq, p->status, sizeof(int) * 2, hipMemcpyDeviceToHost, st) != hipSuccess ||
+                  hipStreamSynchronize(st) != hipSuccess))
+        rc = WTB_ERR_HIP;
+      if (rc) break;
+    }
     const int code = status_to_code(qmode_status(b->hst + 2 * iq));
     if (code) {
       set_error(status_text(code));

@@ -163,6 +163,9 @@ struct BandWork {
   double kev_flops = 0.0;       // summed over the timed launches
 };
 size_t band_work_bytes(int N, int b, int nrhs);
+// the status bit of a reduction whose workgroups waited in vain, set with WTB_ERR_EIG's: the
+// caller takes the one-stage reduction, which has no such waits
+constexpr int kStalled = 1 << 30;
 // eigenvectors from Z (N x ., real) after a reduction that kept its reflectors: columns
 // c0 .. c0 + m - 1; N <= band_vec_rows()
 bool band_vec_two_stage(int N, int m);   // the faster form for m vectors
@@ -170,7 +173,10 @@ size_t band_tau_elems(int N);     // tau1 and tau2 together
 int band_vec_rows();
 int run_band_backtr(hipStream_t s, const BandWork& w, const zc* H, int ld, const double* Z, int c0, int m, zc* X,
                     int ldx, int cus, void* work);
-int band_panel_rows();            // largest N whose COMPLEX*16 panels run in one launch (band 16)
+// whether the COMPLEX*16 panels of an N x N matrix run in one launch each (band 16) on the
+// current device; at most up to N = band_panel_rows()
+bool band_panel_fits(int N);
+int band_panel_rows();
 int band_bind(BandWork& w, void* base, int N, int b, int nrhs);
 int run_band_tridiag(hipStream_t s, BandWork& w, zc* H, int ld, zc* g, double* d, double* e, int* status);
 int run_band_tridiag_f32(hipStream_t s, BandWork& w, zf* H, int ld, zc* g, double* d, double* e, int* status);
