@@ -134,3 +134,21 @@ def test_the_launches_of_eight_streams(ctx):  # noqa: F811
         with bse.BSEBands(ctx, m, prm, lanes=8) as b:
             for _ in range(3):
                 assert np.array_equal(b.run(q), ref), grid
+
+
+@pytest.mark.parametrize("bits", [0xFFFFFFFFFFFFFFFF, 0x7FF8000000000000])
+def test_nan_of_any_bits_does_not_stall(ctx, bits):  # noqa: F811
+    """an empty slot of the panels' exchange is a NaN of all ones; one in the matrix is a value
+    like another (a wait that ran out would take most of a second and then the one-stage form)"""
+    import time
+    from wantibexos_amd import bse
+    n = 300
+    a = np.eye(n, dtype=complex)
+    bse.zheev(ctx, a)
+    a.view(np.uint64)[40, 2 * 100] = bits
+    t = time.perf_counter()
+    try:
+        bse.zheev(ctx, a)
+    except bse.WTBError as e:
+        assert e.code == 10                     # NaN or Inf in the input
+    assert time.perf_counter() - t < 0.2

@@ -1058,9 +1058,9 @@ __device__ inline double lane_value(double x, int l) {
 __device__ inline zc lane_value(zc v, int l) { return mkz(lane_value(v.re, l), lane_value(v.im, l)); }
 
 // Values handed from every workgroup to every workgroup: slot [round][workgroup][B], each
-// slot written once per panel and filled with the bits ~0 before (no arithmetic result has
-// them), so that a reader polls the value itself: no counter, no fence, one store and one
-// load apart.  Rounds 0 .. B - 1 are the panel's columns, B .. B + 5 the tracked vectors;
+// slot written once per panel and filled with the bits ~0 before (a NaN that st_slot never
+// stores: an input's NaN may have them and keeps its bits through arithmetic), so that a
+// reader polls the value itself: no counter, no fence, one store and one load apart.  Rounds 0 .. B - 1 are the panel's columns, B .. B + 5 the tracked vectors;
 // entry nwg of a column's round is row c of the panel.
 struct QrPanelArgs {
   zc* A;                 // the matrix, ld
@@ -1081,6 +1081,15 @@ struct QrPanelArgs {
 __device__ inline bool is_empty(zc v) {
   return __builtin_bit_cast(unsigned long long, v.re) == ~0ull || __builtin_bit_cast(unsigned long long, v.im) == ~0ull;
 }
+
+// a value into its slot, any NaN by the usual bits
+__device__ inline void st_slot(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff, zc v) {
+  if (v.re != v.re) v.re = __builtin_nan("");
+  if (v.im != v.im) v.im = __builtin_nan("");
+  st_buf(rs, voff, soff, v);
+}
+// what a poll of slots starts with: the loads after it are not those of the poll before
+__device__ inline void poll_again() { __asm__ volatile("" ::: "memory"); }
 
 template <int B>
 __host__ __device__ constexpr size_t qr_slots(int nwg_max) { return (size_t)(B + 6) * (nwg_max + 1) * B; }
@@ -1161,6 +1170,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
       zc v[NR][U];
       for (int tries = 0;; ++tries) {
         bool ok = true;
+        poll_again();
 #pragma unroll
         for (int r = 0; r < NR; ++r)
           if (r < nr)
@@ -1237,8 +1247,8 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
 #pragma unroll
         for (int p = 0; p < B; ++p) v[p] = fma_conj(xm, row[p], mkz(0, 0));
         const zc part = block_sums(v);
-        if (sub == 0) st_buf(ex, mine + q * (unsigned)sizeof(zc), c * RS, part);
-        if (blockIdx.x == 0 && sub == 1) st_buf(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
+        if (sub == 0) st_slot(ex, mine + q * (unsigned)sizeof(zc), c * RS, part);
+        if (blockIdx.x == 0 && sub == 1) st_slot(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
         if (c > 0) t_column(c - 1);            // while the sums are on their way
         zc rowv = mkz(0, 0);
         zc tot;
@@ -1294,7 +1304,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
     for (int j = 0; j < B; ++j) v[j] = fma_conj(row[j], g[r], mkz(0, 0));
     if (r > 0) lds_barrier();                  // the partial sums of r - 1 are read
     const zc part = block_sums(v);
-    if (sub == 0) st_buf(ex, mine + q * (unsigned)sizeof(zc), (B + r) * RS, part);
+    if (sub == 0) st_slot(ex, mine + q * (unsigned)sizeof(zc), (B + r) * RS, part);
   }
   t_column(a.k - 1);
 #pragma unroll
@@ -1433,8 +1443,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
   for (int u = 0; u < NE; ++u) {
     const int e = t + 256 * u;
     const zc p = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
-    st_buf(ex, (unsigned)((size_t)blockIdx.x * B * B + e) * (unsigned)sizeof(zc), 0,
-           p);
+    st_slot(ex, (unsigned)((size_t)blockIdx.x * B * B + e) * (unsigned)sizeof(zc), 0, p);
   }
   // while the sums are on their way: the rows of V and X that become W
   zc vv[4][B / 4], xx[4][TI][4];
@@ -1459,6 +1468,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
       zc v[8];
       for (int tries = 0;; ++tries) {
         bool ok = true;
+        poll_again();
 #pragma unroll
         for (int x = 0; x < 8; ++x)
           v[x] = ld_buf(ex, (unsigned)(min(wg0 + x, a.nwg - 1) * (B * B) + e) * (unsigned)sizeof(zc), 0);

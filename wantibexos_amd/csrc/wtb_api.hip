@@ -35,9 +35,6 @@ __global__ void k_upper_to_lower(int n, const zc* __restrict__ a, int lda, zc* _
   zc v = a[(size_t)j + (size_t)lda * i];      // a(j,i), j <= i
   v = conj(v);
   if (i == j) v.im = 0.0;
-  // any NaN by the usual bits: all bits set mark an empty slot of the panels' exchange
-  if (v.re != v.re) v.re = __builtin_nan("");
-  if (v.im != v.im) v.im = __builtin_nan("");
   h[(size_t)i + (size_t)ldh * j] = v;
 }
 
