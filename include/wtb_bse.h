@@ -146,7 +146,8 @@ int wtb_eigsys(wtb_ctx* ctx, const wtb_tb_model* model, int nk, const double* kp
  * a(lda,n) is read.  want_vectors = 0: eigenvalues only.  want_vectors = 1:
  * a is overwritten with the orthonormal eigenvectors (column j <-> w[j]),
  * each scaled so that its last component is real and >= 0 (ZHEEV's vectors
- * have a real last component of either sign). */
+ * have a real last component of either sign).  A NaN or an infinity in the
+ * triangle gives WTB_ERR_NONFINITE. */
 int wtb_zheev(wtb_ctx* ctx, int want_vectors, int n, double* a, int lda, double* w);
 
 /* dielbsev (subroutines/bse_subs.f90:336-378): act(i) = |sum_j x(j,i) h(j)|^2 */

@@ -764,7 +764,8 @@ __global__ __launch_bounds__(256) void k_dcv_gather(DCArgs a) {
   const int n = nd.hi - nd.lo, i = blockIdx.x;
   if (i >= n) return;
   const size_t N = a.N;
-  const double* src = a.Z + (size_t)a.perm[nd.lo + i] * N;
+  // NaN eigenvalues have no order, and an entry of perm may be unset
+  const double* src = a.Z + (size_t)min(max(a.perm[nd.lo + i], nd.lo), nd.hi - 1) * N;
   double* dst = a.Z2 + (size_t)(nd.lo + i) * N;
   for (int r = nd.lo + threadIdx.x; r < nd.hi; r += 256) dst[r] = src[r];
 }

@@ -27,14 +27,17 @@ __global__ void k_split_g(int N, int nrhs, const zc* __restrict__ g, double* __r
     track[(size_t)(2 * q + 1) * N + i] = v.im;
   }
 }
-// lower triangle of the Hermitian matrix whose upper triangle is given (ZHEEV 'U')
-__global__ void k_upper_to_lower(int n, const zc* __restrict__ a, int lda, zc* __restrict__ h, int ldh) {
+// lower triangle of the Hermitian matrix whose upper triangle is given (ZHEEV 'U'); a NaN or
+// an infinity in it sets *status
+__global__ void k_upper_to_lower(int n, const zc* __restrict__ a, int lda, zc* __restrict__ h, int ldh,
+                                 int* __restrict__ status) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   int j = blockIdx.y;
   if (i >= n || i < j) return;
   zc v = a[(size_t)j + (size_t)lda * i];      // a(j,i), j <= i
   v = conj(v);
   if (i == j) v.im = 0.0;
+  if (!isfinite(v.re) || !isfinite(v.im)) atomicOr(status, 1 << WTB_ERR_NONFINITE);
   h[(size_t)i + (size_t)ldh * j] = v;
 }
 
@@ -42,6 +45,7 @@ static int status_to_code(int st) {
   if (st & (1 << WTB_ERR_NOCP)) return WTB_ERR_NOCP;
   if (st & (1 << WTB_ERR_NVAL)) return WTB_ERR_NVAL;
   if (st & (1 << WTB_ERR_NCOND)) return WTB_ERR_NCOND;
+  if (st & (1 << WTB_ERR_NONFINITE)) return WTB_ERR_NONFINITE;
   if (st & (1 << WTB_ERR_EIG)) return WTB_ERR_EIG;
   return WTB_OK;
 }
@@ -52,6 +56,7 @@ static const char* status_text(int code) {
     case WTB_ERR_NOCP: return "no band above the Fermi level at some k (nocp undefined)";
     case WTB_ERR_NVAL: return "Number of valence states higher then ocuppied states";
     case WTB_ERR_NCOND: return "Number of conduction states higher then unocuppied states";
+    case WTB_ERR_NONFINITE: return "NaN or Inf in the matrix";
     case WTB_ERR_EIG: return "The algorithm failed to compute eigenvalues.";
     default: return "";
   }
@@ -1139,8 +1144,8 @@ static int zheev_solve(wtb_ctx* c, int vec, bool two, int n, double* a, int lda,
     if (!rc) rc = dc_prepare(dcw, n, 0, tree, vec);
     if (!rc) {
       hipMemcpyAsync(da, a, sizeof(zc) * lda * n, hipMemcpyHostToDevice, s);
-      hipLaunchKernelGGL(k_upper_to_lower, dim3((n + 255) / 256, n), dim3(256), 0, s, n, da, lda, dh, n);
       hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, s, dst, 1);
+      hipLaunchKernelGGL(k_upper_to_lower, dim3((n + 255) / 256, n), dim3(256), 0, s, n, da, lda, dh, n, dst);
       rc = two ? run_band_tridiag(s, bw, dh, n, nullptr, tw.d, tw.e, dst) : run_tridiag(s, tw, dh, n, nullptr);
     }
     if (!rc) rc = run_dc(s, dcw, tree, tw.d, tw.e, nullptr, dl, dz);
