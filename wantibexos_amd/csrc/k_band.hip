@@ -812,10 +812,10 @@ __global__ __launch_bounds__(256) void k_hmm_sum(int m, int ns, const zc* __rest
 // Hermitian, so that a lane's result lands next to its neighbours' in the column-major
 // matrix.
 template <class T, int B>
-__global__ __launch_bounds__(256, 4) void k_her2k_full(T* __restrict__ A, int ld, int m, int r0, int N,
-                                                    const zc* __restrict__ V, const zc* __restrict__ W) {
+__device__ __forceinline__ void her2k_tile(T* __restrict__ A, int ld, int m, int r0, int N, const zc* __restrict__ V,
+                                           const zc* __restrict__ W, const int bx) {
   // one workgroup per tile on or below the diagonal: t -> tile row ti >= tile column tj
-  const int t = blockIdx.x;
+  const int t = bx;
   int ti = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
   while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
   while (ti * (ti + 1) / 2 > t) --ti;
@@ -959,17 +959,27 @@ __global__ __launch_bounds__(256, 4) void k_her2k_full(T* __restrict__ A, int ld
         }
       }
 }
+template <class T, int B>
+__global__ __launch_bounds__(256, 4) void k_her2k_full(T* __restrict__ A, int ld, int m, int r0, int N,
+                                                    const zc* __restrict__ V, const zc* __restrict__ W) {
+  her2k_tile<T, B>(A, ld, m, r0, N, V, W, blockIdx.x);
+}
 
 // band of width b of the lower triangle into BD (FP64), zero for b < d <= 2b; gc = conj(g)
 template <class T>
-__global__ void k_band_extract(const T* __restrict__ A, int ld, int N, int b, int LB, zc* __restrict__ BD) {
-  const int c = blockIdx.x;
+__device__ __forceinline__ void band_extract(const T* __restrict__ A, int ld, int N, int b, int LB,
+                                             zc* __restrict__ BD, const int bx) {
+  const int c = bx;
   for (int d = threadIdx.x; d < LB; d += blockDim.x) {
     zc v = mkz(0, 0);
     if (d <= b && c + d < N) v = ldz(A[(size_t)(c + d) + (size_t)ld * c]);
     if (d == 0) v.im = 0.0;
     BD[(size_t)c * LB + d] = v;
   }
+}
+template <class T>
+__global__ void k_band_extract(const T* __restrict__ A, int ld, int N, int b, int LB, zc* __restrict__ BD) {
+  band_extract(A, ld, N, b, LB, BD, blockIdx.x);
 }
 
 __global__ void k_conj_vec(int n, const zc* __restrict__ x, zc* __restrict__ y) {
@@ -1108,7 +1118,7 @@ __host__ __device__ constexpr size_t qr_slots(int nwg_max) { return (size_t)(B +
 // update of the rows the rest; the launches that it replaces took about 10 us a column.  The
 // launch needs every workgroup resident: band_panel_wg.
 template <int B>
-__global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
+__device__ __forceinline__ void qr_panel(const QrPanelArgs& a, const int bx) {
   constexpr int SUB = 256 / B;                 // threads per exchanged value
   constexpr int NT = B / SUB;                  // T entries per thread
   __shared__ zc lp[4][4][B / 4][16];           // partial sums [wave][row quarter][column][lane]
@@ -1117,13 +1127,13 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   __shared__ zc t1s[6][B], t2s[6][B];
   __shared__ int bad;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int i = blockIdx.x * 256 + t;          // panel row
+  const int i = bx * 256 + t;          // panel row
   const bool live = i < a.m;
   const int q = t / SUB, sub = t % SUB;        // exchanged value; T row and its columns sub + SUB u
   const size_t N = a.N;
   const unsigned RS = (unsigned)(a.exs * B) * (unsigned)sizeof(zc);   // bytes per round
   const __amdgpu_buffer_rsrc_t ex = dev_buffer(a.ex, (size_t)(B + 6) * RS);
-  const unsigned mine = (unsigned)(blockIdx.x * B) * (unsigned)sizeof(zc);
+  const unsigned mine = (unsigned)(bx * B) * (unsigned)sizeof(zc);
   if (t == 0) bad = 0;
   zc row[B];
   {
@@ -1137,8 +1147,8 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   }
   // the next panel's slots
   const zc empty = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
-  for (int e = t; e < (B + 6) * B; e += 256) a.ex_next[(size_t)(e / B) * a.exs * B + (size_t)blockIdx.x * B + e % B] = empty;
-  if (blockIdx.x == 0)
+  for (int e = t; e < (B + 6) * B; e += 256) a.ex_next[(size_t)(e / B) * a.exs * B + (size_t)bx * B + e % B] = empty;
+  if (bx == 0)
     for (int e = t; e < B * B; e += 256) a.ex_next[(size_t)(e / B) * a.exs * B + (size_t)a.nwg * B + e % B] = empty;
 
   // sum over the workgroup of B values a thread: halved over the lane halves and the rows of
@@ -1237,7 +1247,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
     for (int cc = 0; cc < 4; ++cc) {
       const int c = base + cc;
       if (c < a.k) {
-        if (blockIdx.x == 0 && i == c) {
+        if (bx == 0 && i == c) {
 #pragma unroll
           for (int p = 0; p < B; ++p) rowc[p] = row[p];
         }
@@ -1248,7 +1258,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
         for (int p = 0; p < B; ++p) v[p] = fma_conj(xm, row[p], mkz(0, 0));
         const zc part = block_sums(v);
         if (sub == 0) st_slot(ex, mine + q * (unsigned)sizeof(zc), c * RS, part);
-        if (blockIdx.x == 0 && sub == 1) st_slot(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
+        if (bx == 0 && sub == 1) st_slot(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
         if (c > 0) t_column(c - 1);            // while the sums are on their way
         zc rowv = mkz(0, 0);
         zc tot;
@@ -1318,7 +1328,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
   }
   lds_barrier();
   if (bad) return;
-  if (blockIdx.x == 0) {
+  if (bx == 0) {
     for (int e = t; e < B * B; e += 256) a.Tm[e] = Ts[e % B][e / B];
     if (a.tau && t < a.k) a.tau[t] = Ts[t][t];
   }
@@ -1364,6 +1374,10 @@ __global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
     }
   }
 }
+template <int B>
+__global__ __launch_bounds__(256, 2) void k_qr_panel(QrPanelArgs a) {
+  qr_panel<B>(a, blockIdx.x);
+}
 
 // W = X - 1/2 V (T^H (V^H X)) with X = A22 Y, in one launch: workgroup w takes rows 256 w ..,
 // its part of M = V^H X on FP64 MFMA (operands straight from memory in the MFMA's layout),
@@ -1382,7 +1396,7 @@ struct QrWArgs {
 };
 
 template <int B>
-__global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
+__device__ __forceinline__ void qr_w(const QrWArgs& a, const int bx) {
   constexpr int TI = B / 16, NE = B * B / 256;
   __shared__ zc buf[4 * B * B];                // the waves' parts, then M, Z, T
   typedef zc Mat[B][B + 1];
@@ -1393,12 +1407,12 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   const size_t N = a.N;
-  const int row0 = blockIdx.x * 256;
+  const int row0 = bx * 256;
   const __amdgpu_buffer_rsrc_t ex = dev_buffer(a.ex, (size_t)a.nwg * B * B * sizeof(zc));
   if (t == 0) bad = 0;
   const zc empty = __builtin_bit_cast(zc, make_uint4(~0u, ~0u, ~0u, ~0u));
 #pragma unroll
-  for (int u = 0; u < NE; ++u) a.ex_next[(size_t)blockIdx.x * B * B + t + 256 * u] = empty;
+  for (int u = 0; u < NE; ++u) a.ex_next[(size_t)bx * B * B + t + 256 * u] = empty;
   zc tm[NE];
 #pragma unroll
   for (int u = 0; u < NE; ++u) tm[u] = a.Tm[t + 256 * u];
@@ -1443,7 +1457,7 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
   for (int u = 0; u < NE; ++u) {
     const int e = t + 256 * u;
     const zc p = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
-    st_slot(ex, (unsigned)((size_t)blockIdx.x * B * B + e) * (unsigned)sizeof(zc), 0, p);
+    st_slot(ex, (unsigned)((size_t)bx * B * B + e) * (unsigned)sizeof(zc), 0, p);
   }
   // while the sums are on their way: the rows of V and X that become W
   zc vv[4][B / 4], xx[4][TI][4];
@@ -1533,15 +1547,19 @@ __global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
         }
   }
 }
+template <int B>
+__global__ __launch_bounds__(256, 2) void k_qr_w(QrWArgs a) {
+  qr_w<B>(a, blockIdx.x);
+}
 
 // The 16 columns of the next panel, ahead of k_update_mul (5.4 us, latency-bound): A(:, 0:16) -= (V W^H + W V^H)(:, 0:16)
 // on and below the diagonal, rows 0 .. m - 1 of the trailing matrix at A.  One 16 x 16 MFMA
 // tile a wave, rows over the MFMA's columns as in k_her2k_full.
 template <int B>
-__global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m, int N, const zc* __restrict__ V,
-                                               const zc* __restrict__ W) {
+__device__ __forceinline__ void strip(zc* __restrict__ A, int ld, int m, int N, const zc* __restrict__ V,
+                                      const zc* __restrict__ W, const int bx) {
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
-  const int r = blockIdx.x * 64 + (threadIdx.x >> 6) * 16 + lr, rc = min(r, m - 1), c = min(lr, m - 1);
+  const int r = bx * 64 + (threadIdx.x >> 6) * 16 + lr, rc = min(r, m - 1), c = min(lr, m - 1);
   zc av[B / 2], bv[B / 2], h[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) h[q] = A[(size_t)rc + (size_t)ld * min(lk + 4 * q, m - 1)];
@@ -1564,6 +1582,11 @@ __global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m
     const int cc = lk + 4 * q;
     if (r < m && cc <= r) A[(size_t)r + (size_t)ld * cc] = mkz(h[q].re - cr[q], h[q].im + ci[q]);
   }
+}
+template <int B>
+__global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m, int N, const zc* __restrict__ V,
+                                               const zc* __restrict__ W) {
+  strip<B>(A, ld, m, N, V, W, blockIdx.x);
 }
 
 // One pass over the trailing matrix A (m x m, lower triangle): the update of the panel before,
@@ -1589,17 +1612,17 @@ __global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m
 #define UM_R 128
 __host__ __device__ inline int um_parts(int K, int n, int nt) { return 4 / n * (K + 1) + nt - K; }
 template <int B, bool UPD>
-__global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int ld, int m, int N,
-                                                       const zc* __restrict__ V, const zc* __restrict__ W,
-                                                       const zc* __restrict__ Y, zc* __restrict__ part, int nt, int n) {
+__device__ __forceinline__ void update_mul(zc* __restrict__ A, int ld, int m, int N, const zc* __restrict__ V,
+                                           const zc* __restrict__ W, const zc* __restrict__ Y, zc* __restrict__ part,
+                                           int nt, int n, const int bx) {
   static_assert(B == 16, "one MFMA tile of Y columns");
   __shared__ zc tr[4][16 * 17];                // a wave's tile on its way through
   __shared__ zc red[4][2][4][64];              // the waves' parts of A^H Y
-  const int ng = 4 / n, t = blockIdx.x / ng;
+  const int ng = 4 / n, t = bx / ng;
   int ti = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
   while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
   while (ti * (ti + 1) / 2 > t) --ti;
-  const int tj = t - ti * (ti + 1) / 2, g = tj * ng + (int)blockIdx.x % ng;
+  const int tj = t - ti * (ti + 1) / 2, g = tj * ng + bx % ng;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r0 = ti * UM_R + wave * 32;
   d4 ar[2], ai[2];                             // (A Y)^T of this wave's rows [y]
@@ -1781,15 +1804,26 @@ __global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int l
       for (int q = 0; q < 4; ++q) part[((size_t)g * B + (lane >> 4) + 4 * q) * m + row] = mkz(ar[y][q], ai[y][q]);
   }
 }
+template <int B, bool UPD>
+__global__ __launch_bounds__(256, 2) void k_update_mul(zc* __restrict__ A, int ld, int m, int N,
+                                                       const zc* __restrict__ V, const zc* __restrict__ W,
+                                                       const zc* __restrict__ Y, zc* __restrict__ part, int nt, int n) {
+  update_mul<B, UPD>(A, ld, m, N, V, W, Y, part, nt, n, blockIdx.x);
+}
 
 // X(row, col) = the sum of the parts of k_update_mul, in slot order
 template <int B>
-__global__ __launch_bounds__(256) void k_um_sum(int m, int n, int nt, const zc* __restrict__ part, zc* __restrict__ X,
-                                                int ldx) {
-  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void um_sum(int m, int n, int nt, const zc* __restrict__ part, zc* __restrict__ X, int ldx,
+                                       const int bx) {
+  const size_t e = (size_t)bx * 256 + threadIdx.x;
   if (e >= (size_t)m * B) return;
   const int row = (int)(e % m), col = (int)(e / m);
   X[(size_t)row + (size_t)ldx * col] = strided_sum(part + e, (size_t)m * B, 0, um_parts(row / UM_R, n, nt), 1, mkz(0, 0));
+}
+template <int B>
+__global__ __launch_bounds__(256) void k_um_sum(int m, int n, int nt, const zc* __restrict__ part, zc* __restrict__ X,
+                                                int ldx) {
+  um_sum<B>(m, n, nt, part, X, ldx, blockIdx.x);
 }
 
 __global__ void k_fill_empty(zc* p, size_t n) {
@@ -1915,7 +1949,7 @@ __device__ inline int lds_get(int* f) {
 // four waves that met at barriers and moved every block through memory took 62 ms (band 32,
 // 12 us a sweep).  With eight waves a sweep and barriers, band 16 took 28 ms.
 template <int B, bool VEC>
-__global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseArgs a) {
+__device__ __forceinline__ void chase(const ChaseArgs& a) {
   typedef ChaseDim<B> C;
   constexpr int SW = C::SW, R = C::R, NC = C::NC, P = C::P;
   constexpr int GPW = 64 / B;                  // column groups
@@ -2169,6 +2203,116 @@ __global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseAr
     if (last) publish(nt);
   }
 }
+template <int B, bool VEC>
+__global__ __launch_bounds__((ChaseDim<B>::SW + 1) * 64, 1) void k_chase(ChaseArgs a) {
+  chase<B, VEC>(a);
+}
+
+// ---------------------------------------------------------------------------
+// One matrix's arguments, and sets of matrices
+// ---------------------------------------------------------------------------
+// The arguments that do not change from panel to panel (COMPLEX*16, band 16); the launches of
+// panel p take theirs from these, on the host for one matrix, on the device for a set
+struct BandItem {
+  zc* H;
+  int ld, N, nrhs;
+  zc *V, *X, *V2, *X2;   // of the even and of the odd panels
+  zc *Y, *T, *gc, *part;
+  zc* ex;                // exchange slots of the even, then of the odd panels
+  size_t exn, wo;        // slots of one parity; where k_qr_w's begin
+  int exw;               // workgroups that they hold
+  int* err;
+  int spin;
+  zc* tau1;
+  ChaseArgs chase;
+};
+
+// rows of the trailing matrix of panel p; a panel has at least two
+__host__ __device__ inline int panel_rows(const BandItem& t, int p) { return t.N - 16 * (p + 1); }
+__host__ __device__ inline int panel_wgs(const BandItem& t, int p) { return (panel_rows(t, p) + PR - 1) / PR; }
+__host__ __device__ inline bool last_panel(const BandItem& t, int p) { return panel_rows(t, p + 1) < 2; }
+__host__ __device__ inline zc* trailing(const BandItem& t, int p) { return t.H + (size_t)16 * (p + 1) * (t.ld + 1); }
+__host__ __device__ inline zc* panel_v(const BandItem& t, int p) { return p & 1 ? t.V2 : t.V; }
+__host__ __device__ inline zc* panel_x(const BandItem& t, int p) { return p & 1 ? t.X2 : t.X; }
+__host__ __device__ inline QrPanelArgs qr_panel_args(const BandItem& t, int p) {
+  const int m = panel_rows(t, p);
+  return QrPanelArgs{t.H, t.ld, t.N, 16 * p, 16 * (p + 1), m, m > 16 ? 16 : m - 1, panel_v(t, p), t.Y, t.T, t.gc, t.nrhs,
+                     t.ex + (p & 1) * t.exn, t.ex + ((p + 1) & 1) * t.exn, t.exw + 1, panel_wgs(t, p), t.err + 8, t.spin,
+                     t.tau1 ? t.tau1 + 16 * p : nullptr};
+}
+__host__ __device__ inline QrWArgs qr_w_args(const BandItem& t, int p) {
+  return QrWArgs{panel_rows(t, p), t.N, panel_v(t, p), t.T, panel_x(t, p), t.ex + (p & 1) * t.exn + t.wo,
+                 t.ex + ((p + 1) & 1) * t.exn + t.wo, panel_wgs(t, p), t.err + 8, t.spin};
+}
+// steps of k_update_mul: fewer parts with more steps, more workgroups with fewer (at these
+// sizes about 1200 workgroups either way, 512 run at once; lines at half and one and a half
+// times these sizes measured within 1 %)
+constexpr int UM_4 = 6144, UM_2 = 3072;
+__host__ __device__ inline int um_steps(int m) { return m > UM_4 ? 4 : m > UM_2 ? 2 : 1; }
+__host__ __device__ inline int um_blocks(int m) {
+  const int nt = (m + UM_R - 1) / UM_R;
+  return 4 / um_steps(m) * (nt * (nt + 1) / 2);
+}
+
+// One launch for a set: workgroup b belongs to the matrix whose range [pre[i], pre[i + 1])
+// holds it and runs the one matrix's kernel body on that matrix's arguments with block index
+// b - pre[i], so that every matrix goes through the arithmetic of its own reduction.
+constexpr int kSetMax = 64;
+struct BandSlots {
+  const BandItem* items;       // of slot 0 on
+  int n;
+  int pre[kSetMax + 1];
+};
+__device__ inline int set_slot(const BandSlots& S, int b) {
+  int lo = 0, hi = S.n;        // pre[lo] <= b < pre[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (S.pre[mid] <= b) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+__global__ __launch_bounds__(256) void k_strip_s(BandSlots S, int p) {
+  const int i = set_slot(S, blockIdx.x);
+  const BandItem& t = S.items[i];
+  strip<16>(trailing(t, p - 1), t.ld, panel_rows(t, p - 1), t.N, panel_v(t, p - 1), panel_x(t, p - 1), (int)blockIdx.x - S.pre[i]);
+}
+__global__ __launch_bounds__(256, 2) void k_qr_panel_s(BandSlots S, int p) {
+  const int i = set_slot(S, blockIdx.x);
+  qr_panel<16>(qr_panel_args(S.items[i], p), (int)blockIdx.x - S.pre[i]);
+}
+template <bool UPD>
+__global__ __launch_bounds__(256, 2) void k_update_mul_s(BandSlots S, int p) {
+  const int i = set_slot(S, blockIdx.x);
+  const BandItem& t = S.items[i];
+  const int m = panel_rows(t, p);
+  update_mul<16, UPD>(trailing(t, p), t.ld, m, t.N, panel_v(t, p + 1) + 16, panel_x(t, p + 1) + 16, t.Y, t.part,
+                      (m + UM_R - 1) / UM_R, um_steps(m), (int)blockIdx.x - S.pre[i]);
+}
+__global__ __launch_bounds__(256) void k_um_sum_s(BandSlots S, int p) {
+  const int i = set_slot(S, blockIdx.x);
+  const BandItem& t = S.items[i];
+  const int m = panel_rows(t, p);
+  um_sum<16>(m, um_steps(m), (m + UM_R - 1) / UM_R, t.part, panel_x(t, p), t.N, (int)blockIdx.x - S.pre[i]);
+}
+__global__ __launch_bounds__(256, 2) void k_qr_w_s(BandSlots S, int p) {
+  const int i = set_slot(S, blockIdx.x);
+  qr_w<16>(qr_w_args(S.items[i], p), (int)blockIdx.x - S.pre[i]);
+}
+__global__ __launch_bounds__(256, 4) void k_her2k_s(BandSlots S, int p) {
+  const int i = set_slot(S, blockIdx.x);
+  const BandItem& t = S.items[i];
+  her2k_tile<zc, 16>(t.H, t.ld, panel_rows(t, p), 16 * (p + 1), t.N, panel_v(t, p), panel_x(t, p), (int)blockIdx.x - S.pre[i]);
+}
+__global__ void k_band_extract_s(BandSlots S) {
+  const int i = set_slot(S, blockIdx.x);
+  const BandItem& t = S.items[i];
+  band_extract(t.H, t.ld, t.N, 16, 33, t.chase.BD, (int)blockIdx.x - S.pre[i]);
+}
+__global__ __launch_bounds__((ChaseDim<16>::SW + 1) * 64, 1) void k_chase_s(BandSlots S) {
+  const ChaseArgs a = S.items[set_slot(S, blockIdx.x)].chase;
+  chase<16, false>(a);
+}
 
 // d, e of the tridiagonal from the band; g = conj(gc).  After a stalled wait the band is
 // unfinished and may hold anything: status is set and what follows works on zeros.
@@ -2184,8 +2328,6 @@ __global__ void k_band_finish(const zc* __restrict__ BD, int N, int LB, double* 
   for (int r = 0; r < nrhs; ++r) g[(size_t)r * N + j] = bad ? mkz(0, 0) : conj(gc[(size_t)r * N + j]);
 }
 
-// control block of the chase: its error flag and sweep counter 0 (the panel's flag, [8],
-// is kept)
 // X = Q2 Z: the chase's reflectors, sweeps last to first, onto columns kept in LDS.  Bound by
 // the vector ALU: 8 N^2 flops a column as short dot products.  The wpc waves of a pair of
 // columns take its 64-row pieces (four reflectors of B rows) in turn, lane = row; the four
@@ -2282,11 +2424,6 @@ __global__ __launch_bounds__(768) void k_chase_back(ChaseBackArgs a) {
   }
 }
 
-__global__ void k_chase_init(int* ctl) {
-  const int i = threadIdx.x;
-  if (i == 0 || i == 32) ctl[i] = 0;
-}
-
 __global__ void k_zero_ints(int* p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
@@ -2303,35 +2440,33 @@ static size_t qr_ex_elems(int nwg_max) {
 
 int band_panel_rows() { return QP_WG * PR + 16; }
 
-// Most workgroups of a panel's launch on the current device: an eighth of those resident at
-// once, so that the launches of eight streams (a set's lanes, or several threads' plans; a
-// process has four hardware queues by default) all get theirs, and at most QP_WG.  256
-// compute units hold two of these workgroups each: 64.  A chase beside them takes the LDS of
-// one of the two from up to 176 units, but ends by itself.  More launches than that at once,
-// or another process's, can keep each other waiting; then a wait ends at its limit and the
-// caller solves by the one-stage form (kStalled).
-static int band_panel_wg() {
+// The panels' workgroups that the current device holds at once
+static int band_resident() {
   static std::atomic<int> known[64];           // + 1; 0: not looked up yet
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   if (const int k = known[dev].load(std::memory_order_relaxed)) return k - 1;
-  int cus = 0, a = 0, b = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_qr_panel<16>, 256, 0) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_qr_w<16>, 256, 0) != hipSuccess)
-    return 0;
-  const int n = std::min(QP_WG, cus * std::min(a, b) / 8);
-  known[dev].store(n + 1, std::memory_order_relaxed);
-  return n;
+  int cus = 0, n = 1 << 20;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  for (const void* k : {(const void*)k_qr_panel<16>, (const void*)k_qr_w<16>, (const void*)k_qr_panel_s, (const void*)k_qr_w_s}) {
+    int per = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 256, 0) != hipSuccess) return 0;
+    n = std::min(n, per);
+  }
+  known[dev].store(cus * n + 1, std::memory_order_relaxed);
+  return cus * n;
 }
 
-bool band_panel_fits(int N) { return N <= band_panel_rows() && (N - 16 + PR - 1) / PR <= band_panel_wg(); }
+// Most workgroups of a panel's launch: an eighth of those, so that the launches of eight
+// streams (a set's lanes, or several threads' plans; a process has four hardware queues by
+// default) all get theirs, and at most QP_WG.  256 compute units hold two of these workgroups
+// each: 64.  A chase beside them takes the LDS of one of the two from up to 176 units, but
+// ends by itself.  More launches than that at once, or another process's, can keep each other
+// waiting; then a wait ends at its limit and the caller solves by the one-stage form
+// (kStalled).
+static int band_panel_wg() { return std::min(QP_WG, band_resident() / 8); }
 
-// steps of k_update_mul: fewer parts with more steps, more workgroups with fewer (at these
-// sizes about 1200 workgroups either way, 512 run at once; lines at half and one and a half
-// times these sizes measured within 1 %)
-constexpr int UM_4 = 6144, UM_2 = 3072;
-static int um_steps(int m) { return m > UM_4 ? 4 : m > UM_2 ? 2 : 1; }
+bool band_panel_fits(int N) { return N <= band_panel_rows() && (N - 16 + PR - 1) / PR <= band_panel_wg(); }
 
 // slots of the partial products for at most N rows: k_hmm_b's K slices, k_update_mul's parts
 static size_t hb_slots(int N, int b) {
@@ -2455,20 +2590,53 @@ static void gram(hipStream_t s, BandWork& w, int m, const zc* A, const zc* Y0, i
   hipLaunchKernelGGL(k_gram_sum<B>, dim3((nout + 63) / 64), dim3(256), 0, s, P, w.gp, n1, out0, out1);
 }
 
+// whether the reduction of a COMPLEX*16 matrix takes one-launch panels
+static bool qr_form(const BandWork& w) { return w.b == 16 && w.panel_wg >= (w.N - 16 + PR - 1) / PR; }
+static int wait_polls(const BandWork& w) { return w.wait_limit > 0 ? w.wait_limit : 1 << 20; }
+static int ex_wgs(const BandWork& w) { return min(w.nwg_max, QP_WG); }   // workgroups that the slots hold
+
+static ChaseArgs chase_args(const BandWork& w, int nrhs) {
+  ChaseArgs ca;
+  ca.BD = w.BD;
+  ca.N = w.N;
+  ca.gc = w.gc;
+  ca.nrhs = nrhs;
+  ca.prog = w.prog;
+  ca.ctl = w.err;
+  // polls of about half a microsecond each: about a second; in LDS about two seconds
+  ca.spin_limit = w.wait_limit > 0 ? w.wait_limit : 1 << 21;
+  ca.lds_limit = w.wait_limit > 0 ? w.wait_limit : 1 << 25;
+  ca.Vc = nullptr;
+  ca.ld = 0;
+  ca.tau = w.tau2;
+  ca.kt = chase_ntasks(w.N, w.b, 0);
+  return ca;
+}
+
+static BandItem band_item(const BandWork& w, zc* H, int ld, int nrhs) {
+  return BandItem{H, ld, w.N, nrhs, w.V, w.X, w.V2, w.X2, w.Y, w.T, w.gc, w.hb, w.ex, qr_ex_elems<16>(ex_wgs(w)),
+                  qr_slots<16>(ex_wgs(w)), ex_wgs(w), w.err, wait_polls(w), w.tau1, chase_args(w, nrhs)};
+}
+
+// workgroups of the chase: as many as groups of sweeps can be at work at once, each following
+// the one before by more than two tasks a sweep
+static int chase_wgs(int N, int b) {
+  const int sw = (b == 16) ? ChaseDim<16>::SW : ChaseDim<32>::SW;
+  return min((N - 1 + sw - 1) / sw, min(256, chase_ntasks(N, b, 0) / (2 * sw) + 4));
+}
+
 template <class T, int B>
 static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   const int N = w.N, b = B;
-  const int exw = min(w.nwg_max, QP_WG);               // workgroups that the slots hold
-  const size_t exn = qr_ex_elems<B>(exw);
   // COMPLEX*16 panels of at most panel_wg workgroups: one launch for the panel and one for W
   // (5 launches a panel, one of them a pass over the trailing matrix that updates it for the
   // panel before and multiplies it with this one's Y).  The limit does not depend on how many
   // streams run, so that the results do not either.  The COMPLEX*8 form keeps the separate kernels, whose roundings
   // its stored matrix amplifies.
-  const bool qr = std::is_same<T, zc>::value && B == 16 && w.panel_wg >= (N - b + PR - 1) / PR;
-  const int spin = w.wait_limit > 0 ? w.wait_limit : 1 << 20;
-  if (qr)
-    hipLaunchKernelGGL(k_fill_empty, dim3((unsigned)((2 * exn + 255) / 256)), dim3(256), 0, s, w.ex, 2 * exn);
+  const bool qr = std::is_same<T, zc>::value && qr_form(w);
+  BandItem it{};
+  if constexpr (std::is_same<T, zc>::value)
+    if (qr) it = band_item(w, H, ld, nrhs);
   for (int p = 0;; ++p) {
     const int c0 = p * b, r0 = c0 + b;
     if (r0 >= N) break;
@@ -2492,22 +2660,16 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
     const dim3 g(a.nwg), blk(PR);
     if constexpr (std::is_same<T, zc>::value && B == 16)
       if (qr) {
-        zc *ex = w.ex + (size_t)(p & 1) * exn, *exo = w.ex + (size_t)((p + 1) & 1) * exn;
-        const size_t wo = qr_slots<B>(exw);
-        zc *V = p & 1 ? w.V2 : w.V, *X = p & 1 ? w.X2 : w.X;          // this panel's; the one's before:
-        const zc *Vo = p & 1 ? w.V : w.V2, *Xo = p & 1 ? w.X : w.X2;
-        zc* A22 = H + r0 + (size_t)ld * r0;
+        zc *V = panel_v(it, p), *X = panel_x(it, p);                  // this panel's; the one's before:
+        const zc *Vo = panel_v(it, p + 1), *Xo = panel_x(it, p + 1);
         if (p > 0)
           hipLaunchKernelGGL((k_strip<B>), dim3((m + B + 63) / 64), blk, 0, s, H + c0 + (size_t)ld * c0, ld, m + B, N, Vo, Xo);
-        QrPanelArgs q{H, ld, N, c0, r0, m, k, V, w.Y, w.T, w.gc, nrhs, ex, exo, exw + 1, a.nwg, w.err + 8, spin,
-                      w.tau1 ? w.tau1 + c0 : nullptr};
-        hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, q);
+        hipLaunchKernelGGL((k_qr_panel<B>), g, blk, 0, s, qr_panel_args(it, p));
         const int n = um_steps(m), nt = (m + UM_R - 1) / UM_R;
-        const dim3 gt(4 / n * (nt * (nt + 1) / 2));
         auto um = p > 0 ? k_update_mul<B, true> : k_update_mul<B, false>;
         const bool tev = w.kev && w.kev_used < w.kev_cap;
         if (tev) hipEventRecord(w.kev[2 * w.kev_used], s);
-        hipLaunchKernelGGL(um, gt, blk, 0, s, A22, ld, m, N, Vo + B, Xo + B, w.Y, w.hb, nt, n);
+        hipLaunchKernelGGL(um, dim3(um_blocks(m)), blk, 0, s, trailing(it, p), ld, m, N, Vo + B, Xo + B, w.Y, w.hb, nt, n);
         if (tev) {
           hipEventRecord(w.kev[2 * w.kev_used++ + 1], s);
           // the update's two products of B reflectors on the lower triangle, the product with Y
@@ -2515,10 +2677,9 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
         }
         const size_t tot = (size_t)m * B;
         hipLaunchKernelGGL(k_um_sum<B>, dim3((unsigned)((tot + 255) / 256)), blk, 0, s, m, n, nt, w.hb, X, N);
-        QrWArgs x{m, N, V, w.T, X, ex + wo, exo + wo, a.nwg, w.err + 8, spin};
-        hipLaunchKernelGGL((k_qr_w<B>), g, blk, 0, s, x);
+        hipLaunchKernelGGL((k_qr_w<B>), g, blk, 0, s, qr_w_args(it, p));
         // the last panel's update, which no further product waits for
-        if (m - B <= 0 || min(b, m - B - 1) <= 0) {
+        if (last_panel(it, p)) {
           const int nu = (m + 63) / 64;
           hipLaunchKernelGGL((k_her2k_full<T, B>), dim3(nu * (nu + 1) / 2), blk, 0, s, H, ld, m, r0, N, V, X);
         }
@@ -2526,7 +2687,7 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
       }
     if (w.panel_resident > 0 && a.nwg <= w.panel_resident) {
       hipLaunchKernelGGL((k_panel<T, B>), g, blk, 0, s, a, w.V, w.bar + (size_t)p * (BMAX + 1), w.err + 8,
-                         (long long)spin);
+                         (long long)wait_polls(w));
     } else {
       for (int c = 0; c <= k; ++c) hipLaunchKernelGGL((k_pqr_col<T, B>), g, blk, 0, s, a, c);
       hipLaunchKernelGGL((k_pfin<T, B>), g, blk, 0, s, a, w.V);
@@ -2544,6 +2705,29 @@ static int stage1(hipStream_t s, BandWork& w, T* H, int ld, int nrhs) {
   return WTB_OK;
 }
 
+// what the reduction finds before its first launch: flags, counters and slots cleared, the
+// tracked vectors conjugated
+static void band_begin(hipStream_t s, BandWork& w, const zc* g, int nrhs, bool qr) {
+  const int N = w.N;
+  if (nrhs > 0)
+    hipLaunchKernelGGL(k_conj_vec, dim3((unsigned)(((size_t)nrhs * N + 255) / 256)), dim3(256), 0, s, nrhs * N, g,
+                       w.gc);
+  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, w.err, 64);
+  hipLaunchKernelGGL(k_zero_ints, dim3((N + 64 + 255) / 256), dim3(256), 0, s, w.prog, N + 1);
+  if (qr) {
+    const size_t exn = 2 * qr_ex_elems<16>(ex_wgs(w));
+    hipLaunchKernelGGL(k_fill_empty, dim3((unsigned)((exn + 255) / 256)), dim3(256), 0, s, w.ex, exn);
+  } else {
+    const int nb = (N / w.b + 2) * (BMAX + 1);
+    hipLaunchKernelGGL(k_zero_ints, dim3((nb + 255) / 256), dim3(256), 0, s, w.bar, nb);
+  }
+}
+
+static void band_finish(hipStream_t s, const BandWork& w, zc* g, double* d, double* e, int nrhs, int* status) {
+  hipLaunchKernelGGL(k_band_finish, dim3((w.N + 255) / 256), dim3(256), 0, s, w.BD, w.N, w.LB, d, e, w.gc, g, nrhs,
+                     w.err, status);
+}
+
 template <class T>
 static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d, double* e, int* status) {
   const int N = w.N, b = w.b, nrhs = g ? w.nrhs : 0;
@@ -2557,46 +2741,95 @@ static int run_band_t(hipStream_t s, BandWork& w, T* H, int ld, zc* g, double* d
     if (!std::is_same<T, zc>::value || b != 16 || N > band_vec_rows() || !band_panel_fits(N)) return WTB_ERR_LIMIT;
     hipLaunchKernelGGL(k_zero_ints, dim3((4 * N + 255) / 256), dim3(256), 0, s, (int*)w.tau1, 4 * N);
   }
-  if (nrhs > 0)
-    hipLaunchKernelGGL(k_conj_vec, dim3((unsigned)(((size_t)nrhs * N + 255) / 256)), dim3(256), 0, s, nrhs * N, g,
-                       w.gc);
   w.kev_used = 0;
   w.kev_flops = 0.0;
-  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, w.err, 64);
-  {
-    const int nb = (N / b + 2) * (BMAX + 1);
-    hipLaunchKernelGGL(k_zero_ints, dim3((nb + 255) / 256), dim3(256), 0, s, w.bar, nb);
-  }
+  band_begin(s, w, g, nrhs, std::is_same<T, zc>::value && qr_form(w));
   int rc = (b == 16) ? stage1<T, 16>(s, w, H, ld, nrhs) : stage1<T, 32>(s, w, H, ld, nrhs);
   if (rc) return rc;
   hipLaunchKernelGGL(k_band_extract<T>, dim3(N), dim3(64), 0, s, H, ld, N, b, w.LB, w.BD);
-  hipLaunchKernelGGL(k_zero_ints, dim3((N + 64 + 255) / 256), dim3(256), 0, s, w.prog, N + 1);
-  hipLaunchKernelGGL(k_chase_init, dim3(1), dim3(64), 0, s, w.err);
-  ChaseArgs ca;
-  ca.BD = w.BD;
-  ca.N = N;
-  ca.gc = w.gc;
-  ca.nrhs = nrhs;
-  ca.prog = w.prog;
-  ca.ctl = w.err;
-  // polls of about half a microsecond each: about a second; in LDS about two seconds
-  ca.spin_limit = w.wait_limit > 0 ? w.wait_limit : 1 << 21;
-  ca.lds_limit = w.wait_limit > 0 ? w.wait_limit : 1 << 25;
-  // groups of sweeps that can be at work at once: each follows the one before by more than
-  // two tasks a sweep
-  const int sw = (b == 16) ? ChaseDim<16>::SW : ChaseDim<32>::SW;
-  const int ngrp = (N - 1 + sw - 1) / sw;
-  const int P = min(ngrp, min(256, chase_ntasks(N, b, 0) / (2 * sw) + 4));
-  ca.Vc = nullptr;
+  ChaseArgs ca = chase_args(w, nrhs);
   if constexpr (std::is_same<T, zc>::value)
     if (w.tau1) ca.Vc = H;
   ca.ld = ld;
-  ca.tau = w.tau2;
-  ca.kt = chase_ntasks(N, b, 0);
-  auto chase = b == 32 ? k_chase<32, false> : ca.Vc ? k_chase<16, true> : k_chase<16, false>;
-  hipLaunchKernelGGL(chase, dim3(P), dim3((sw + 1) * 64), 0, s, ca);
-  hipLaunchKernelGGL(k_band_finish, dim3((N + 255) / 256), dim3(256), 0, s, w.BD, N, w.LB, d, e, w.gc, g, nrhs,
-                     w.err, status);
+  auto kern = b == 32 ? k_chase<32, false> : ca.Vc ? k_chase<16, true> : k_chase<16, false>;
+  const int sw = (b == 16) ? ChaseDim<16>::SW : ChaseDim<32>::SW;
+  hipLaunchKernelGGL(kern, dim3(chase_wgs(N, b)), dim3((sw + 1) * 64), 0, s, ca);
+  band_finish(s, w, g, d, e, nrhs, status);
+  WTB_LAUNCH_CHECK();
+  return WTB_OK;
+}
+
+// ---- a set of reductions in shared launches -----------------------------------------------
+// One launch per kernel and panel for every matrix that still has that panel, one launch of the
+// chase for all.  A lane of its own per matrix instead keeps 4 to 20 compute units busy with
+// one latency chain, at most four of them at once (a process's hardware queues): 64 models of
+// N = 256 .. 1024 took 356 ms on one lane and 124 on four.
+bool band_in_set(const BandWork& w) { return qr_form(w) && w.N >= 32 && !w.tau1; }
+
+int band_panel_wgs(int N) { return (N - 16 + PR - 1) / PR; }
+
+// A set's panel launch takes up to half of the workgroups that the device holds at once (its
+// members' workgroups wait only for those of the same member), and leaves `beside` of them to
+// panels that run at the same time.
+int band_set_wg(int beside) { return std::min(band_resident() / 2, band_resident() - beside); }
+
+int band_set_prepare(BandSet& S) {
+  band_set_free(S);
+  if (S.items.empty()) return WTB_OK;
+  // largest first: the matrices that have panel p are the first ones
+  std::stable_sort(S.items.begin(), S.items.end(), [](const BandSetItem& x, const BandSetItem& y) { return x.w->N > y.w->N; });
+  std::vector<BandItem> h;
+  for (const auto& x : S.items) h.push_back(band_item(*x.w, x.H, x.ld, x.g ? x.w->nrhs : 0));
+  WTB_HIP(hipMalloc(&S.d_items, sizeof(BandItem) * h.size()));
+  WTB_HIP(hipMemcpy(S.d_items, h.data(), sizeof(BandItem) * h.size(), hipMemcpyHostToDevice));
+  return WTB_OK;
+}
+
+void band_set_free(BandSet& S) {
+  if (S.d_items) (void)hipFree(S.d_items);
+  S.d_items = nullptr;
+}
+
+void band_set_begin(hipStream_t s, const BandSetItem& x) { band_begin(s, *x.w, x.g, x.g ? x.w->nrhs : 0, true); }
+void band_set_finish(hipStream_t s, const BandSetItem& x) {
+  band_finish(s, *x.w, x.g, x.d, x.e, x.g ? x.w->nrhs : 0, x.status);
+}
+
+int run_band_set(hipStream_t s, const BandSet& S) {
+  if (S.items.empty()) return WTB_OK;
+  if (!S.d_items) return WTB_ERR_ARG;
+  const BandItem* dev = static_cast<const BandItem*>(S.d_items);
+  const int M = (int)S.items.size();
+  auto rows = [&](int i, int p) { return S.items[i].w->N - 16 * (p + 1); };
+  // items first .. last - 1, blocks(i) workgroups each, in launches of at most kSetMax members
+  // and `most` workgroups
+  auto launch = [&](auto kern, int first, int last, auto blocks, int most, int threads, auto... args) {
+    for (int i = first; i < last;) {
+      BandSlots L;
+      L.items = dev + i;
+      L.n = 0;
+      L.pre[0] = 0;
+      for (; i < last && L.n < kSetMax && (L.n == 0 || L.pre[L.n] + blocks(i) <= most); ++i, ++L.n)
+        L.pre[L.n + 1] = L.pre[L.n] + blocks(i);
+      hipLaunchKernelGGL(kern, dim3(L.pre[L.n]), dim3(threads), 0, s, L, args...);
+    }
+  };
+  const int any = 1 << 30, set_wg = S.max_wg;
+  for (int p = 0, n = M;; ++p) {
+    while (n > 0 && rows(n - 1, p) < 2) --n;
+    if (n == 0) break;
+    auto wgs = [&](int i) { return (rows(i, p) + PR - 1) / PR; };
+    if (p > 0) launch(k_strip_s, 0, n, [&](int i) { return (rows(i, p) + 16 + 63) / 64; }, any, 256, p);
+    launch(k_qr_panel_s, 0, n, wgs, set_wg, 256, p);
+    launch(p > 0 ? k_update_mul_s<true> : k_update_mul_s<false>, 0, n, [&](int i) { return um_blocks(rows(i, p)); }, any, 256, p);
+    launch(k_um_sum_s, 0, n, [&](int i) { return (rows(i, p) * 16 + 255) / 256; }, any, 256, p);
+    launch(k_qr_w_s, 0, n, wgs, set_wg, 256, p);
+    int f = n;                                 // members whose last panel this is
+    while (f > 0 && rows(f - 1, p + 1) < 2) --f;
+    launch(k_her2k_s, f, n, [&](int i) { const int u = (rows(i, p) + 63) / 64; return u * (u + 1) / 2; }, any, 256, p);
+  }
+  launch(k_band_extract_s, 0, M, [&](int i) { return S.items[i].w->N; }, any, 64);
+  launch(k_chase_s, 0, M, [&](int i) { return chase_wgs(S.items[i].w->N, 16); }, any, (ChaseDim<16>::SW + 1) * 64);
   WTB_LAUNCH_CHECK();
   return WTB_OK;
 }

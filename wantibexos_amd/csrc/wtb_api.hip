@@ -830,6 +830,13 @@ static bool plan_one_stage(const wtb_bse_plan* p) {
   if (p->qmode || p->sp_only) return false;
   return !plan_two_stage(p);
 }
+// whether it is the COMPLEX*16 two-stage form, which a batch runs in shared launches
+static bool plan_band_set(const wtb_bse_plan* p) {
+  return !p->qmode && !p->sp_only && !p->mixed && plan_two_stage(p) && band_in_set(p->bw);
+}
+static BandSetItem plan_set_item(wtb_bse_plan* p) {
+  return BandSetItem{&p->bw, p->H, (int)p->ldh, p->g, p->tw.d, p->tw.e, p->status};
+}
 
 // stages (d2)-(e): everything after the reduction
 static int plan_enqueue_post(wtb_bse_plan* p) {
@@ -1816,21 +1823,24 @@ int wtb_bse_plan_tune(wtb_bse_plan* p, int* best, double* ms) {
 // batching form: many models in one captured graph.  Stages (a)-(c) of every matrix run
 // on parallel streams (lanes); the one-stage reductions then run as groups in lockstep
 // (one launch per kernel and column step for all matrices of a group, the groups being
-// the matrices of one element type and panel width); stages (d2)-(e) run on the lanes
-// again.  Matrices with another reduction (two-stage) run their whole pipeline on
-// their lane before the groups.
+// the matrices of one element type and panel width), the COMPLEX*16 two-stage ones as a set
+// (one launch per kernel and panel, one of the chase); stages (d2)-(e) run on the lanes
+// again.  The other matrices (two-stage of band 32, and those for which a lane of their own is
+// better: batch_group) run their whole pipeline on their lane beside the groups and the set.
 // ---------------------------------------------------------------------------
 struct wtb_bse_batch {
   wtb_ctx* ctx = nullptr;
   std::vector<wtb_bse_plan*> plans;
   std::vector<hipStream_t> lanes;
   std::vector<int> lane_of;             // plan -> lane
+  std::vector<char> shared;             // lane -> has grouped plans
   std::vector<hipEvent_t> ev_done;      // one per lane
   hipEvent_t ev_start = nullptr;
   hipEvent_t ev_mid = nullptr;          // the groups' reductions are done
   hipEvent_t ev_jac = nullptr;          // the batched Jacobi eigensolves are done
   std::vector<TriGroup> groups;
-  std::vector<char> grouped;            // plan -> reduced in a group
+  BandSet set;
+  std::vector<char> grouped;            // plan -> reduced in a group (1) or in the set (2)
   std::vector<JacobiItem> jitems;       // the grouped plans' Jacobi eigensolves (stage b)
   JacobiItem* d_jitems = nullptr;
   bool stale = true;                    // groups and graph to be (re)built
@@ -1842,20 +1852,76 @@ static void batch_drop(wtb_bse_batch* b) {
   b->gexec = nullptr;
   for (auto& g : b->groups) tri_group_free(g);
   b->groups.clear();
+  band_set_free(b->set);
+  b->set.items.clear();
   if (b->d_jitems) hipFree(b->d_jitems);
   b->d_jitems = nullptr;
   b->jitems.clear();
   b->stale = true;
 }
 
+// Lanes: longest processing time first, to the least loaded lane.  A plan that runs whole takes
+// about 11 us N + 1.3e-10 ms N^3 (5.8 ms at N = 576, 22 at 2116, 72 at 5184, 540 at 14400); of
+// one that is reduced with others the lane runs what comes before and after, a tenth of that
+// or less.
+static void batch_lanes(wtb_bse_batch* b) {
+  const int n = (int)b->plans.size();
+  std::vector<int> order(n);
+  for (int i = 0; i < n; ++i) order[i] = i;
+  auto cost = [&](int i) {
+    const double N = b->plans[i]->N;
+    return b->grouped[i] ? 20.0 + 0.1 * N : N + 1.2e-8 * N * N * N;
+  };
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost(x) > cost(y); });
+  std::vector<double> load(b->lanes.size(), 0.0);
+  b->lane_of.assign(n, 0);
+  b->shared.assign(b->lanes.size(), 0);
+  for (int i : order) {
+    const int l = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    b->lane_of[i] = l;
+    load[l] += cost(i);
+    b->plans[i]->stream = b->lanes[l];
+    if (b->grouped[i]) b->shared[l] = 1;
+  }
+}
+
 // the groups: one per (element type, panel width) among the plans with a one-stage
-// reduction
+// reduction; the set of the COMPLEX*16 two-stage ones
+//
+// A matrix of more than kSetMaxN rows fills the device in its own launches for most of its
+// reduction, and runs whole on a lane if each such matrix has one; so do one or two matrices
+// with a lane each.  Set / lanes on four lanes, ms: 2, 3, 4 of N = 2304 28.2 / 27.7, 30.5 / 31.2,
+// 33.6 / 33.9; of 2704 34.8 / 33.4, 38.3 / 38.1, 43.2 / 42.6; of 4096 three and four 76.6 /
+// 70.8, 89.1 / 79.9; eight of 5184 258 / 257, four of them 147 / 127; three of 1024 and of 256
+// 15 / 15.5, 3.1 / 3.7.  On one lane the set is always ahead: eight of 576 .. 2304 34 / 106,
+// 64 of 256 .. 1024 58 / 356, two of 5184 100 / 142.
+constexpr int kSetMaxN = 2500;
+
 static int batch_group(wtb_bse_batch* b) {
   batch_drop(b);
-  const int n = (int)b->plans.size();
+  const int n = (int)b->plans.size(), lanes = (int)b->lanes.size();
   b->grouped.assign(n, 0);
+  int cand = 0, large = 0, beside = 0, widest = 0;
+  for (const auto* p : b->plans) {
+    if (!plan_band_set(p)) continue;
+    ++cand;
+    if (p->N > kSetMaxN) {
+      ++large;
+      beside += band_panel_wgs(p->N);
+    } else {
+      widest = std::max(widest, band_panel_wgs(p->N));
+    }
+  }
+  const bool all_whole = cand <= std::min(2, lanes);
+  const bool large_whole = large <= lanes && widest <= band_set_wg(beside);
+  b->set.max_wg = band_set_wg(large_whole ? beside : 0);
   for (int i = 0; i < n; ++i) {
     wtb_bse_plan* p = b->plans[i];
+    if (plan_band_set(p) && !all_whole && !(large_whole && p->N > kSetMaxN)) {
+      p->bw.wait_limit = b->ctx->wait_limit;
+      b->set.items.push_back(plan_set_item(p));
+      b->grouped[i] = 2;
+    }
     if (!plan_one_stage(p)) continue;
     const int nb = (p->tw.panel >= 8 && p->tw.panel <= p->tw.nb) ? p->tw.panel : p->tw.nb;
     TriGroup* g = nullptr;
@@ -1870,10 +1936,12 @@ static int batch_group(wtb_bse_batch* b) {
     g->items.push_back(TriGroupItem{&p->tw, p->mixed ? (void*)p->Hf : (void*)p->H, (int)p->ldh, p->g});
     b->grouped[i] = 1;
   }
+  batch_lanes(b);
   for (auto& g : b->groups) {
     const int rc = tri_group_prepare(g);
     if (rc) return rc;
   }
+  if (const int rc = band_set_prepare(b->set)) return rc;
   for (int i = 0; i < n; ++i)
     if (b->grouped[i]) b->jitems.push_back(plan_jacobi_item(b->plans[i]));
   if (!b->jitems.empty()) {
@@ -1889,39 +1957,54 @@ static int batch_group(wtb_bse_batch* b) {
 static int batch_enqueue(wtb_bse_batch* b) {
   hipStream_t s = b->ctx->stream;
   const int n = (int)b->plans.size();
-  auto fork = [&](hipEvent_t e) -> int {
+  // to all lanes or to those with grouped plans
+  auto fork = [&](hipEvent_t e, bool all) -> int {
     WTB_HIP(hipEventRecord(e, s));
-    for (hipStream_t l : b->lanes) WTB_HIP(hipStreamWaitEvent(l, e, 0));
+    for (size_t l = 0; l < b->lanes.size(); ++l)
+      if (all || b->shared[l]) WTB_HIP(hipStreamWaitEvent(b->lanes[l], e, 0));
     return WTB_OK;
   };
-  auto join = [&]() -> int {
+  auto join = [&](bool all) -> int {
     for (size_t l = 0; l < b->lanes.size(); ++l) {
+      if (!all && !b->shared[l]) continue;
       WTB_HIP(hipEventRecord(b->ev_done[l], b->lanes[l]));
       WTB_HIP(hipStreamWaitEvent(s, b->ev_done[l], 0));
     }
     return WTB_OK;
   };
   int rc;
+  // the plans that run whole, on lanes that have nothing else at once, else behind stage (c) of
+  // the lane's grouped ones
+  auto whole = [&](bool shared) -> int {
+    for (int i = 0; i < n; ++i)
+      if (!b->grouped[i] && (b->shared[b->lane_of[i]] != 0) == shared)
+        if (const int r = plan_enqueue(b->plans[i])) return r;
+    return WTB_OK;
+  };
   // stage (a) of the grouped matrices on the lanes, every model's Jacobi eigensolves in one
-  // batched launch, then stages (b')-(c) on the lanes again; the other plans run whole
-  if ((rc = fork(b->ev_start))) return rc;
+  // batched launch, then stages (b')-(c) on the lanes again
+  if ((rc = fork(b->ev_start, true)) || (rc = whole(false))) return rc;
+  for (int i = 0; i < n; ++i)
+    if (b->grouped[i] && (rc = plan_enqueue_pre_a(b->plans[i]))) return rc;
+  if ((rc = join(false))) return rc;
+  if (!b->jitems.empty() && (rc = launch_jacobi_batch(s, b->d_jitems, b->jitems))) return rc;
+  if ((rc = fork(b->ev_jac, false))) return rc;
   for (int i = 0; i < n; ++i) {
     wtb_bse_plan* p = b->plans[i];
-    rc = b->grouped[i] ? plan_enqueue_pre_a(p) : plan_enqueue(p);
-    if (rc) return rc;
+    if (b->grouped[i] && (rc = plan_enqueue_pre(p, false, true))) return rc;
+    if (b->grouped[i] == 2) band_set_begin(p->stream, plan_set_item(p));
   }
-  if ((rc = join())) return rc;
-  if (!b->jitems.empty() && (rc = launch_jacobi_batch(s, b->d_jitems, b->jitems))) return rc;
-  if ((rc = fork(b->ev_jac))) return rc;
-  for (int i = 0; i < n; ++i)
-    if (b->grouped[i] && (rc = plan_enqueue_pre(b->plans[i], false, true))) return rc;
-  if ((rc = join())) return rc;
+  if ((rc = join(false)) || (rc = whole(true))) return rc;
   for (const auto& g : b->groups)
     if ((rc = run_tridiag_group(s, g))) return rc;
-  if ((rc = fork(b->ev_mid))) return rc;
-  for (int i = 0; i < n; ++i)
-    if (b->grouped[i] && (rc = plan_enqueue_post(b->plans[i]))) return rc;
-  return join();
+  if ((rc = run_band_set(s, b->set))) return rc;
+  if ((rc = fork(b->ev_mid, false))) return rc;
+  for (int i = 0; i < n; ++i) {
+    wtb_bse_plan* p = b->plans[i];
+    if (b->grouped[i] == 2) band_set_finish(p->stream, plan_set_item(p));
+    if (b->grouped[i] && (rc = plan_enqueue_post(p))) return rc;
+  }
+  return join(true);
 }
 
 int wtb_bse_batch_create(wtb_ctx* c, int n, const wtb_tb_model* models, const wtb_bse_params* prms, int nlanes,
@@ -1958,21 +2041,9 @@ int wtb_bse_batch_create(wtb_ctx* c, int n, const wtb_tb_model* models, const wt
     wtb_bse_batch_destroy(b);
     return rc;
   }
-  // longest processing time first: the longest goes to the least loaded lane.  A plan takes
-  // about 11 us N + 1.3e-10 ms N^3 (5.8 ms at N = 576, 22 at 2116, 72 at 5184, 540 at 14400);
-  // with N^3 alone eight models of N = 576 .. 2304 took 44 ms on four lanes, 38 with this
-  std::vector<int> order(n);
-  for (int i = 0; i < n; ++i) order[i] = i;
-  std::sort(order.begin(), order.end(), [&](int x, int y) { return b->plans[x]->N > b->plans[y]->N; });
-  std::vector<double> load(nlanes, 0.0);
-  b->lane_of.assign(n, 0);
-  for (int i : order) {
-    const int l = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    b->lane_of[i] = l;
-    const double N = b->plans[i]->N;
-    load[l] += N + 1.2e-8 * N * N * N;
-    b->plans[i]->stream = b->lanes[l];
-    if (nlanes > 1) b->plans[i]->bw.panel_resident = 0;   // lanes share the device
+  for (auto* p : b->plans) {
+    p->stream = b->lanes[0];                      // batch_lanes spreads them
+    if (nlanes > 1) p->bw.panel_resident = 0;     // lanes share the device
   }
   *out = b;
   return WTB_OK;

@@ -179,6 +179,30 @@ bool band_panel_fits(int N);
 int band_panel_rows();
 int band_bind(BandWork& w, void* base, int N, int b, int nrhs);
 int run_band_tridiag(hipStream_t s, BandWork& w, zc* H, int ld, zc* g, double* d, double* e, int* status);
+// A set of such reductions (COMPLEX*16, band 16, no reflectors kept) in shared launches: each
+// matrix gets bitwise the results of run_band_tridiag on it alone.  begin and finish are each
+// matrix's own launches before and after, on any stream ordered with the set's.
+struct BandSetItem {
+  BandWork* w;
+  zc* H;
+  int ld;
+  zc* g;             // may be null
+  double *d, *e;
+  int* status;
+};
+struct BandSet {
+  std::vector<BandSetItem> items;    // sorted by size in band_set_prepare
+  int max_wg = 0;                    // most panel workgroups of one launch (band_set_wg)
+  void* d_items = nullptr;           // their kernel arguments on the device
+};
+int band_panel_wgs(int N);             // workgroups of the first panel's launch
+int band_set_wg(int beside);
+bool band_in_set(const BandWork& w);   // whether a reduction may be a member
+int band_set_prepare(BandSet& S);
+void band_set_free(BandSet& S);
+void band_set_begin(hipStream_t s, const BandSetItem& x);
+int run_band_set(hipStream_t s, const BandSet& S);
+void band_set_finish(hipStream_t s, const BandSetItem& x);
 int run_band_tridiag_f32(hipStream_t s, BandWork& w, zf* H, int ld, zc* g, double* d, double* e, int* status);
 
 // stage (d): tridiagonal divide and conquer (eigenvalues + Z^T x for tracked vectors)
