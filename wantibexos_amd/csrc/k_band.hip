@@ -60,6 +60,11 @@ __device__ inline zc zdiv(zc a, zc b) {
   return mkz(xr / den, xi / den);
 }
 
+// any NaN by its usual bits (the panels' exchange gives those of all ones a meaning)
+__device__ inline zc clean_nan(zc v) {
+  return mkz(v.re != v.re ? __builtin_nan("") : v.re, v.im != v.im ? __builtin_nan("") : v.im);
+}
+
 __device__ inline zc shfl_xor_z(zc v, int off) { return mkz(__shfl_xor(v.re, off), __shfl_xor(v.im, off)); }
 
 // lane ^ 16 within 32 lanes, by a swizzle
@@ -984,7 +989,7 @@ __global__ void k_band_extract(const T* __restrict__ A, int ld, int N, int b, in
 
 __global__ void k_conj_vec(int n, const zc* __restrict__ x, zc* __restrict__ y) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = conj(x[i]);
+  if (i < n) y[i] = clean_nan(conj(x[i]));
 }
 
 // sum over groups of SUB (8 or 16) consecutive lanes, the same bits in each: ^1, ^2, then
@@ -1068,9 +1073,10 @@ __device__ inline double lane_value(double x, int l) {
 __device__ inline zc lane_value(zc v, int l) { return mkz(lane_value(v.re, l), lane_value(v.im, l)); }
 
 // Values handed from every workgroup to every workgroup: slot [round][workgroup][B], each
-// slot written once per panel and filled with the bits ~0 before (a NaN that st_slot never
-// stores: an input's NaN may have them and keeps its bits through arithmetic), so that a
-// reader polls the value itself: no counter, no fence, one store and one load apart.  Rounds 0 .. B - 1 are the panel's columns, B .. B + 5 the tracked vectors;
+// slot written once per panel and filled with the bits ~0 before (a NaN; one of the input's
+// could have them and keep them through arithmetic, so whatever the slots' sums are formed
+// from is cleaned of such: the panel's columns, X and the tracked vectors), so that a reader
+// polls the value itself: no counter, no fence, one store and one load apart.  Rounds 0 .. B - 1 are the panel's columns, B .. B + 5 the tracked vectors;
 // entry nwg of a column's round is row c of the panel.
 struct QrPanelArgs {
   zc* A;                 // the matrix, ld
@@ -1092,12 +1098,6 @@ __device__ inline bool is_empty(zc v) {
   return __builtin_bit_cast(unsigned long long, v.re) == ~0ull || __builtin_bit_cast(unsigned long long, v.im) == ~0ull;
 }
 
-// a value into its slot, any NaN by the usual bits
-__device__ inline void st_slot(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff, zc v) {
-  if (v.re != v.re) v.re = __builtin_nan("");
-  if (v.im != v.im) v.im = __builtin_nan("");
-  st_buf(rs, voff, soff, v);
-}
 // what a poll of slots starts with: the loads after it are not those of the poll before
 __device__ inline void poll_again() { __asm__ volatile("" ::: "memory"); }
 
@@ -1143,6 +1143,10 @@ __device__ __forceinline__ void qr_panel(const QrPanelArgs& a, const int bx) {
     if (!live) {
 #pragma unroll
       for (int j = 0; j < B; ++j) row[j] = mkz(0, 0);
+    }
+    if (a.c0 == 0) {                           // (the later panels' columns come from strip)
+#pragma unroll
+      for (int j = 0; j < B; ++j) row[j] = clean_nan(row[j]);
     }
   }
   // the next panel's slots
@@ -1257,8 +1261,8 @@ __device__ __forceinline__ void qr_panel(const QrPanelArgs& a, const int bx) {
 #pragma unroll
         for (int p = 0; p < B; ++p) v[p] = fma_conj(xm, row[p], mkz(0, 0));
         const zc part = block_sums(v);
-        if (sub == 0) st_slot(ex, mine + q * (unsigned)sizeof(zc), c * RS, part);
-        if (bx == 0 && sub == 1) st_slot(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
+        if (sub == 0) st_buf(ex, mine + q * (unsigned)sizeof(zc), c * RS, part);
+        if (bx == 0 && sub == 1) st_buf(ex, (unsigned)(a.nwg * B + q) * (unsigned)sizeof(zc), c * RS, rowc[q]);
         if (c > 0) t_column(c - 1);            // while the sums are on their way
         zc rowv = mkz(0, 0);
         zc tot;
@@ -1314,7 +1318,7 @@ __device__ __forceinline__ void qr_panel(const QrPanelArgs& a, const int bx) {
     for (int j = 0; j < B; ++j) v[j] = fma_conj(row[j], g[r], mkz(0, 0));
     if (r > 0) lds_barrier();                  // the partial sums of r - 1 are read
     const zc part = block_sums(v);
-    if (sub == 0) st_slot(ex, mine + q * (unsigned)sizeof(zc), (B + r) * RS, part);
+    if (sub == 0) st_buf(ex, mine + q * (unsigned)sizeof(zc), (B + r) * RS, part);
   }
   t_column(a.k - 1);
 #pragma unroll
@@ -1457,7 +1461,7 @@ __device__ __forceinline__ void qr_w(const QrWArgs& a, const int bx) {
   for (int u = 0; u < NE; ++u) {
     const int e = t + 256 * u;
     const zc p = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
-    st_slot(ex, (unsigned)((size_t)bx * B * B + e) * (unsigned)sizeof(zc), 0, p);
+    st_buf(ex, (unsigned)((size_t)bx * B * B + e) * (unsigned)sizeof(zc), 0, p);
   }
   // while the sums are on their way: the rows of V and X that become W
   zc vv[4][B / 4], xx[4][TI][4];
@@ -1580,7 +1584,7 @@ __device__ __forceinline__ void strip(zc* __restrict__ A, int ld, int m, int N, 
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int cc = lk + 4 * q;
-    if (r < m && cc <= r) A[(size_t)r + (size_t)ld * cc] = mkz(h[q].re - cr[q], h[q].im + ci[q]);
+    if (r < m && cc <= r) A[(size_t)r + (size_t)ld * cc] = clean_nan(mkz(h[q].re - cr[q], h[q].im + ci[q]));
   }
 }
 template <int B>
@@ -1818,7 +1822,7 @@ __device__ __forceinline__ void um_sum(int m, int n, int nt, const zc* __restric
   const size_t e = (size_t)bx * 256 + threadIdx.x;
   if (e >= (size_t)m * B) return;
   const int row = (int)(e % m), col = (int)(e / m);
-  X[(size_t)row + (size_t)ldx * col] = strided_sum(part + e, (size_t)m * B, 0, um_parts(row / UM_R, n, nt), 1, mkz(0, 0));
+  X[(size_t)row + (size_t)ldx * col] = clean_nan(strided_sum(part + e, (size_t)m * B, 0, um_parts(row / UM_R, n, nt), 1, mkz(0, 0)));
 }
 template <int B>
 __global__ __launch_bounds__(256) void k_um_sum(int m, int n, int nt, const zc* __restrict__ part, zc* __restrict__ X,
