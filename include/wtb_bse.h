@@ -328,10 +328,13 @@ int wtb_mlp_train(wtb_mlp* mlp, int S, const float* X, const float* t, int epoch
 int wtb_mlp_destroy(wtb_mlp* mlp);
 
 /* ------------------------------------------------------------------------
- * Panel width of the blocked Householder reduction (8..32 columns per
- * trailing MFMA update; default 32) and its autotuner, which times the
+ * Panel width of the one-stage (blocked Householder) reduction (8..32 columns
+ * per trailing MFMA update; default 32) and its autotuner, which times the
  * reduction for widths 16, 20, 24, 32 on the plan's own matrix and keeps the
- * fastest (ms[4]: their times).  No counterpart in the reference.
+ * fastest (ms[4]: their times).  A plan that takes the two-stage reduction
+ * (wtb_bse_plan_set_reduction) has no such panels: the width is kept for when it
+ * does not, and the tuner returns it at once with times of 0.  No counterpart
+ * in the reference.
  * ------------------------------------------------------------------------ */
 int wtb_bse_plan_set_panel(wtb_bse_plan* plan, int nb);
 int wtb_bse_plan_tune(wtb_bse_plan* plan, int* best, double* ms);

@@ -549,8 +549,9 @@ class BSEPlan:
         _check(lib().wtb_bse_plan_set_panel(self.h, int(nb)))
 
     def tune(self):
-        """Time the reduction for panel widths 16, 20, 24, 32 on this matrix and keep the
-        fastest.  Returns (best, {width: ms})."""
+        """Time the one-stage reduction for panel widths 16, 20, 24, 32 on this matrix and keep
+        the fastest.  Returns (best, {width: ms}); a plan that takes the two-stage reduction
+        has no such panels and gets its width back with times of 0."""
         best = np.zeros(1, dtype=np.int32)
         ms = np.zeros(4)
         _check(lib().wtb_bse_plan_tune(self.h, _p(best), _p(ms)))

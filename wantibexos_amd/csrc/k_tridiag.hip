@@ -1214,7 +1214,7 @@ int tridiag_bind(TridiagWork& tw, void* base, int N, int nb, int nrhs) {
 }
 
 // the panel width a reduction runs with: the tuned one when it fits the binding
-static int tri_panel(const TridiagWork& tw) {
+int tri_panel(const TridiagWork& tw) {
   return (tw.panel >= 8 && tw.panel <= tw.nb) ? tw.panel : tw.nb;
 }
 

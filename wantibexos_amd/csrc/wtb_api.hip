@@ -1789,6 +1789,12 @@ int wtb_bse_plan_tune(wtb_bse_plan* p, int* best, double* ms) {
     set_error("wtb_bse_plan_tune: null plan");
     return WTB_ERR_ARG;
   }
+  if (plan_two_stage(p)) {
+    // no panels of the one-stage form run: nothing to time, the width stays
+    for (int k = 0; ms && k < 4; ++k) ms[k] = 0.0;
+    if (best) *best = tri_panel(p->tw);
+    return WTB_OK;
+  }
   WTB_HIP(hipSetDevice(p->ctx->device));
   const int cand[4] = {16, 20, 24, 32};
   const bool timing0 = p->timing;
@@ -1923,7 +1929,7 @@ static int batch_group(wtb_bse_batch* b) {
       b->grouped[i] = 2;
     }
     if (!plan_one_stage(p)) continue;
-    const int nb = (p->tw.panel >= 8 && p->tw.panel <= p->tw.nb) ? p->tw.panel : p->tw.nb;
+    const int nb = tri_panel(p->tw);
     TriGroup* g = nullptr;
     for (auto& x : b->groups)
       if (x.f32 == p->mixed && x.nb == nb) g = &x;

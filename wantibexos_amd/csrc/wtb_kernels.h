@@ -107,6 +107,7 @@ int tridiag_bind(TridiagWork& tw, void* base, int N, int nb, int nrhs);
 int run_tridiag(hipStream_t s, TridiagWork& tw, zc* d_H, int ldh, zc* d_g);
 // the same reduction on a COMPLEX*8 matrix (precision form)
 int run_tridiag_f32(hipStream_t s, TridiagWork& tw, zf* d_H, int ldh, zc* d_g);
+int tri_panel(const TridiagWork& tw);   // the panel width they run with
 // A group of such reductions of one element type and panel width, run in lockstep: one
 // launch per kernel and column step serves every matrix of the group, and each matrix
 // gets bitwise the results of run_tridiag / run_tridiag_f32 on it alone.
