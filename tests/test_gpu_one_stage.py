@@ -68,3 +68,17 @@ def test_lockstep_groups(ctx, lanes):  # noqa: F811
                 got = b.results(i)
                 for k in ("W", "act", "eps"):
                     assert np.array_equal(got[k], ref[k]), (i, k)
+
+
+def test_kernel_times_are_those_of_the_form_that_ran(ctx):  # noqa: F811
+    from wantibexos_amd import bse
+    with bse.BSEPlan(ctx, model(), params(12, 12)) as plan:
+        plan.set_timing(2)
+        seen = []
+        for form in (False, None, False, None):
+            plan.set_reduction(form)
+            plan.execute()
+            plan.results()
+            seen.append((plan.kernel_ms()[1], plan.kernel_flops() > 0))
+    # 575 GEMVs; 35 panels of 16 columns
+    assert seen == [(575, False), (35, True)] * 2

@@ -691,6 +691,7 @@ static int plan_reduce(wtb_bse_plan* p, zc* g, int* status) {
     p->bw.kev = p->kernel_timing ? p->kev.data() : nullptr;
     p->bw.kev_cap = p->kernel_timing ? p->N : 0;
     p->bw.wait_limit = p->ctx->wait_limit;
+    p->tw.kev_used = 0;                     // the timed launches are this form's
     // the band reduction reads and updates the lower triangle only
     if (p->mixed) return run_band_tridiag_f32(s, p->bw, p->Hf, (int)p->ldh, g, p->tw.d, p->tw.e, status);
     return run_band_tridiag(s, p->bw, p->H, (int)p->ldh, g, p->tw.d, p->tw.e, status);
