@@ -2472,9 +2472,13 @@ static int band_panel_wg() { return std::min(QP_WG, band_resident() / 8); }
 
 bool band_panel_fits(int N) { return N <= band_panel_rows() && (N - 16 + PR - 1) / PR <= band_panel_wg(); }
 
+// whether one-launch panels may run, which keep the V and W of the panel before
+static bool second_panel(int N, int b) { return b == 16 && N <= band_panel_rows(); }
+
 // slots of the partial products for at most N rows: k_hmm_b's K slices, k_update_mul's parts
+// (9 MB at N = 1024 beside a matrix of 17, 129 at 5184 beside 430, 420 at 14400 beside 3318)
 static size_t hb_slots(int N, int b) {
-  if (b != 16 || N > band_panel_rows()) return HB_SMAX;
+  if (!second_panel(N, b)) return HB_SMAX;
   auto slots = [](int m) { const int nt = (m + UM_R - 1) / UM_R; return um_parts(nt - 1, um_steps(m), nt); };
   return std::max({(int)HB_SMAX, slots(N), slots(std::min(N, UM_4)), slots(std::min(N, UM_2))});
 }
@@ -2499,7 +2503,7 @@ size_t band_work_bytes(int N, int b, int nrhs) {
   add(sizeof(zc) * nwg * BMAX * BMAX);        // K slices of the small products
   add(sizeof(zc) * GRAM_PMAX * BMAX * (BMAX + 16));   // partials of the tall-skinny products
   add(sizeof(zc) * hb_slots(N, b) * (size_t)N * b);    // partials of X = A22 Y
-  add(sizeof(zc) * 2 * (size_t)N * b);                 // V2, X2
+  if (second_panel(N, b)) add(sizeof(zc) * 2 * (size_t)N * b);   // V2, X2
   add(sizeof(zc) * (size_t)N * LB);           // band
   add(sizeof(zc) * (size_t)N * (nrhs > 0 ? nrhs : 1));   // gc
   add(sizeof(int) * ((size_t)N + 1));         // prog
@@ -2542,8 +2546,11 @@ int band_bind(BandWork& w, void* base, int N, int b, int nrhs) {
   w.gw_elems = nwg * BMAX * BMAX;
   w.gp = (zc*)take(sizeof(zc) * GRAM_PMAX * BMAX * (BMAX + 16));
   w.hb = (zc*)take(sizeof(zc) * hb_slots(N, b) * (size_t)N * b);
-  w.V2 = (zc*)take(sizeof(zc) * 2 * (size_t)N * b);
-  w.X2 = w.V2 + (size_t)N * b;
+  w.V2 = w.X2 = nullptr;
+  if (second_panel(N, b)) {
+    w.V2 = (zc*)take(sizeof(zc) * 2 * (size_t)N * b);
+    w.X2 = w.V2 + (size_t)N * b;
+  }
   w.BD = (zc*)take(sizeof(zc) * (size_t)N * w.LB);
   w.gc = (zc*)take(sizeof(zc) * (size_t)N * (nrhs > 0 ? nrhs : 1));
   w.prog = (int*)take(sizeof(int) * ((size_t)N + 1));
