@@ -64,6 +64,14 @@ FP64_PEAK = 78.6        # TFLOP/s, dense FP64 MFMA
 FP32_PEAK = 157.3       # TFLOP/s, dense FP32 MFMA
 
 
+def update_kernel(precision, reduction, band, N):
+    """The two-stage reduction's timed trailing update: one pass over the trailing matrix with
+    the FP64 matrix's one-launch panels (band 16, the default's band up to N = 16400), else
+    the update alone."""
+    one_launch = precision != "mixed" and N <= 16400 and (reduction != "two" or band == 16)
+    return "k_update_mul" if one_launch else "k_her2k_full"
+
+
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
@@ -375,7 +383,7 @@ def bench_bands(args, cfg, model):
     avg_s = k_ms * 1e-3 / max(k_n, 1)
     if k_flops > 0:
         per_launch = k_flops / max(k_n, 1)
-        kname = "k_her2k_full" if args.precision == "mixed" or (args.reduction == "two" and args.band == 32) else "k_update_mul"
+        kname = update_kernel(args.precision, args.reduction, args.band, N)
         ach = per_launch / avg_s / 1e12
         peak = FP32_PEAK if args.precision == "mixed" else FP64_PEAK
         roofline = dict(bound="mfma", achieved=round(ach, 2), peak=peak, unit="TFLOP/s", frac=round(ach / peak, 4),
@@ -634,7 +642,7 @@ def main():
     if k_flops > 0:
         # two-stage reduction: the dense -> band stage's trailing update, MFMA-bound
         per_launch = k_flops / max(k_n, 1)
-        kname = "k_her2k_full" if args.precision == "mixed" or (args.reduction == "two" and args.band == 32) else "k_update_mul"
+        kname = update_kernel(args.precision, args.reduction, args.band, N)
         ach = per_launch / avg_s / 1e12
         peak = FP32_PEAK if args.precision == "mixed" else FP64_PEAK
         log(f"{kname}: {k_n} launches, avg {avg_s * 1e6:.2f} us, {per_launch / 1e9:.3f} GFLOP/launch")
