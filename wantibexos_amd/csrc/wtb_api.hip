@@ -664,7 +664,8 @@ static void plan_drop_graph(wtb_bse_plan* p);
 // Stage (d1): the lower triangle of the plan's matrix (FP64 or COMPLEX*8) to the real
 // tridiagonal tw.d, tw.e, with Q^T applied to g (may be NULL).  Two-stage when nothing
 // downstream needs the Householder reflectors (exciton vectors, the refinement); its
-// bulge chase reports a stalled wait through status.
+// launches report a stalled wait through status, and whoever reads that solves by the
+// one-stage form (plan_redo).
 //
 // By default (two_stage = -1) the COMPLEX*16 matrix takes the two-stage reduction at every
 // size that has a panel.  Whole plan, one-stage / two-stage with band 16, MI355X:
@@ -2477,7 +2478,9 @@ int wtb_bse_bands_set_vectors(wtb_bse_bands* b, int first, int count) {
 // hardware queue each (four by default) and later ones the least used queue; before the
 // queues are all there, two lanes of one object can land on one and run one after the other
 // (12 q-points of N = 1024 on four lanes: 62.5 ms in a new process, 33.0 with these).  Four
-// streams first, and any lanes up to the number of queues get different ones.
+// streams first, and any lanes up to the number of queues get different ones.  This rests on
+// how the runtime hands out queues and on there being four; where that differs the lanes are
+// only slower, not wrong.  A batch needs none: its reductions share launches.
 struct LaneSpacers {
   hipStream_t st[4] = {};
   LaneSpacers() {
