@@ -1598,8 +1598,8 @@ __global__ __launch_bounds__(256) void k_strip(zc* __restrict__ A, int ld, int m
 // A workgroup takes 128 rows (block I) and 32 n columns of block J <= I, a wave 32 rows of
 // them, and goes through the columns in steps of 32.  Every element is read and written once
 // and serves both A(I, J) Y(J) -> X(I), accumulated over the steps, and A(I, J)^H Y(I) -> X(J),
-// summed over the waves: the update, accumulated onto the elements, leaves a 16 x 16 tile in
-// the MFMA's result layout, which is its layout for an operand whose sum runs over the tile's
+// summed over the waves: the update, and with it the elements, is a 16 x 16 tile in the MFMA's
+// result layout, which is its layout for an operand whose sum runs over the tile's
 // columns, so the first product needs no data movement, and the second one transposes the
 // tile through LDS.  The parts go to part[slot][col][row], the rows of block K in the slots
 // 0 .. um_parts(K) - 1 (first the 4 (K + 1) / n column groups left of and in block K, then the
@@ -1647,18 +1647,13 @@ __device__ __forceinline__ void update_mul(zc* __restrict__ A, int ld, int m, in
     if (on) {
       // h[x][y][2 e], [2 e + 1]: re and im of column c0 + 8 x + 4 e + lk, row r0 + 16 y + lr,
       // which are rows lk + 8 e and lk + 8 e + 4 of the MFMA's result: 16 bytes go to and come
-      // from four registers next to each other
+      // from four registers next to each other.  The update is summed from zero and the
+      // elements added to it, one rounding an element and panel instead of one a product.
       d4 h[4][2];
 #pragma unroll
       for (int x = 0; x < 4; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const zc v = A[(size_t)min(r0 + 16 * y + lr, m - 1) + (size_t)ld * min(c0 + 8 * x + 4 * e + lk, m - 1)];
-            h[x][y][2 * e] = v.re;
-            h[x][y][2 * e + 1] = v.im;
-          }
+        for (int y = 0; y < 2; ++y) h[x][y] = d4{0, 0, 0, 0};
       zc ya[4][2], yb[2][4];                   // Y of the step's columns and of the rows
 #pragma unroll
       for (int x = 0; x < 4; ++x)
@@ -1695,6 +1690,16 @@ __device__ __forceinline__ void update_mul(zc* __restrict__ A, int ld, int m, in
             for (int y = 0; y < 2; ++y) h[x][y] = mfma16x16x4(a2[x], b[y].im, h[x][y]);
         }
       }
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const zc v = A[(size_t)min(r0 + 16 * y + lr, m - 1) + (size_t)ld * min(c0 + 8 * x + 4 * e + lk, m - 1)];
+            h[x][y][2 * e] += v.re;
+            h[x][y][2 * e + 1] += v.im;
+          }
       if (edge) {                              // nothing above the diagonal or outside
 #pragma unroll
         for (int x = 0; x < 4; ++x)
