@@ -230,8 +230,8 @@ def bench_davidson(args, cfg, model):
 def bench_batch(args):
     """Batching form: a set of uneven models (different Wannier counts and k grids) through
     the batch API (one captured graph for the set: per-matrix build and post-processing on
-    --lanes streams, the one-stage reductions in lockstep, one launch per kernel and column
-    step for all matrices), against the same plans run one after the other (results equal
+    --lanes streams, the reductions in launches shared by all matrices: one per kernel and
+    panel of the FP64 two-stage form, one per kernel and column step of the one-stage form), against the same plans run one after the other (results equal
     bit for bit) and against plain FP64 plans of the same models one after the other."""
     import dataclasses
     from concurrent.futures import ProcessPoolExecutor

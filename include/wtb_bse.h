@@ -341,9 +341,10 @@ int wtb_bse_plan_tune(wtb_bse_plan* plan, int* best, double* ms);
 
 /* ------------------------------------------------------------------------
  * Batching form (no counterpart in the reference, which solves one model
- * per run): many independent models of uneven sizes, one plan each, assigned
- * to nlanes streams largest-first; execute() replays every matrix's captured
- * graph on its stream and joins on the context stream; results() as for a plan.
+ * per run): many independent models of uneven sizes, one plan each, their
+ * builds and post-processing on nlanes streams, their reductions in launches
+ * that serve all of them (the largest whole on streams of their own); execute()
+ * replays the set's captured graph on the context stream; results() as for a plan.
  * ------------------------------------------------------------------------ */
 typedef struct wtb_bse_batch wtb_bse_batch;
 int wtb_bse_batch_create(wtb_ctx* ctx, int n, const wtb_tb_model* models, const wtb_bse_params* prms,
